@@ -55,8 +55,8 @@ __host__ __device__ inline bool dispatch_fits(int E_cols, int k) {
 //  4. the copy, 512-byte column slabs of the 64 rows at a time: waves 0-7
 //     stream slabs of x into one half of an LDS double buffer, waves 8-15 write
 //     the other half to x_perm in position order, so consecutive lanes write
-//     consecutive positions: K-blocked, one run of (slots of an expert) x 64
-//     bytes per K-block; row-major, whole 512-byte slab rows.  Producers and
+//     consecutive positions: one run of (slots of an expert) x 64 bytes per
+//     K-block.  Columns past D are written as zeros up to Dk.  Producers and
 //     consumers run separate loops with the same barriers, so neither waits
 //     on the other's memory operations.  The first two slabs are loaded into
 //     the producers' registers during steps 1-3 (slab 0 with step 1's loads,
@@ -67,7 +67,7 @@ __host__ __device__ inline bool dispatch_fits(int E_cols, int k) {
 //     rows are loaded with that hint too (no later kernel of the forward reads
 //     them); a smaller x is still in L2 from the router and loads faster
 //     without it.
-template <typename T, bool kKBlocked, bool kNtX>
+template <typename T, bool kNtX, bool kPad>
 __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(DispatchArgs a) {
     extern __shared__ __align__(16) unsigned char s_raw[];
     // parts > 1: blocks b * parts .. b * parts + parts - 1 share chunk b, each
@@ -92,7 +92,8 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(DispatchArgs a) 
     // the copy's geometry (step 4) and the producers' slab loads
     constexpr int EPC = 16 / sizeof(T);
     const int nck = a.D / EPC;  // 16-byte chunks per row (D % 8 == 0)
-    const int nslab_all = (nck + kSlabPieces - 1) / kSlabPieces;
+    const int nckp = a.Dk / EPC;  // and per row of x_perm
+    const int nslab_all = (nckp + kSlabPieces - 1) / kSlabPieces;
     const int per_part = (nslab_all + parts - 1) / parts;
     const int sl0 = min(part * per_part, nslab_all);        // this block's first slab
     const int nslab = min(per_part, nslab_all - sl0);       // and its count (may be 0)
@@ -285,10 +286,12 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(DispatchArgs a) 
     if (producer) {
         // producers: slab sl + 1 into LDS while the consumers write slab sl;
         // four 16-byte pieces per thread, in named registers
-        auto stash = [&](int buf, int u, const uint4& v) {
+        // (slab sl; kPad: chunks past the row's end are padding, zeros)
+        auto stash = [&](int sl, int u, const uint4& v) {
             const int q = tid + u * kProdThreads;
-            *reinterpret_cast<uint4*>(slab + (buf * kRouterRows + q / kSlabPieces) * kSlabStride +
-                                      (q % kSlabPieces) * 16) = v;
+            const bool real = !kPad || (sl0 + sl) * kSlabPieces + q % kSlabPieces < nck;
+            *reinterpret_cast<uint4*>(slab + ((sl & 1) * kRouterRows + q / kSlabPieces) * kSlabStride +
+                                      (q % kSlabPieces) * 16) = real ? v : make_uint4(0, 0, 0, 0);
         };
         stash(0, 0, f0);
         stash(0, 1, f1);
@@ -296,11 +299,10 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(DispatchArgs a) 
         stash(0, 3, f3);
         __syncthreads();
         for (int sl = 0; sl < nslab; ++sl) {
-            const int buf = (sl + 1) & 1;  // slabs past the end are never read
-            stash(buf, 0, v0);
-            stash(buf, 1, v1);
-            stash(buf, 2, v2);
-            stash(buf, 3, v3);
+            stash(sl + 1, 0, v0);  // slabs past the end are never read
+            stash(sl + 1, 1, v1);
+            stash(sl + 1, 2, v2);
+            stash(sl + 1, 3, v3);
             v0 = fetch(sl + 2, 0);
             v1 = fetch(sl + 2, 1);
             v2 = fetch(sl + 2, 2);
@@ -314,48 +316,33 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(DispatchArgs a) 
         __syncthreads();
         for (int sl = 0; sl < nslab; ++sl) {
             const unsigned char* sb = slab + (sl & 1) * kRouterRows * kSlabStride;
-            if constexpr (kKBlocked) {
-                // A thread owns piece ct % kPPK of slots ct / kPPK, + kCons / kPPK,
-                // ...: for each, one position and row lookup, then the slab's
-                // K-blocks of that piece, their LDS reads all in flight before
-                // the stores (a_cap * KB elements apart).  Lanes 4i..4i+3 write
-                // slot i's 64 bytes of a K-block: one store instruction covers
-                // 16 consecutive positions.  (The slab holds whole K-blocks:
-                // the K-blocked layout needs D % KB == 0.)
-                constexpr int kKbs = kSlabPieces / kPPK;  // K-blocks per slab
-                const int piece = ct % kPPK;
-                const int kb0 = (sl0 + sl) * kKbs;
-                const int nkb = min(kKbs, nck / kPPK - kb0);
-                const int64_t kstep = a.a_cap * KB;
-                for (int pr = ct / kPPK; pr < npairs; pr += kCons / kPPK) {
-                    const int p = s_ppos[pr];
-                    if (p < 0 || p >= a.a_cap) continue;
-                    const unsigned char* src = sb + s_prow[pr] * kSlabStride + piece * 16;
-                    T* dst = xp + ((int64_t)kb0 * a.a_cap + p) * KB + piece * EPC;
-                    if (nkb == kKbs) {
-                        uint4 val[kKbs];
+            // A thread owns piece ct % kPPK of slots ct / kPPK, + kCons / kPPK,
+            // ...: for each, one position and row lookup, then the slab's
+            // K-blocks of that piece, their LDS reads all in flight before
+            // the stores (a_cap * KB elements apart).  Lanes 4i..4i+3 write
+            // slot i's 64 bytes of a K-block: one store instruction covers
+            // 16 consecutive positions.  (A slab holds whole K-blocks.)
+            constexpr int kKbs = kSlabPieces / kPPK;  // K-blocks per slab
+            const int piece = ct % kPPK;
+            const int kb0 = (sl0 + sl) * kKbs;
+            const int nkb = min(kKbs, nckp / kPPK - kb0);
+            const int64_t kstep = a.a_cap * KB;
+            for (int pr = ct / kPPK; pr < npairs; pr += kCons / kPPK) {
+                const int p = s_ppos[pr];
+                if (p < 0 || p >= a.a_cap) continue;
+                const unsigned char* src = sb + s_prow[pr] * kSlabStride + piece * 16;
+                T* dst = xp + ((int64_t)kb0 * a.a_cap + p) * KB + piece * EPC;
+                if (nkb == kKbs) {
+                    uint4 val[kKbs];
 #pragma unroll
-                        for (int q = 0; q < kKbs; ++q)
-                            val[q] = *reinterpret_cast<const uint4*>(src + q * kKBlockBytes);
+                    for (int q = 0; q < kKbs; ++q)
+                        val[q] = *reinterpret_cast<const uint4*>(src + q * kKBlockBytes);
 #pragma unroll
-                        for (int q = 0; q < kKbs; ++q) store16_nt(dst + q * kstep, val[q]);
-                    } else {
-                        for (int q = 0; q < nkb; ++q)
-                            store16_nt(dst + q * kstep,
-                                       *reinterpret_cast<const uint4*>(src + q * kKBlockBytes));
-                    }
-                }
-            } else {
-                // (slot, piece): whole 512-byte slab rows
-                const int npieces = npairs * kSlabPieces;
-                for (int v = ct; v < npieces; v += kCons) {
-                    const int pr = v / kSlabPieces, h = v % kSlabPieces;
-                    const int c = (sl0 + sl) * kSlabPieces + h;
-                    const int p = s_ppos[pr];
-                    if (c >= nck || p < 0 || p >= a.a_cap) continue;
-                    const uint4 val =
-                        *reinterpret_cast<const uint4*>(sb + s_prow[pr] * kSlabStride + h * 16);
-                    store16_nt(xp + (int64_t)p * a.D + (int64_t)c * EPC, val);
+                    for (int q = 0; q < kKbs; ++q) store16_nt(dst + q * kstep, val[q]);
+                } else {
+                    for (int q = 0; q < nkb; ++q)
+                        store16_nt(dst + q * kstep,
+                                   *reinterpret_cast<const uint4*>(src + q * kKBlockBytes));
                 }
             }
             __syncthreads();
@@ -487,19 +474,21 @@ __global__ void dense_tiles_kernel(int64_t rows, int BM, int max_tiles, TileInfo
     }
 }
 
-// x (rows x D, row-major) to the K-blocked layout of the MFMA GEMMs: one
-// 16-byte chunk per thread, coalesced reads, 64-byte runs written.
+// x (rows x D, row-major) to the K-blocked layout of the GEMMs (Dk columns,
+// zeros past D): one 16-byte chunk per thread, coalesced reads, 64-byte runs
+// written.
 template <typename T>
 __global__ __launch_bounds__(256) void kblock_kernel(const T* __restrict__ x, T* __restrict__ xk,
-                                                     int64_t rows, int D, int64_t a_cap) {
+                                                     int64_t rows, int D, int Dk, int64_t a_cap) {
     constexpr int EPC = 16 / sizeof(T);
-    const int nchunk = D / EPC;
+    const int nchunk = Dk / EPC;
     const int64_t total = rows * nchunk;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
          i += (int64_t)gridDim.x * blockDim.x) {
         const int64_t r = i / nchunk;
         const int64_t col = (i % nchunk) * EPC;
-        const uint4 v = *reinterpret_cast<const uint4*>(x + r * D + col);
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (col < D) v = *reinterpret_cast<const uint4*>(x + r * D + col);
         constexpr int KB = kblock_elems<T>();
         *reinterpret_cast<uint4*>(xk + ((col / KB) * a_cap + r) * KB + col % KB) = v;
     }
@@ -512,23 +501,23 @@ hipError_t launch_dispatch_t(const DispatchArgs& a, hipStream_t s) {
     if (a.nchunks != nblk || a.count_rows < kMinRouterBlockRows || a.count_rows > kRouterRows ||
         kRouterRows % a.count_rows != 0 || a.E_cols < 1 || a.E_cols > kMaxExperts + 1 || a.k_slots < 1 ||
         a.k_slots > a.E_cols || a.BM < 1 || !dispatch_fits(a.E_cols, a.k_slots) ||
-        (a.kblocked && (int64_t)a.D * (int64_t)sizeof(T) % kKBlockBytes != 0))
+        a.Dk != padded_k(a.D, sizeof(T)))
         return hipErrorInvalidValue;
     const size_t lds = dispatch_lds(a.E_cols, a.k_slots);
-    // the x_perm layout and the load hint as compile-time choices: no tests in
-    // the copy loop.  Nontemporal x loads: headline 14,232 rows (87 MB)
+    // the load hint and the padding as compile-time choices: no test in the copy loop.
+    // Nontemporal x loads: headline 14,232 rows (87 MB)
     // 41.9 -> 40.2 us; one 4,680-row segment (29 MB, in L2 after the router)
     // 17.6 -> 19.5 us (A/B on one box, two repeats each).
     const bool nt_x = a.rows * (int64_t)a.D * (int64_t)sizeof(T) > kL2TotalBytes;
-    auto kern = a.kblocked ? (nt_x ? dispatch_kernel<T, true, true> : dispatch_kernel<T, true, false>)
-                           : (nt_x ? dispatch_kernel<T, false, true> : dispatch_kernel<T, false, false>);
+    auto kern = a.Dk == a.D ? (nt_x ? dispatch_kernel<T, true, false> : dispatch_kernel<T, false, false>)
+                            : (nt_x ? dispatch_kernel<T, true, true> : dispatch_kernel<T, false, true>);
     hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                          (int)lds);
     if (err != hipSuccess) return err;
     // several blocks per chunk when the chunks alone would leave CUs idle
     // (the copy splits by slabs, the bookkeeping is repeated), as long as the
     // grid stays within one block per CU: more blocks than CUs measured slower
-    const int nslab = (int)((a.D * sizeof(T) + kSlabBytes - 1) / kSlabBytes);
+    const int nslab = (int)((a.Dk * sizeof(T) + kSlabBytes - 1) / kSlabBytes);
     const int parts = std::max(1, std::min({kDispCUs / nblk, nslab, kDispMaxParts}));
     launch_kernel(kern, dim3(nblk * parts), dim3(kDispThreads), lds, s, a);
     return hipGetLastError();
@@ -574,25 +563,24 @@ hipError_t launch_dense_tiles(int64_t rows, int BM, int max_tiles, TileInfo* til
     return hipGetLastError();
 }
 
-hipError_t launch_kblock(DType dt, const void* x, void* xk, int64_t rows, int D, int64_t a_cap,
-                         hipStream_t s) {
+hipError_t launch_kblock(DType dt, const void* x, void* xk, int64_t rows, int D, int Dk,
+                         int64_t a_cap, hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    if ((int64_t)D * (int64_t)dtype_size(dt) % kKBlockBytes != 0 || a_cap < rows)
-        return hipErrorInvalidValue;
-    const int64_t chunks = rows * (D / (16 / (int)dtype_size(dt)));
+    if (Dk != padded_k(D, (int)dtype_size(dt)) || a_cap < rows) return hipErrorInvalidValue;
+    const int64_t chunks = rows * (Dk / (16 / (int)dtype_size(dt)));
     const unsigned nblk = (unsigned)std::min<int64_t>((chunks + 255) / 256, 65536);
     switch (dt) {
         case DType::BF16:
             launch_kernel(kblock_kernel<__bf16>, dim3(nblk), dim3(256), 0, s,
-                          (const __bf16*)x, (__bf16*)xk, rows, D, a_cap);
+                          (const __bf16*)x, (__bf16*)xk, rows, D, Dk, a_cap);
             break;
         case DType::F16:
             launch_kernel(kblock_kernel<_Float16>, dim3(nblk), dim3(256), 0, s,
-                          (const _Float16*)x, (_Float16*)xk, rows, D, a_cap);
+                          (const _Float16*)x, (_Float16*)xk, rows, D, Dk, a_cap);
             break;
         case DType::F32:
             launch_kernel(kblock_kernel<float>, dim3(nblk), dim3(256), 0, s,
-                          (const float*)x, (float*)xk, rows, D, a_cap);
+                          (const float*)x, (float*)xk, rows, D, Dk, a_cap);
             break;
         default: return hipErrorInvalidValue;
     }

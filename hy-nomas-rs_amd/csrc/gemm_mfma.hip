@@ -39,46 +39,13 @@
 
 #include "kernels.hpp"
 #include "lds_dma.hpp"
+#include "mfma.hpp"
 #include "tile_map.hpp"
 
 namespace nomas {
 
 namespace {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-// A lane's 16-byte operand fragment (one row, 64 bytes of k per stage split
-// over the 4 lane groups) feeds kSub MFMAs: one 16x16x32 for 16-bit types,
-// four 16x16x4 for f32 (MFMA t takes element t; lane group g then holds
-// k = 4 g + t of the stage, the same for both operands).
-template <typename T> struct Mfma;
-template <> struct Mfma<__bf16> {
-    typedef bf16x8_t V;
-    static constexpr int kSub = 1;
-    static __device__ __forceinline__ f32x4_t run(V a, V b, f32x4_t c, int) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-    }
-};
-template <> struct Mfma<_Float16> {
-    typedef f16x8_t V;
-    static constexpr int kSub = 1;
-    static __device__ __forceinline__ f32x4_t run(V a, V b, f32x4_t c, int) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-    }
-};
-template <> struct Mfma<float> {
-    typedef f32x4_t V;
-    static constexpr int kSub = 4;
-    static __device__ __forceinline__ f32x4_t run(V a, V b, f32x4_t c, int t) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], b[t], c, 0, 0, 0);
-    }
-};
-
-enum { kGateUp = 0, kDown = 1 };
-
-constexpr int kStages = 4;  // LDS ring depth; the main loop is unrolled over one turn
 // Waves along the token rows of a tile: 2 (4 waves, one per SIMD, 128 x 128
 // outputs each) or 4 (8 waves, two per SIMD, 64 token rows x 128 weight rows
 // each: while one wave of a SIMD waits, the other issues MFMAs).
@@ -97,7 +64,8 @@ __device__ __forceinline__ int swz(int r) { return (r >> 1) & 3; }
 // swizzle); with stride 0 the buffer is a plain byte range [0, num_records).
 constexpr int kBufferRsrcWord3 = 0x00020000;
 
-template <typename T, int MODE, int BM, int BN, int BK, int S, int NWM>
+// kPad: the widths are padded (GemmArgs::n_out).
+template <typename T, int MODE, int BM, int BN, int BK, int S, int NWM, bool kPad>
 __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs a) {
     using V = typename Mfma<T>::V;
     constexpr int kThreads = NWM * 2 * kWave;     // NWM x 2 waves
@@ -140,7 +108,8 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
     // live row tiles (the dispatch never lists more than max_tiles); the
     // block's unit: by its time-order index, or in the tail a ticket's
     const int live = min(*a.tile_total, a.max_tiles);
-    const long long units = unit_count(live, N / BN, KT_tile / S), first_tail = tail_start(units);
+    const int turns = a.split_ws ? KT_tile / S : 1;  // (one turn: no tile is split)
+    const long long units = unit_count(live, N / BN, turns), first_tail = tail_start(units);
     long long L = time_order(blockIdx.x);
     if (L >= first_tail) {
         __shared__ int s_ticket;
@@ -151,7 +120,7 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
         if (L >= units) return;
     }
     WorkUnit wu;
-    unit_at(L, N / BN, live, KT_tile / S, &wu);
+    unit_at(L, N / BN, live, turns, &wu);
     const int mt = wu.mt, nt = wu.nt;
     const TileInfo ti = a.tiles[mt];
     const int e = ti.expert, row0 = ti.row0, nrows = ti.rows;
@@ -419,7 +388,19 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
     typedef typename std::conditional<sizeof(T) == 2, uint2, uint4>::type Raw4;
     if constexpr (MODE == kGateUp) {
         // h is written K-blocked for the down GEMM: (row, c) at
-        // ((c / BK) * a_cap + row) * BK + c % BK
+        // ((c / BK) * a_cap + row) * BK + c % BK.  Hidden units past n_out are
+        // padding: silu(0) * 0 (not their computed value, which a non-finite
+        // x row would make NaN, times the down GEMM's zero weights).
+        if (kPad && (n0 + BN) / 2 > a.n_out) {
+#pragma unroll
+            for (int i = 0; i < SN; ++i)
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    if ((n0 + wn * WN + i / 4 * 64) / 2 + i % 2 * 16 + 4 * lq + s >= a.n_out) {
+#pragma unroll
+                        for (int j = 0; j < SM; ++j) acc[i][j][s] = 0.0f;
+                    }
+        }
 #pragma unroll
         for (int p = 0; p < SN / 4; ++p) {
 #pragma unroll
@@ -436,9 +417,7 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                     for (int s = 0; s < 4; ++s) {
                         const float g = acc[4 * p + b][j][s];
                         const float u = acc[4 * p + b + 2][j][s];
-                        // silu(g) * u; the reciprocal (1 ulp) and the exponential
-                        // add a few f32 ulps, far inside the output tolerance
-                        hv[s] = Elt<T>::from_f32(g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u);
+                        hv[s] = Elt<T>::from_f32(swiglu<T>(g, u));
                     }
                     Raw4 raw;
                     __builtin_memcpy(&raw, hv, sizeof(raw));
@@ -500,8 +479,9 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                     const int q = tid + (g0 + u) * kThreads;
                     const int sr = q / kRowChunks, ch = q % kRowChunks;
                     const int tr = (sr / kWR) * WM + rd * kWR + sr % kWR;
-                    if (tr < nrows) {
-                        T* dst = out + (int64_t)(row0 + tr) * N + n0 + ch * EPC;
+                    // (n_out % 8 == 0: a piece is whole or padding)
+                    if (tr < nrows && (!kPad || n0 + ch * EPC < a.n_out)) {
+                        T* dst = out + (int64_t)(row0 + tr) * (kPad ? a.n_out : N) + n0 + ch * EPC;
                         if (a.out_nt) store16_nt(dst, v[u]);
                         else *reinterpret_cast<uint4*>(dst) = v[u];
                     }
@@ -521,32 +501,42 @@ hipError_t launch_mfma_t(const GemmArgs& a, hipStream_t s) {
     // whole column tiles, and whole turns of the ring in K
     constexpr int BK = kblock_elems<T>();
     if (a.N % BN != 0 || a.K % (BK * kStages) != 0) return hipErrorInvalidValue;
-    if (a.split_ws == nullptr || a.split_cnt == nullptr || a.tail_cnt == nullptr)
-        return hipErrorInvalidValue;
+    if (a.split_cnt == nullptr || a.tail_cnt == nullptr) return hipErrorInvalidValue;
+    const int n_cols = MODE == kGateUp ? a.N / 2 : a.N;
+    if (a.n_out < 1 || a.n_out > n_cols || (MODE == kDown && a.n_out % 8 != 0)) return hipErrorInvalidValue;
     // whole tiles, plus one round for the K-split units of a short last round
     static_assert(kSplitUnits == kRound, "the split units fill one round");
     const int64_t grid = tile_grid(a.max_tiles, a.N / BN) + kSplitUnits;
     if (a.max_tiles <= 0) return hipSuccess;
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
-    launch_kernel((gemm_mfma_kernel<T, MODE, BM, BN, BK, kStages, kWaveRows>), dim3((unsigned)grid),
-                  dim3(kWaveRows * 2 * kWave), 0, s, a);
+    const dim3 g((unsigned)grid), b(kWaveRows * 2 * kWave);
+    if (a.n_out == n_cols)
+        launch_kernel((gemm_mfma_kernel<T, MODE, BM, BN, BK, kStages, kWaveRows, false>), g, b, 0, s, a);
+    else
+        launch_kernel((gemm_mfma_kernel<T, MODE, BM, BN, BK, kStages, kWaveRows, true>), g, b, 0, s, a);
     return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_gemm_gate_up_mfma(DType dt, const GemmArgs& a, hipStream_t s) {
-    if (dt == DType::BF16) return launch_mfma_t<__bf16, kGateUp>(a, s);
-    if (dt == DType::F16) return launch_mfma_t<_Float16, kGateUp>(a, s);
-    if (dt == DType::F32) return launch_mfma_t<float, kGateUp>(a, s);
+hipError_t launch_gemm_mfma(DType dt, bool gate_up, const GemmArgs& a, hipStream_t s) {
+    switch (dt) {
+        case DType::F32: return gate_up ? launch_mfma_t<float, kGateUp>(a, s) : launch_mfma_t<float, kDown>(a, s);
+        case DType::BF16: return gate_up ? launch_mfma_t<__bf16, kGateUp>(a, s) : launch_mfma_t<__bf16, kDown>(a, s);
+        case DType::F16:
+            return gate_up ? launch_mfma_t<_Float16, kGateUp>(a, s) : launch_mfma_t<_Float16, kDown>(a, s);
+    }
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_gemm_down_mfma(DType dt, const GemmArgs& a, hipStream_t s) {
-    if (dt == DType::BF16) return launch_mfma_t<__bf16, kDown>(a, s);
-    if (dt == DType::F16) return launch_mfma_t<_Float16, kDown>(a, s);
-    if (dt == DType::F32) return launch_mfma_t<float, kDown>(a, s);
-    return hipErrorInvalidValue;
+hipError_t launch_gemm_gate_up(DType dt, const GemmArgs& a, const GemmPlan& plan, hipStream_t s) {
+    return plan.waves1 ? launch_gemm_rows(dt, true, a, plan.bm, plan.waves1, s)
+                       : launch_gemm_mfma(dt, true, a, s);
+}
+
+hipError_t launch_gemm_down(DType dt, const GemmArgs& a, const GemmPlan& plan, hipStream_t s) {
+    return plan.waves2 ? launch_gemm_rows(dt, false, a, plan.bm, plan.waves2, s)
+                       : launch_gemm_mfma(dt, false, a, s);
 }
 
 }  // namespace nomas

@@ -1,0 +1,221 @@
+// Grouped expert GEMMs for calls of few rows (bf16 / f16 / f32 in, f32
+// accumulate): the same operands, layouts and epilogues as gemm_mfma.hip, on
+// tiles of 16 NT token rows x 64 weight rows.
+//
+// What bounds these calls is the weights' way from HBM (few rows per expert)
+// or how few 256 x 256 tiles there are (small widths), so the work is split
+// finely and nothing waits for anything:
+//  - A block's NW waves take the same tile, each its own 1/NW of the k steps;
+//    the waves' partial sums meet in LDS once, at the end, and are added in
+//    wave order.  There is no barrier in the k loop.  With one wave (padded
+//    widths) a tile's sums run in gemm_mfma's order, from the bias through
+//    ascending k with the same MFMAs: results then do not depend on which of
+//    the two kernels, and so on how many rows, a call has.
+//  - Operands go straight from global memory to registers: K-blocked, the 16
+//    rows x 64 bytes of one MFMA fragment are 1 KB of consecutive memory, read
+//    by one instruction, and no other wave of the block needs them.  A ring
+//    of P steps of fragments per wave is in flight.
+//  - Units run weight tile by weight tile, the row tiles of one expert next to
+//    each other, in eight contiguous shares, one per XCD (block i runs on XCD
+//    i % 8): the row tiles of an expert then find its weights in their XCD's
+//    L2.
+// Measured (gate/up + down, one MI355X, against gemm_mfma's 256 x 256 tiles or,
+// for padded widths, the earlier vector-unit kernel): 16 rows of 8 experts of
+// 1536 x 4096 in bf16 37 + 47 -> 28 + 16 us (7.0 and 6.2 TB/s of weights); 64
+// rows 41 + 52 -> 34 + 20 us; 512 rows of 512 x 1024, 4 experts, 36 + 29 -> 13 +
+// 9 us; 208 rows of 64 x 128 in f32, 4 experts, 19 + 20 -> 5 + 5 us.
+#include <type_traits>
+
+#include "kernels.hpp"
+#include "mfma.hpp"
+
+namespace nomas {
+
+namespace {
+
+constexpr int kRowsBN = 64;  // weight rows per tile: 32 gate + 32 up rows, or 64 down rows
+
+template <typename T, int MODE, int NT, int NW>
+__global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
+    using V = typename Mfma<T>::V;
+    constexpr int BM = 16 * NT, BN = kRowsBN, NB = BN / 16;
+    constexpr int BK = kblock_elems<T>();
+    constexpr int kSub = Mfma<T>::kSub;
+    // steps in flight per wave
+    constexpr int P = NW == 1 ? (NT == 1 ? 8 : NT == 2 ? 6 : 4) : (NT <= 2 ? 4 : 3);
+    __shared__ f32x4_t s_part[NW][NB][NT][kWave];
+
+    const int N = a.N, K = a.K;
+    const int live = min(*a.tile_total, a.max_tiles);
+    // down: weight tiles past the real columns have nothing to store
+    const int ntn = (int)((MODE == kDown ? a.n_out + BN - 1 : N) / BN);
+    const long long units = (long long)live * ntn;
+    const long long share = (units + kNumXcd - 1) / kNumXcd;
+    const long long q = blockIdx.x / kNumXcd, u = (blockIdx.x % kNumXcd) * share + q;
+    if (q >= share || u >= units) return;
+    const int mt = (int)(u % live), n0 = (int)(u / live) * BN;
+    const TileInfo ti = a.tiles[mt];
+    const int e = ti.expert, row0 = ti.row0, nrows = ti.rows;
+    if (e < 0 || e >= a.num_experts || nrows < 1 || nrows > BM || row0 < 0 ||
+        row0 + (int64_t)nrows > a.a_cap)
+        return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, lq = lane >> 4;
+
+    // this wave's k steps (none in gate/up tiles that hold padding only)
+    const int kt_all = K / BK;
+    const bool pad_tile = MODE == kGateUp && n0 / 2 >= a.n_out;
+    const int s0 = pad_tile ? 0 : kt_all * wave / NW, s1 = pad_tile ? 0 : kt_all * (wave + 1) / NW;
+    const int64_t wstep = (int64_t)N * BK, xstep = a.a_cap * BK;
+    const T* Wt = static_cast<const T*>(a.W) + ((int64_t)e * kt_all * N + n0) * BK;
+    const T* Xt = static_cast<const T*>(a.X) + (int64_t)row0 * BK;
+    const uint32_t woff = (uint32_t)(l16 * kKBlockBytes + lq * 16);
+    uint32_t xoff[NT];  // rows past the tile's end read its last row (never stored)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+        xoff[j] = (uint32_t)(min(j * 16 + l16, nrows - 1) * kKBlockBytes + lq * 16);
+
+    auto bias = [&](int i) -> f32x4_t {
+        const float4 b = *reinterpret_cast<const float4*>(a.bias + (int64_t)e * N + n0 + i * 16 + 4 * lq);
+        return f32x4_t{b.x, b.y, b.z, b.w};
+    };
+    f32x4_t acc[NB][NT];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = NW == 1 ? bias(i) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    V fa[P][NB], fb[P][NT];
+    auto fetch = [&](int s, V (&wa)[NB], V (&xb)[NT]) {  // past the end: the last step again
+        const int st = max(min(s, s1 - 1), 0);
+        const char* w = reinterpret_cast<const char*>(Wt + st * wstep);
+        const char* x = reinterpret_cast<const char*>(Xt + st * xstep);
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+            wa[i] = *reinterpret_cast<const V*>(w + i * 16 * kKBlockBytes + woff);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) xb[j] = *reinterpret_cast<const V*>(x + xoff[j]);
+    };
+#pragma unroll
+    for (int p = 0; p < P; ++p) fetch(s0 + p, fa[p], fb[p]);
+    for (int st = s0; st < s1; st += P) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            if (st + p < s1) {
+#pragma unroll
+                for (int t = 0; t < kSub; ++t)
+#pragma unroll
+                    for (int i = 0; i < NB; ++i)
+#pragma unroll
+                        for (int j = 0; j < NT; ++j)
+                            acc[i][j] = Mfma<T>::run(fa[p][i], fb[p][j], acc[i][j], t);
+            }
+            fetch(st + p + P, fa[p], fb[p]);
+        }
+    }
+    // Epilogue.  Lane (l16, lq) of block (i, j) holds token row 16 j + l16 and
+    // weight rows 16 i + 4 lq + (0..3).  Blocks (i, j) and (i + 2, j) finish
+    // together: a gate block and its up block, or two blocks of down columns.
+    T* out = static_cast<T*>(a.out);
+    typedef typename std::conditional<sizeof(T) == 2, uint2, uint4>::type Raw4;
+    auto finish = [&](int i, int j, const f32x4_t (&v)[2]) {
+        const int m = j * 16 + l16;
+        if (m >= nrows) return;
+        if constexpr (MODE == kGateUp) {
+            const int hc = n0 / 2 + i * 16 + 4 * lq;
+            T hv[4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                hv[s] = hc + s < a.n_out ? Elt<T>::from_f32(swiglu<T>(v[0][s], v[1][s]))
+                                         : Elt<T>::from_f32(0.0f);
+            Raw4 raw;
+            __builtin_memcpy(&raw, hv, sizeof(raw));
+            *reinterpret_cast<Raw4*>(out + ((int64_t)(hc / BK) * a.a_cap + row0 + m) * BK + hc % BK) = raw;
+        } else {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int n = n0 + (i + 2 * h) * 16 + 4 * lq;
+                if (n >= a.n_out) continue;  // (n_out % 8 == 0: 4 columns are real or padding)
+                T ov[4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s) ov[s] = Elt<T>::from_f32(v[h][s]);
+                Raw4 raw;
+                __builtin_memcpy(&raw, ov, sizeof(raw));
+                *reinterpret_cast<Raw4*>(out + (int64_t)(row0 + m) * a.n_out + n) = raw;
+            }
+        }
+    };
+    if constexpr (NW == 1) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const f32x4_t v[2] = {acc[i][j], acc[i + 2][j]};
+                finish(i, j, v);
+            }
+    } else {
+        // the waves' partial sums in wave order; wave w takes pairs w, w + NW, ...
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) s_part[wave][i][j][lane] = acc[i][j];
+        __syncthreads();
+        for (int it = wave; it < 2 * NT; it += NW) {
+            const int i = it & 1, j = it >> 1;
+            f32x4_t v[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                f32x4_t t = s_part[0][i + 2 * h][j][lane];
+#pragma unroll
+                for (int w = 1; w < NW; ++w) t += s_part[w][i + 2 * h][j][lane];
+                v[h] = t + bias(i + 2 * h);
+            }
+            finish(i, j, v);
+        }
+    }
+}
+
+template <typename T, int MODE, int NT, int NW>
+hipError_t launch_rows_t(const GemmArgs& a, hipStream_t s) {
+    const int n_cols = MODE == kGateUp ? a.N / 2 : a.N;
+    if (a.N % kMfmaBN != 0 || a.K % (kblock_elems<T>() * kStages) != 0 || a.n_out < 1 || a.n_out > n_cols ||
+        (MODE == kDown && a.n_out % 8 != 0))
+        return hipErrorInvalidValue;
+    if (a.max_tiles <= 0) return hipSuccess;
+    const int64_t ntn = (MODE == kDown ? a.n_out + kRowsBN - 1 : a.N) / kRowsBN;
+    const int64_t grid = round_up((int64_t)a.max_tiles * ntn, kNumXcd);
+    if (grid > 0x7fffffff) return hipErrorInvalidValue;
+    launch_kernel((gemm_rows_kernel<T, MODE, NT, NW>), dim3((unsigned)grid), dim3(NW * kWave), 0, s, a);
+    return hipGetLastError();
+}
+
+template <typename T, int MODE>
+hipError_t launch_rows(const GemmArgs& a, int bm, int waves, hipStream_t s) {
+    switch (bm * 100 + waves) {
+        case 1601: return launch_rows_t<T, MODE, 1, 1>(a, s);
+        case 3201: return launch_rows_t<T, MODE, 2, 1>(a, s);
+        case 6401: return launch_rows_t<T, MODE, 4, 1>(a, s);
+        case 1604: return launch_rows_t<T, MODE, 1, 4>(a, s);
+        case 3204: return launch_rows_t<T, MODE, 2, 4>(a, s);
+        case 6404: return launch_rows_t<T, MODE, 4, 4>(a, s);
+        case 6402: return launch_rows_t<T, MODE, 4, 2>(a, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+hipError_t launch_gemm_rows(DType dt, bool gate_up, const GemmArgs& a, int bm, int waves, hipStream_t s) {
+    switch (dt) {
+        case DType::F32:
+            return gate_up ? launch_rows<float, kGateUp>(a, bm, waves, s) : launch_rows<float, kDown>(a, bm, waves, s);
+        case DType::BF16:
+            return gate_up ? launch_rows<__bf16, kGateUp>(a, bm, waves, s) : launch_rows<__bf16, kDown>(a, bm, waves, s);
+        case DType::F16:
+            return gate_up ? launch_rows<_Float16, kGateUp>(a, bm, waves, s)
+                           : launch_rows<_Float16, kDown>(a, bm, waves, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace nomas

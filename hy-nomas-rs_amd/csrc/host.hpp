@@ -137,19 +137,19 @@ int st_to_f32(const StTensor& t, std::vector<float>* out);
 // by one forward are where the next one looks for them.
 struct Workspace {
     int64_t cap_rows = 0;  // rows the buffers are laid out for (a multiple of 64)
-    int32_t* split_cnt = nullptr;    // MFMA path: arrival counters of K-split tiles
-    float* split_ws = nullptr;       // MFMA path: their f32 partial tiles
+    int32_t* split_cnt = nullptr;    // arrival counters of K-split tiles
+    float* split_ws = nullptr;       // their f32 partial tiles (null: no tile is split)
     int32_t* idx = nullptr;          // rows x k_slots
     float* w = nullptr;              // rows x k_slots
     float* gap = nullptr;            // rows
     int32_t* pos = nullptr;          // rows x k_slots
     int32_t* chunk_counts = nullptr; // chunks x E_cols
-    int32_t* expert_count = nullptr; // E_cols
+    int32_t* expert_count = nullptr; // E_cols, for each piece of the forward
     int32_t* expert_off = nullptr;   // E_cols + 1
     TileInfo* tiles = nullptr;       // max_tiles
     int32_t* tile_total = nullptr;   // 3: tile count, the GEMMs' tail counters
-    void* xperm = nullptr;           // a_cap x D
-    void* h = nullptr;               // a_cap x H
+    void* xperm = nullptr;           // a_cap x Dk (D padded, K-blocked)
+    void* h = nullptr;               // a_cap x Hp (H padded, K-blocked)
     void* yperm = nullptr;           // a_cap x D (MoE only)
     void* block_h = nullptr;         // forward_block: rows x D
 };
@@ -233,24 +233,36 @@ public:
     int64_t experts() const { return E_; }
     int64_t top_k() const { return k_; }
     DType dtype() const { return dt_; }
-    bool uses_mfma() const { return mfma_; }
+    // whether the widths are whole GEMM tiles (no operand is padded)
+    bool uses_mfma() const { return tiled_; }
     bool dense_only() const { return dense_only_; }
 
 private:
     int ensure_workspace(int64_t rows);
     void free_workspace();
+    // The GEMM kernels of a forward on `rows` rows.  The pieces of one call all
+    // take the plan of the whole call (plan_rows_), so that its rows are
+    // summed as in one forward.
+    GemmPlan gemm_plan(int64_t rows) const;
+    int64_t plan_rows_ = 0;  // rows of the pieced call in progress, else 0
     int max_tiles(int64_t rows) const;
     // Lays out the buffers of a forward on up to `cap` rows (a multiple of
     // 64) from `base` (nullptr: sizes only) and returns the bytes used.
-    size_t layout(int64_t cap, bool block, uint8_t* base, Workspace* w) const;
+    // `route_cap` (0: cap): rows of the routing, when the forward runs in
+    // pieces of `cap` rows.
+    size_t layout(int64_t cap, bool block, uint8_t* base, Workspace* w, int64_t route_cap = 0) const;
+    // The bytes that decide whether a no-allocation forward is taken: those of
+    // layout() with x_perm and h unpadded.
+    size_t scratch_need(int64_t cap) const;
 
     int64_t D_, H_, E_, k_;
     int64_t Ecols_, kslots_;  // with the shared dense branch: E + 1, k + 1
     double shared_dense_;
     DType dt_;
     int device_;
-    bool mfma_;
-    int BM_;
+    bool tiled_;  // D and H are whole GEMM tiles
+    // D and H as the GEMMs see them: K to whole ring turns, weight rows to whole tiles
+    int64_t Dk_, Dn_, Hp_;
     bool dense_only_ = false;
     int forward_dense(const void* x, void* y, int64_t rows, hipStream_t s);
     int check_forward(const void* x, const void* y, int64_t rows) const;
@@ -258,15 +270,16 @@ private:
     // the stages of a routed forward on the buffers of `w`
     int run_routed(const void* x, void* y, int64_t rows, hipStream_t s, const BlockArgs* blk,
                    const Workspace& w);
-    int finish_forward(int64_t rows, hipStream_t s, const Workspace& w);
+    int finish_forward(int64_t rows, hipStream_t s, const Workspace& w, int scratch_pieces = 1);
+    void set_widths();
     bool want_block_ = false;  // the workspace holds h for forward_block
 
     // device weights
     void* d_wr_ = nullptr;
-    void* d_w1_ = nullptr;    // gate/up: MFMA packed [Ecols][2H][D], else [Ecols][2][H][D]
-    float* d_b1_ = nullptr;   // matching layout, f32
-    void* d_w2_ = nullptr;    // down [Ecols][D][H]
-    float* d_b2_ = nullptr;   // [Ecols][D]
+    void* d_w1_ = nullptr;    // gate/up, K-blocked: [Ecols][Dk / KB][2 Hp][KB]
+    float* d_b1_ = nullptr;   // [Ecols][2 Hp], f32
+    void* d_w2_ = nullptr;    // down, K-blocked: [Ecols][Hp / KB][Dn][KB]
+    float* d_b2_ = nullptr;   // [Ecols][Dn]
 
     // the handle's workspace (sized for ws_.cap_rows rows)
     void* d_ws_ = nullptr;
@@ -292,7 +305,9 @@ private:
     // [rows][k_slots], gap [rows], then each piece's expert counts [E_cols]
     void* d_route_ = nullptr;
     size_t route_bytes_ = 0;
-    int host_pieces_ = 0;  // pieces of the last forward when it was pieced, else 0
+    int host_pieces_ = 0;  // pieces of the last forward when it was a pieced host one, else 0
+    // pieces of the last no-allocation forward: counts of each in last_ws_.expert_count
+    int scratch_pieces_ = 1;
 
     int64_t last_rows_ = -1;
     hipStream_t last_stream_ = nullptr;

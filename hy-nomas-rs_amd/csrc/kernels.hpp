@@ -43,10 +43,9 @@ inline void launch_kernel(F kernel, dim3 grid, dim3 block, uint32_t lds, hipStre
     hipExtLaunchKernelGGL(kernel, grid, block, lds, s, start, stop, 0u, args...);
 }
 
-// Tile height (token rows) of the MFMA and of the general grouped GEMM.
+// Output tile of the grouped GEMMs: token rows and weight rows.
 constexpr int kMfmaBM = 256;
 constexpr int kMfmaBN = 256;
-constexpr int kSimtBM = 64;
 
 // The FFN half of a DiT block around the MoE (block.rs:96-101):
 //   h   = modulate(norm2(x), shift, scale)   (norm.rs:55-65, modulate.rs:69-79)
@@ -82,15 +81,26 @@ struct RouterArgs {
 };
 
 
-// K-blocked layout (MFMA path): a matrix of R rows and K columns is stored as
+// K-blocked layout: a matrix of R rows and K columns is stored as
 // column blocks of KB = 64 bytes of elements (32 for 16-bit types, 16 for
 // f32), each R rows x KB contiguous elements, i.e. element (r, k) at
 // ((k / KB) * R + r) * KB + k % KB.  One k step of a GEMM tile (256 rows x
 // 64 bytes) is then a single contiguous 16 KB run of memory, fetched as whole
 // 128-byte lines.
+//
+// Any dim and hidden width run on the same GEMMs: the operands are padded with
+// zeros when they are laid out (weights at upload, x_perm by the dispatch, h
+// by the gate/up epilogue), K to whole turns of the GEMM's LDS ring and the
+// weight rows to whole tiles, so no GEMM loop has a remainder.
 constexpr int kKBlockBytes = 64;
+constexpr int kStages = 4;  // K steps (K-blocks) per turn of the ring
 template <typename T>
 __host__ __device__ constexpr int kblock_elems() { return kKBlockBytes / (int)sizeof(T); }
+__host__ __device__ constexpr int64_t round_up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
+// Columns of a K-blocked operand with K = `k` columns of es-byte elements.
+__host__ __device__ constexpr int64_t padded_k(int64_t k, int es) {
+    return round_up(k, kStages * kKBlockBytes / es);
+}
 
 struct DispatchArgs {
     const void* x;
@@ -107,9 +117,9 @@ struct DispatchArgs {
     TileInfo* tiles;        // max_tiles
     int32_t* tile_total;    // 3: the tile count, then the two GEMMs' tail counters (cleared)
     int32_t* tok_pos;  // rows x k_slots
-    void* x_perm;      // a_cap x D, row-major or K-blocked
+    void* x_perm;      // a_cap x Dk, K-blocked (R = a_cap)
+    int Dk;            // padded_k(D): columns D .. Dk - 1 are written as zeros
     int64_t a_cap;     // rows of x_perm (positions must stay below)
-    int kblocked;      // 1: write x_perm K-blocked (R = a_cap), 0: row-major
 };
 
 struct GemmArgs {
@@ -120,19 +130,23 @@ struct GemmArgs {
     const TileInfo* tiles;
     const int32_t* tile_total;
     int max_tiles;
-    int N;  // output columns of the weight GEMM (2H for gate/up, D for down)
-    int K;
+    int N;  // weight rows, whole tiles (2 x padded H for gate/up, padded D for down)
+    int K;  // padded to whole ring turns
+    // real output columns: H (hidden units past it are written as zeros, which
+    // the down GEMM multiplies with zero weights) or D (columns past it are not
+    // stored; also the row stride of out)
+    int n_out;
     int num_experts;  // experts with weights (tiles naming others are skipped)
     int64_t a_cap;    // rows of X / out (tiles reaching beyond are skipped)
-    // MFMA path: f32 partial sums of tiles split along K (kSplitUnits units of
-    // kSplitUnitFloats each) and one arrival counter per split tile (zero
-    // between launches: the last part to arrive resets it)
+    // f32 partial sums of tiles split along K (kSplitUnits units of
+    // kSplitUnitFloats each; null: no tile is split) and one arrival counter per
+    // split tile (zero between launches: the last part to arrive resets it)
     float* split_ws;
     int32_t* split_cnt;
-    // MFMA path: the ticket counter of the tail units handed out at run time
+    // the ticket counter of the tail units handed out at run time
     // (zero before the launch: the kernel that writes the tile table clears it)
     int32_t* tail_cnt = nullptr;
-    // down GEMM (MFMA path): write `out` with the nontemporal hint.  For
+    // down GEMM: write `out` with the nontemporal hint.  For
     // outputs larger than the chip's last-level cache, which the combine reads
     // back once: their lines then go to HBM as they are written instead of
     // being evicted dirty while the combine streams them in.
@@ -145,6 +159,12 @@ constexpr int64_t kL2TotalBytes = (int64_t)32 << 20;
 // One split unit's partial tile: 256 x 256 f32.
 constexpr int64_t kSplitUnitFloats = 256 * 256;
 constexpr int kSplitUnits = 256;
+
+// Which kernels run a forward's two GEMMs (gemm_plan.hpp).
+struct GemmPlan {
+    int bm;              // token rows per tile of the tile table
+    int waves1, waves2;  // gate/up, down: waves per block of gemm_rows, 0: gemm_mfma
+};
 
 struct CombineArgs {
     const void* y_perm;
@@ -180,19 +200,19 @@ hipError_t launch_gated_residual(DType dt, const void* x, const void* y, const f
                                  void* out, int64_t rows, int D, int64_t seq, hipStream_t s);
 hipError_t launch_router(DType dt, const RouterArgs& a, hipStream_t s);
 hipError_t launch_dispatch(DType dt, const DispatchArgs& a, hipStream_t s);
-// MFMA grouped GEMMs (bf16 / f16): W packed as described in moe_layer.cpp.
-hipError_t launch_gemm_gate_up_mfma(DType dt, const GemmArgs& a, hipStream_t s);
-hipError_t launch_gemm_down_mfma(DType dt, const GemmArgs& a, hipStream_t s);
-// General grouped GEMMs (any dtype, any shape).
-hipError_t launch_gemm_gate_up_simt(DType dt, const GemmArgs& a, hipStream_t s);
-hipError_t launch_gemm_down_simt(DType dt, const GemmArgs& a, hipStream_t s);
+// Grouped GEMMs: W packed as described in moe_layer.cpp, the tile table in
+// tiles of plan.bm rows.
+hipError_t launch_gemm_gate_up(DType dt, const GemmArgs& a, const GemmPlan& plan, hipStream_t s);
+hipError_t launch_gemm_down(DType dt, const GemmArgs& a, const GemmPlan& plan, hipStream_t s);
+hipError_t launch_gemm_mfma(DType dt, bool gate_up, const GemmArgs& a, hipStream_t s);
+hipError_t launch_gemm_rows(DType dt, bool gate_up, const GemmArgs& a, int bm, int waves, hipStream_t s);
 hipError_t launch_combine(DType dt, const CombineArgs& a, hipStream_t s);
 // Dense feed-forward (no routing): the tile table of `rows` rows of one
 // expert in BM-row tiles (max_tiles entries written), and x re-laid out
-// K-blocked ((col / 32) * a_cap + row) * 32 + col % 32 for the MFMA GEMM.
+// K-blocked with Dk = padded_k(D) columns for the gate/up GEMM.
 hipError_t launch_dense_tiles(int64_t rows, int BM, int max_tiles, TileInfo* tiles,
                               int32_t* tile_total, hipStream_t s);
-hipError_t launch_kblock(DType dt, const void* x, void* xk, int64_t rows, int D, int64_t a_cap,
-                         hipStream_t s);
+hipError_t launch_kblock(DType dt, const void* x, void* xk, int64_t rows, int D, int Dk,
+                         int64_t a_cap, hipStream_t s);
 
 }  // namespace nomas

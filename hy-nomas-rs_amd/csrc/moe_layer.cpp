@@ -13,8 +13,10 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
+#include "gemm_plan.hpp"
 #include "host.hpp"
 
 namespace nomas {
@@ -41,6 +43,33 @@ struct DeviceGuard {
         if (prev >= 0) (void)hipSetDevice(prev);
     }
 };
+
+// Sets a member for the time of a call.
+struct Scoped {
+    int64_t& v;
+    Scoped(int64_t& v_, int64_t n) : v(v_) { v = n; }
+    ~Scoped() { v = 0; }
+};
+
+// Runs fn(begin, end) over [0, n), on a few threads when there are enough
+// bytes to move (a thread that cannot be started: its part runs here).
+template <typename F>
+void over_rows(int64_t n, size_t bytes, const F& fn) {
+    const unsigned hw = std::thread::hardware_concurrency();
+    const int parts = bytes < ((size_t)1 << 20) ? 1 : (int)std::max(1u, std::min(8u, hw / 2));
+    std::vector<std::thread> ts;
+    ts.reserve((size_t)parts);
+    for (int p = 1; p < parts; ++p) {
+        const int64_t b = n * p / parts, e = n * (p + 1) / parts;
+        try {
+            ts.emplace_back([&fn, b, e] { fn(b, e); });
+        } catch (...) {
+            fn(b, e);
+        }
+    }
+    fn(0, n / parts);
+    for (std::thread& t : ts) t.join();
+}
 
 inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
@@ -106,8 +135,7 @@ MoeLayer::MoeLayer(const nomas_moe_config& cfg, int64_t dim, int64_t hidden, DTy
     const bool dense = cfg.shared_dense > 0.0;
     Ecols_ = E_ + (dense ? 1 : 0);
     kslots_ = k_ + (dense ? 1 : 0);
-    mfma_ = D_ % kMfmaBN == 0 && H_ % (kMfmaBN / 2) == 0;
-    BM_ = mfma_ ? kMfmaBM : kSimtBM;
+    set_widths();
 }
 
 MoeLayer::MoeLayer(DenseTag, int64_t dim, int64_t hidden, DType dt, int device)
@@ -115,8 +143,16 @@ MoeLayer::MoeLayer(DenseTag, int64_t dim, int64_t hidden, DType dt, int device)
     Ecols_ = 1;
     kslots_ = 1;
     dense_only_ = true;
-    mfma_ = D_ % kMfmaBN == 0 && H_ % (kMfmaBN / 2) == 0;
-    BM_ = mfma_ ? kMfmaBM : kSimtBM;
+    set_widths();
+}
+
+void MoeLayer::set_widths() {
+    const int es = (int)dtype_size(dt_);
+    tiled_ = D_ % kMfmaBN == 0 && H_ % (kMfmaBN / 2) == 0;
+    Dk_ = padded_k(D_, es);
+    Dn_ = round_up(D_, kMfmaBN);
+    Hp_ = round_up(H_, kMfmaBN / 2);  // 2 Hp: whole tiles of gate/up rows, and whole ring turns
+    static_assert(kMfmaBN / 2 * 2 % (kStages * kKBlockBytes) == 0, "also whole turns of 16-bit columns");
 }
 
 MoeLayer::~MoeLayer() {
@@ -179,52 +215,39 @@ int MoeLayer::upload(const void* router_w, const void* gate_w, const void* gate_
     // the end-of-forward event, made here so that no forward creates anything
     if (!done_) HIP_TRY(hipEventCreateWithFlags(&done_, kDoneFlags));
 
-    // gate/up
-    std::vector<uint8_t> w1((size_t)(Ecols_ * 2 * H * D) * es);
-    std::vector<float> b1((size_t)(Ecols_ * 2 * H));
-    for (int64_t e = 0; e < Ecols_; ++e) {
-        const uint8_t* gw = wsrc(gate_w, dg_w, e, H * D);
-        const uint8_t* uw = wsrc(up_w, du_w, e, H * D);
-        for (int64_t p = 0; p < 2 * H; ++p) {
-            int64_t src_row;
-            bool is_up;
-            if (mfma_) {  // rows 64g..64g+31 gate 32g.., rows 64g+32.. up 32g..
-                const int64_t grp = p / 64, w = p % 64;
-                is_up = w >= 32;
-                src_row = grp * 32 + (w % 32);
-            } else {      // [gate rows][up rows]
-                is_up = p >= H;
-                src_row = p % H;
-            }
-            const uint8_t* src = (is_up ? uw : gw) + src_row * D * es;
-            if (mfma_) {  // K-blocked: (e, p, k) at ((e * D/KB + k/KB) * 2H + p) * KB + k % KB
-                const int64_t KB = kKBlockBytes / (int64_t)es, nkb = D / KB;
-                for (int64_t kb = 0; kb < nkb; ++kb)
-                    std::memcpy(&w1[(size_t)(((e * nkb + kb) * 2 * H + p) * KB) * es],
-                                src + kb * KB * es, (size_t)KB * es);
-            } else {
-                std::memcpy(&w1[(size_t)((e * 2 * H + p) * D) * es], src, (size_t)D * es);
-            }
-            b1[(size_t)(e * 2 * H + p)] = is_up ? bsrc(up_b, du_b, e, H, src_row)
-                                                : bsrc(gate_b, dg_b, e, H, src_row);
+    // K-blocked with zero padding: element (row, k) of an expert at
+    // ((e * nkb + k / KB) * rows + row) * KB + k % KB.
+    const int64_t KB = kKBlockBytes / (int64_t)es;
+    auto pack_row = [&](std::vector<uint8_t>& w, int64_t e, int64_t nkb, int64_t nrows, int64_t row,
+                        const uint8_t* src, int64_t k) {
+        uint8_t* dst = &w[(size_t)((e * nkb * nrows + row) * KB) * es];
+        for (int64_t k0 = 0; k0 < k; k0 += KB, dst += (size_t)(nrows * KB) * es)
+            std::memcpy(dst, src + k0 * es, (size_t)std::min(KB, k - k0) * es);
+    };
+    // gate/up: rows 64g..64g+31 gate 32g.., rows 64g+32.. up 32g..
+    std::vector<uint8_t> w1((size_t)(Ecols_ * 2 * Hp_ * Dk_) * es);
+    std::vector<float> b1((size_t)(Ecols_ * 2 * Hp_));
+    over_rows(Ecols_ * 2 * Hp_, w1.size(), [&](int64_t r0, int64_t r1) {
+        for (int64_t r = r0; r < r1; ++r) {
+            const int64_t e = r / (2 * Hp_), p = r % (2 * Hp_);
+            const bool is_up = p % 64 >= 32;
+            const int64_t src_row = p / 64 * 32 + p % 32;
+            if (src_row >= H) continue;
+            pack_row(w1, e, Dk_ / KB, 2 * Hp_, p,
+                     (is_up ? wsrc(up_w, du_w, e, H * D) : wsrc(gate_w, dg_w, e, H * D)) + src_row * D * es, D);
+            b1[(size_t)r] = is_up ? bsrc(up_b, du_b, e, H, src_row) : bsrc(gate_b, dg_b, e, H, src_row);
         }
-    }
+    });
     // down
-    std::vector<uint8_t> w2((size_t)(Ecols_ * D * H) * es);
-    std::vector<float> b2((size_t)(Ecols_ * D));
-    for (int64_t e = 0; e < Ecols_; ++e) {
-        const uint8_t* src = wsrc(down_w, dd_w, e, D * H);
-        if (mfma_) {  // K-blocked: (e, n, k) at ((e * H/KB + k/KB) * D + n) * KB + k % KB
-            const int64_t KB = kKBlockBytes / (int64_t)es, nkb = H / KB;
-            for (int64_t n = 0; n < D; ++n)
-                for (int64_t kb = 0; kb < nkb; ++kb)
-                    std::memcpy(&w2[(size_t)(((e * nkb + kb) * D + n) * KB) * es],
-                                src + (n * H + kb * KB) * es, (size_t)KB * es);
-        } else {
-            std::memcpy(&w2[(size_t)(e * D * H) * es], src, (size_t)(D * H) * es);
+    std::vector<uint8_t> w2((size_t)(Ecols_ * Dn_ * Hp_) * es);
+    std::vector<float> b2((size_t)(Ecols_ * Dn_));
+    over_rows(Ecols_ * D, w2.size(), [&](int64_t r0, int64_t r1) {
+        for (int64_t r = r0; r < r1; ++r) {
+            const int64_t e = r / D, n = r % D;
+            pack_row(w2, e, Hp_ / KB, Dn_, n, wsrc(down_w, dd_w, e, D * H) + n * H * es, H);
+            b2[(size_t)(e * Dn_ + n)] = bsrc(down_b, dd_b, e, D, n);
         }
-        for (int64_t d = 0; d < D; ++d) b2[(size_t)(e * D + d)] = bsrc(down_b, dd_b, e, D, d);
-    }
+    });
 
     for (void* p : {d_wr_, d_w1_, (void*)d_b1_, d_w2_, (void*)d_b2_})
         if (p) (void)hipFree(p);
@@ -291,15 +314,23 @@ int MoeLayer::upload_f32(const MoeParamsF32& p) {
 
 // ---- workspace --------------------------------------------------------------
 
-int MoeLayer::max_tiles(int64_t rows) const {
-    const int64_t A = rows * kslots_;
-    return (int)((A + BM_ - 1) / BM_ + Ecols_);
+GemmPlan MoeLayer::gemm_plan(int64_t rows) const {
+    return nomas::gemm_plan(dt_, std::max(rows, plan_rows_) * kslots_, Ecols_, Dk_, Hp_, D_, H_);
 }
 
-size_t MoeLayer::layout(int64_t cap, bool block, uint8_t* base, Workspace* w) const {
+int MoeLayer::max_tiles(int64_t rows) const {
+    const int64_t A = rows * kslots_;
+    const int bm = gemm_plan(rows).bm;
+    return (int)((A + bm - 1) / bm + Ecols_);
+}
+
+size_t MoeLayer::layout(int64_t cap, bool block, uint8_t* base, Workspace* w,
+                        int64_t route_cap) const {
     const int64_t A = cap * kslots_;
+    if (route_cap == 0) route_cap = cap;
+    const int64_t RA = route_cap * kslots_, pieces = (route_cap + cap - 1) / cap;
     const size_t es = dtype_size(dt_);
-    const int mt = max_tiles(cap);
+    const int mt = (int)max_gemm_tiles(A, Ecols_);
     size_t off = 0;
     auto take = [&](size_t bytes) -> uint8_t* {
         const size_t o = off;
@@ -313,25 +344,32 @@ size_t MoeLayer::layout(int64_t cap, bool block, uint8_t* base, Workspace* w) co
     // so that nothing else ever writes there: in the shared scratch array they
     // stay zero from one forward to the next, whichever layer ran before.
     v.split_cnt = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * kSplitUnits));
-    if (mfma_)
+    // (none for padded widths: their results do not depend on how the rows are
+    // split over calls)
+    if (tiled_)
         v.split_ws = reinterpret_cast<float*>(take(sizeof(float) * kSplitUnitFloats * kSplitUnits));
-    v.idx = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * A));
-    v.w = reinterpret_cast<float*>(take(sizeof(float) * A));
-    v.gap = reinterpret_cast<float*>(take(sizeof(float) * cap));
+    v.idx = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * RA));
+    v.w = reinterpret_cast<float*>(take(sizeof(float) * RA));
+    v.gap = reinterpret_cast<float*>(take(sizeof(float) * route_cap));
     v.pos = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * A));
     // one histogram per router block, of at least kMinRouterBlockRows rows
     v.chunk_counts = reinterpret_cast<int32_t*>(
         take(sizeof(int32_t) * (cap / kMinRouterBlockRows) * Ecols_));
-    v.expert_count = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * Ecols_));
+    v.expert_count = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * pieces * Ecols_));
     v.expert_off = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * (Ecols_ + 1)));
     v.tiles = reinterpret_cast<TileInfo*>(take(sizeof(TileInfo) * mt));
     v.tile_total = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * 3));  // + tail counters
-    v.xperm = take(es * A * D_);
-    v.h = take(es * A * H_);
+    v.xperm = take(es * A * Dk_);
+    v.h = take(es * A * Hp_);
     if (!dense_only_) v.yperm = take(es * A * D_);  // dense: the down GEMM writes y
     if (block) v.block_h = take(es * cap * D_);
     if (w) *w = v;
     return off;
+}
+
+size_t MoeLayer::scratch_need(int64_t cap) const {
+    const int64_t pad = (Dk_ - D_) + (Hp_ - H_);  // zero columns of x_perm and h
+    return layout(cap, false, nullptr, nullptr) - (size_t)(pad * cap * kslots_) * dtype_size(dt_);
 }
 
 void MoeLayer::free_workspace() {
@@ -351,12 +389,10 @@ int MoeLayer::ensure_workspace(int64_t rows) {
     HIP_TRY(hipMalloc(&ws, bytes));
     d_ws_ = ws;
     layout(cap, want_block_, static_cast<uint8_t*>(ws), &ws_);
-    if (mfma_) {
-        // the split-tile counters start at zero; the GEMMs keep them there.
-        // Finished before any stream (blocking or not) can use the workspace.
-        HIP_TRY(hipMemset(ws_.split_cnt, 0, sizeof(int32_t) * kSplitUnits));
-        HIP_TRY(hipDeviceSynchronize());
-    }
+    // the split-tile counters start at zero; the GEMMs keep them there.
+    // Finished before any stream (blocking or not) can use the workspace.
+    HIP_TRY(hipMemset(ws_.split_cnt, 0, sizeof(int32_t) * kSplitUnits));
+    HIP_TRY(hipDeviceSynchronize());
     return NOMAS_OK;
 }
 
@@ -425,13 +461,13 @@ int MoeLayer::forward_noalloc(const void* x, void* y, int64_t rows, hipStream_t 
     if (rc != NOMAS_OK) return rc;
     if (rows == 0) { last_rows_ = 0; last_in_scratch_ = false; return NOMAS_OK; }
     const int64_t cap = (rows + kRouterRows - 1) / kRouterRows * kRouterRows;
-    const size_t need = layout(cap, false, nullptr, nullptr);
+    const size_t need = scratch_need(cap);
     if (need > kScratchBytes) {
         // the most rows that fit, for the message
         int64_t lo = 0, hi = cap / kRouterRows;
         while (lo < hi) {
             const int64_t mid = (lo + hi + 1) / 2;
-            if (layout(mid * kRouterRows, false, nullptr, nullptr) <= kScratchBytes) lo = mid;
+            if (scratch_need(mid * kRouterRows) <= kScratchBytes) lo = mid;
             else hi = mid - 1;
         }
         return set_error(NOMAS_ERR_INVALID_ARGUMENT,
@@ -439,6 +475,21 @@ int MoeLayer::forward_noalloc(const void* x, void* y, int64_t rows, hipStream_t 
                          "holds %zu (at most %lld rows for this layer): use nomas_moe_forward",
                          (long long)rows, need, kScratchBytes, (long long)(lo * kRouterRows));
     }
+    // Widths that are padded can need more than the call's own bytes: such a
+    // call runs in row pieces that fit (each an ordinary forward over its
+    // rows; the routing of all rows is kept).
+    int64_t lo = 0, hi = cap / kRouterRows;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi + 1) / 2;
+        if (layout(mid * kRouterRows, false, nullptr, nullptr, cap) <= kScratchBytes) lo = mid;
+        else hi = mid - 1;
+    }
+    const int64_t piece = lo * kRouterRows;
+    if (piece == 0)
+        return set_error(NOMAS_ERR_INVALID_ARGUMENT,
+                         "rows=%lld do not fit the no-allocation forward's device scratch of %zu "
+                         "bytes with this layer's padded widths: use nomas_moe_forward",
+                         (long long)rows, kScratchBytes);
     DeviceGuard g(device_);
     if (!g.ok) return set_error(NOMAS_ERR_HIP, "hipSetDevice(%d) failed", device_);
     void* base = nullptr;
@@ -446,23 +497,35 @@ int MoeLayer::forward_noalloc(const void* x, void* y, int64_t rows, hipStream_t 
     rc = scratch_acquire(device_, s, &base, &gen);
     if (rc != NOMAS_OK) return rc;
     Workspace w;
-    layout(cap, false, static_cast<uint8_t*>(base), &w);
+    layout(piece, false, static_cast<uint8_t*>(base), &w, cap);
     if (done_recorded_ && s != last_stream_) HIP_TRY(hipStreamWaitEvent(s, done_, 0));
-    rc = run_routed(x, y, rows, s, nullptr, w);
-    if (rc != NOMAS_OK) {
-        last_rows_ = -1;  // as in forward_impl
-        return rc;
+    const Scoped whole(plan_rows_, rows);
+    int pieces = 0;
+    for (int64_t off = 0; off < rows; off += piece, ++pieces) {
+        Workspace p = w;
+        p.idx += off * kslots_;
+        p.w += off * kslots_;
+        p.gap += off;
+        p.expert_count += pieces * Ecols_;
+        const size_t o = (size_t)off * D_ * dtype_size(dt_);
+        rc = run_routed(static_cast<const uint8_t*>(x) + o, static_cast<uint8_t*>(y) + o,
+                        std::min(piece, rows - off), s, nullptr, p);
+        if (rc != NOMAS_OK) {
+            last_rows_ = -1;  // as in forward_impl
+            return rc;
+        }
     }
     last_in_scratch_ = true;
     last_scratch_gen_ = gen;
-    return finish_forward(rows, s, w);
+    return finish_forward(rows, s, w, pieces);
 }
 
-int MoeLayer::finish_forward(int64_t rows, hipStream_t s, const Workspace& w) {
+int MoeLayer::finish_forward(int64_t rows, hipStream_t s, const Workspace& w, int scratch_pieces) {
     // done_ is created with the weights; recording it allocates nothing
     HIP_TRY(hipEventRecord(done_, s));
     done_recorded_ = true;
     host_pieces_ = 0;  // routing() reads this forward's workspace
+    scratch_pieces_ = scratch_pieces;
     last_rows_ = rows;
     last_stream_ = s;
     last_ws_ = w;
@@ -541,7 +604,8 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     da.chunk_counts = w.chunk_counts;
     da.nchunks = nch;
     da.count_rows = ra.block_rows;
-    da.BM = BM_;
+    const GemmPlan plan = gemm_plan(rows);
+    da.BM = plan.bm;
     da.max_tiles = mt;
     da.expert_count = w.expert_count;
     da.expert_off = w.expert_off;
@@ -549,8 +613,8 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     da.tile_total = w.tile_total;
     da.tok_pos = w.pos;
     da.x_perm = w.xperm;
+    da.Dk = (int)Dk_;
     da.a_cap = a_cap;
-    da.kblocked = mfma_ ? 1 : 0;
     STAGE(launch_dispatch(dt_, da, s), "dispatch");
     if ((rc = mark(3))) return rc;
 
@@ -562,15 +626,15 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     g1.tiles = w.tiles;
     g1.tile_total = w.tile_total;
     g1.max_tiles = mt;
-    g1.N = (int)(2 * H_);
-    g1.K = (int)D_;
+    g1.N = (int)(2 * Hp_);
+    g1.K = (int)Dk_;
+    g1.n_out = (int)H_;
     g1.num_experts = (int)Ecols_;
     g1.a_cap = a_cap;
     g1.split_ws = w.split_ws;
     g1.split_cnt = w.split_cnt;
     g1.tail_cnt = w.tile_total + 1;
-    STAGE(mfma_ ? launch_gemm_gate_up_mfma(dt_, g1, s) : launch_gemm_gate_up_simt(dt_, g1, s),
-          "gate/up GEMM");
+    STAGE(launch_gemm_gate_up(dt_, g1, plan, s), "gate/up GEMM");
     if ((rc = mark(4))) return rc;
 
     GemmArgs g2 = g1;
@@ -579,11 +643,11 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     g2.bias = d_b2_;
     g2.out = w.yperm;
     g2.tail_cnt = w.tile_total + 2;
-    g2.N = (int)D_;
-    g2.K = (int)H_;
+    g2.N = (int)Dn_;
+    g2.K = (int)Hp_;
+    g2.n_out = (int)D_;
     g2.out_nt = rows * kslots_ * D_ * (int64_t)dtype_size(dt_) > kLastLevelCacheBytes;
-    STAGE(mfma_ ? launch_gemm_down_mfma(dt_, g2, s) : launch_gemm_down_simt(dt_, g2, s),
-          "down GEMM");
+    STAGE(launch_gemm_down(dt_, g2, plan, s), "down GEMM");
     if ((rc = mark(5))) return rc;
 
     CombineArgs ca;
@@ -607,11 +671,11 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
 
 // Dense feed-forward: the stages of the routed forward that remain.  Stage
 // slots for profiling: router (none), scan = tile table, dispatch = K-blocked
-// copy of x (MFMA path only), gate/up, down (written straight into y), combine
-// (none).
+// copy of x, gate/up, down (written straight into y), combine (none).
 int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s) {
     int rc;
     const Workspace& w = ws_;
+    const GemmPlan plan = gemm_plan(rows);
     const int mt = max_tiles(rows);
     hipEvent_t* ev = nullptr;
     uint8_t* empty = nullptr;
@@ -633,30 +697,28 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     } while (0)
     if ((rc = mark(0))) return rc;
     if ((rc = mark(1))) return rc;
-    STAGE(launch_dense_tiles(rows, BM_, mt, w.tiles, w.tile_total, s), "tile table");
+    STAGE(launch_dense_tiles(rows, plan.bm, mt, w.tiles, w.tile_total, s), "tile table");
     if ((rc = mark(2))) return rc;
-    // the MFMA GEMMs read K-blocked rows; the general path reads x in place
-    if (mfma_) STAGE(launch_kblock(dt_, x, w.xperm, rows, (int)D_, w.cap_rows, s), "K-blocked copy");
+    STAGE(launch_kblock(dt_, x, w.xperm, rows, (int)D_, (int)Dk_, w.cap_rows, s), "K-blocked copy");
     if ((rc = mark(3))) return rc;
 
     GemmArgs g1;
-    g1.X = mfma_ ? w.xperm : x;
+    g1.X = w.xperm;
     g1.W = d_w1_;
     g1.bias = d_b1_;
     g1.out = w.h;
     g1.tiles = w.tiles;
     g1.tile_total = w.tile_total;
     g1.max_tiles = mt;
-    g1.N = (int)(2 * H_);
-    g1.K = (int)D_;
+    g1.N = (int)(2 * Hp_);
+    g1.K = (int)Dk_;
+    g1.n_out = (int)H_;
     g1.num_experts = 1;
-    // MFMA: the K-blocked buffers' row capacity; general: rows of x (row-major)
-    g1.a_cap = mfma_ ? w.cap_rows : rows;
+    g1.a_cap = w.cap_rows;  // the K-blocked buffers' row capacity
     g1.split_ws = w.split_ws;
     g1.split_cnt = w.split_cnt;
     g1.tail_cnt = w.tile_total + 1;
-    STAGE(mfma_ ? launch_gemm_gate_up_mfma(dt_, g1, s) : launch_gemm_gate_up_simt(dt_, g1, s),
-          "gate/up GEMM");
+    STAGE(launch_gemm_gate_up(dt_, g1, plan, s), "gate/up GEMM");
     if ((rc = mark(4))) return rc;
 
     GemmArgs g2 = g1;
@@ -665,10 +727,10 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     g2.bias = d_b2_;
     g2.out = y;  // rows stay in order: the output is y itself
     g2.tail_cnt = w.tile_total + 2;
-    g2.N = (int)D_;
-    g2.K = (int)H_;
-    STAGE(mfma_ ? launch_gemm_down_mfma(dt_, g2, s) : launch_gemm_down_simt(dt_, g2, s),
-          "down GEMM");
+    g2.N = (int)Dn_;
+    g2.K = (int)Hp_;
+    g2.n_out = (int)D_;
+    STAGE(launch_gemm_down(dt_, g2, plan, s), "down GEMM");
     if ((rc = mark(5))) return rc;
     if ((rc = mark(6))) return rc;
 #undef STAGE
@@ -760,6 +822,7 @@ int MoeLayer::forward_host_pieces(const void* x, void* y, int64_t rows, int np, 
         host_pieces_ = 0;
         return code;
     };
+    const Scoped whole(plan_rows_, rows);
     int n_pieces = 0;
     for (int p = 0; p < np; ++p) {
         const int64_t off = p * per, n = std::min(per, rows - off);
@@ -838,16 +901,15 @@ int MoeLayer::routing(int32_t* idx, float* w, int32_t* counts, float* gap) {
             }
     }
     if (counts) {
-        if (host_pieces_ > 0) {  // the pieces' counts, added
-            std::vector<int32_t> pc((size_t)host_pieces_ * Ecols_);
-            HIP_TRY(hipMemcpy(pc.data(), s_gap + rows, pc.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
-            for (int64_t e = 0; e < E_; ++e) {
-                int64_t c = 0;
-                for (int p = 0; p < host_pieces_; ++p) c += pc[(size_t)p * Ecols_ + e];
-                counts[e] = (int32_t)c;
-            }
-        } else {
-            HIP_TRY(hipMemcpy(counts, last_ws_.expert_count, sizeof(int32_t) * E_, hipMemcpyDeviceToHost));
+        // the counts of each piece, added
+        const int n = host_pieces_ > 0 ? host_pieces_ : scratch_pieces_;
+        const void* src = host_pieces_ > 0 ? static_cast<const void*>(s_gap + rows) : last_ws_.expert_count;
+        std::vector<int32_t> pc((size_t)n * Ecols_);
+        HIP_TRY(hipMemcpy(pc.data(), src, pc.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+        for (int64_t e = 0; e < E_; ++e) {
+            int64_t c = 0;
+            for (int p = 0; p < n; ++p) c += pc[(size_t)p * Ecols_ + e];
+            counts[e] = (int32_t)c;
         }
     }
     if (gap) HIP_TRY(hipMemcpy(gap, s_gap, sizeof(float) * rows, hipMemcpyDeviceToHost));
