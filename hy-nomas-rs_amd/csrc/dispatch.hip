@@ -11,6 +11,7 @@
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "mfma.hpp"
 #include "seam.hpp"
 
 namespace nomas {
@@ -331,6 +332,26 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(DispatchArgs a) 
                 const int p = s_ppos[pr];
                 if (p < 0 || p >= a.a_cap) continue;
                 const unsigned char* src = sb + s_prow[pr] * kSlabStride + piece * 16;
+                if constexpr (sizeof(T) == 4) {
+                    // two K-blocks of 16 columns are one block of planes: the
+                    // thread's chunk of each is its 8 values of every plane's row
+                    unsigned char* dst = static_cast<unsigned char*>(a.x_perm) +
+                                         ((int64_t)(kb0 / 2) * kPlanes * a.a_cap + p) * kKBlockBytes + piece * 16;
+#pragma unroll
+                    for (int q = 0; q < kKbs; q += 2) {
+                        if (q >= nkb) break;
+                        float v[8];
+                        load16(reinterpret_cast<const float*>(src + q * kKBlockBytes), v);
+                        load16(reinterpret_cast<const float*>(src + (q + 1) * kKBlockBytes), v + 4);
+                        uint32_t pl[kPlanes][4];
+                        split_exact_n<8>(v, pl);
+#pragma unroll
+                        for (int t = 0; t < kPlanes; ++t)
+                            store16_nt(dst + (q / 2 * kPlanes + t) * a.a_cap * kKBlockBytes,
+                                       make_uint4(pl[t][0], pl[t][1], pl[t][2], pl[t][3]));
+                    }
+                    continue;
+                }
                 T* dst = xp + ((int64_t)kb0 * a.a_cap + p) * KB + piece * EPC;
                 if (nkb == kKbs) {
                     uint4 val[kKbs];
@@ -489,8 +510,20 @@ __global__ __launch_bounds__(256) void kblock_kernel(const T* __restrict__ x, T*
         const int64_t col = (i % nchunk) * EPC;
         uint4 v = make_uint4(0, 0, 0, 0);
         if (col < D) v = *reinterpret_cast<const uint4*>(x + r * D + col);
-        constexpr int KB = kblock_elems<T>();
-        *reinterpret_cast<uint4*>(xk + ((col / KB) * a_cap + r) * KB + col % KB) = v;
+        if constexpr (sizeof(T) == 4) {  // the planes of 4 values, 8 bytes each
+            const float f[4] = {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z),
+                                __uint_as_float(v.w)};
+            uint32_t pl[kPlanes][2];
+            split_exact_n<4>(f, pl);
+            unsigned char* dst = reinterpret_cast<unsigned char*>(xk) +
+                                 (col / 32 * kPlanes * a_cap + r) * kKBlockBytes + col / 4 % 4 * 16 + col / 16 % 2 * 8;
+#pragma unroll
+            for (int p = 0; p < kPlanes; ++p)
+                *reinterpret_cast<uint2*>(dst + p * a_cap * kKBlockBytes) = make_uint2(pl[p][0], pl[p][1]);
+        } else {
+            constexpr int KB = kblock_elems<T>();
+            *reinterpret_cast<uint4*>(xk + ((col / KB) * a_cap + r) * KB + col % KB) = v;
+        }
     }
 }
 

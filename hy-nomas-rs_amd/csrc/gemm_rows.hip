@@ -40,9 +40,13 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
     using V = typename Mfma<T>::V;
     constexpr int BM = 16 * NT, BN = kRowsBN, NB = BN / 16;
     constexpr int BK = kblock_elems<T>();
-    constexpr int kSub = Mfma<T>::kSub;
+    constexpr bool kSplit = sizeof(T) == 4;  // f32: bf16 planes (mfma.hpp), two K-blocks a step
+    constexpr int KS = kSplit ? 2 : 1;       // weight K-blocks per step
+    constexpr int XS = kSplit ? kPlanes : 1; // token blocks per step
     // steps in flight per wave
-    constexpr int P = NW == 1 ? (NT == 1 ? 8 : NT == 2 ? 6 : 4) : (NT <= 2 ? 4 : 3);
+    constexpr int P = kSplit    ? (NT == 1 ? 3 : 2)
+                      : NW == 1 ? (NT == 1 ? 8 : NT == 2 ? 6 : 4)
+                                : (NT <= 2 ? 4 : 3);
     __shared__ f32x4_t s_part[NW][NB][NT][kWave];
 
     const int N = a.N, K = a.K;
@@ -64,12 +68,12 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
     const int l16 = lane & 15, lq = lane >> 4;
 
     // this wave's k steps (none in gate/up tiles that hold padding only)
-    const int kt_all = K / BK;
+    const int kt_all = K / BK, st_all = kt_all / KS;
     const bool pad_tile = MODE == kGateUp && n0 / 2 >= a.n_out;
-    const int s0 = pad_tile ? 0 : kt_all * wave / NW, s1 = pad_tile ? 0 : kt_all * (wave + 1) / NW;
-    const int64_t wstep = (int64_t)N * BK, xstep = a.a_cap * BK;
+    const int s0 = pad_tile ? 0 : st_all * wave / NW, s1 = pad_tile ? 0 : st_all * (wave + 1) / NW;
+    const int64_t wstep = (int64_t)N * BK, xstep = a.a_cap * kKBlockBytes;  // (elements, bytes)
     const T* Wt = static_cast<const T*>(a.W) + ((int64_t)e * kt_all * N + n0) * BK;
-    const T* Xt = static_cast<const T*>(a.X) + (int64_t)row0 * BK;
+    const char* Xt = static_cast<const char*>(a.X) + (int64_t)row0 * kKBlockBytes;
     const uint32_t woff = (uint32_t)(l16 * kKBlockBytes + lq * 16);
     uint32_t xoff[NT];  // rows past the tile's end read its last row (never stored)
 #pragma unroll
@@ -85,16 +89,24 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
     for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = NW == 1 ? bias(i) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    V fa[P][NB], fb[P][NT];
-    auto fetch = [&](int s, V (&wa)[NB], V (&xb)[NT]) {  // past the end: the last step again
-        const int st = max(min(s, s1 - 1), 0);
-        const char* w = reinterpret_cast<const char*>(Wt + st * wstep);
-        const char* x = reinterpret_cast<const char*>(Xt + st * xstep);
+    V fa[P][KS][NB], fb[P][XS][NT];
+    auto load = [&](int st, V (&wa)[KS][NB], V (&xb)[XS][NT]) {  // the fragments of step st
 #pragma unroll
-        for (int i = 0; i < NB; ++i)
-            wa[i] = *reinterpret_cast<const V*>(w + i * 16 * kKBlockBytes + woff);
+        for (int c = 0; c < KS; ++c) {
+            const char* w = reinterpret_cast<const char*>(Wt + (st * KS + c) * wstep);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) xb[j] = *reinterpret_cast<const V*>(x + xoff[j]);
+            for (int i = 0; i < NB; ++i)
+                wa[c][i] = *reinterpret_cast<const V*>(w + i * 16 * kKBlockBytes + woff);
+        }
+#pragma unroll
+        for (int c = 0; c < XS; ++c) {
+            const char* x = Xt + (st * XS + c) * xstep;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) xb[c][j] = *reinterpret_cast<const V*>(x + xoff[j]);
+        }
+    };
+    auto fetch = [&](int s, V (&wa)[KS][NB], V (&xb)[XS][NT]) {  // past the end: the last step again
+        load(max(min(s, s1 - 1), 0), wa, xb);
     };
 #pragma unroll
     for (int p = 0; p < P; ++p) fetch(s0 + p, fa[p], fb[p]);
@@ -102,15 +114,61 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             if (st + p < s1) {
+                if constexpr (kSplit) {
 #pragma unroll
-                for (int t = 0; t < kSub; ++t)
+                    for (int i = 0; i < NB; ++i) {
+                        u32x4_t pa[kPlanes];
+                        split_all(fa[p][0][i], fa[p][KS - 1][i], pa);
+#pragma unroll
+                        for (int m = 0; m < kProducts; ++m)
+#pragma unroll
+                            for (int j = 0; j < NT; ++j)
+                                acc[i][j] = mfma_plane(pa[product_a(m)],
+                                                       __builtin_bit_cast(u32x4_t, fb[p][product_b(m)][j]), acc[i][j]);
+                    }
+                } else {
 #pragma unroll
                     for (int i = 0; i < NB; ++i)
 #pragma unroll
                         for (int j = 0; j < NT; ++j)
-                            acc[i][j] = Mfma<T>::run(fa[p][i], fb[p][j], acc[i][j], t);
+                            acc[i][j] = Mfma<T>::run(fa[p][0][i], fb[p][0][j], acc[i][j]);
+                }
             }
             fetch(st + p + P, fa[p], fb[p]);
+        }
+    }
+    if constexpr (kSplit) {
+        // as in gemm_mfma: sums that are not finite again, with f32 MFMAs
+        float t = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) t = not_finite(acc[i][j], t);
+        if (__any(t != t)) {
+            f32x4_t again[NB][NT];
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) again[i][j] = NW == 1 ? bias(i) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int st = s0; st < s1; ++st) {
+                V wa[KS][NB], xb[XS][NT];
+                load(st, wa, xb);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    u32x4_t pl[kPlanes];
+#pragma unroll
+                    for (int c = 0; c < kPlanes; ++c) pl[c] = __builtin_bit_cast(u32x4_t, xb[c][j]);
+#pragma unroll
+                    for (int k8 = 0; k8 < 8; ++k8)
+#pragma unroll
+                        for (int i = 0; i < NB; ++i)
+                            again[i][j] = mfma_f32(wa[k8 / 4][i][k8 % 4], unsplit(pl, k8), again[i][j]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) keep_finite(acc[i][j], again[i][j]);
         }
     }
     // Epilogue.  Lane (l16, lq) of block (i, j) holds token row 16 j + l16 and
@@ -123,14 +181,10 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
         if (m >= nrows) return;
         if constexpr (MODE == kGateUp) {
             const int hc = n0 / 2 + i * 16 + 4 * lq;
-            T hv[4];
+            float hv[4];
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
-                hv[s] = hc + s < a.n_out ? Elt<T>::from_f32(swiglu<T>(v[0][s], v[1][s]))
-                                         : Elt<T>::from_f32(0.0f);
-            Raw4 raw;
-            __builtin_memcpy(&raw, hv, sizeof(raw));
-            *reinterpret_cast<Raw4*>(out + ((int64_t)(hc / BK) * a.a_cap + row0 + m) * BK + hc % BK) = raw;
+            for (int s = 0; s < 4; ++s) hv[s] = hc + s < a.n_out ? swiglu<T>(v[0][s], v[1][s]) : 0.0f;
+            store_hidden<T>(a.out, a.a_cap, row0 + m, hc, hv);
         } else {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {

@@ -148,8 +148,8 @@ struct Workspace {
     int32_t* expert_off = nullptr;   // E_cols + 1
     TileInfo* tiles = nullptr;       // max_tiles
     int32_t* tile_total = nullptr;   // 3: tile count, the GEMMs' tail counters
-    void* xperm = nullptr;           // a_cap x Dk (D padded, K-blocked)
-    void* h = nullptr;               // a_cap x Hp (H padded, K-blocked)
+    void* xperm = nullptr;           // a_cap x Dk (D padded, K-blocked; f32: planes)
+    void* h = nullptr;               // a_cap x Hp (H padded, likewise)
     void* yperm = nullptr;           // a_cap x D (MoE only)
     void* block_h = nullptr;         // forward_block: rows x D
 };
@@ -252,7 +252,7 @@ private:
     // pieces of `cap` rows.
     size_t layout(int64_t cap, bool block, uint8_t* base, Workspace* w, int64_t route_cap = 0) const;
     // The bytes that decide whether a no-allocation forward is taken: those of
-    // layout() with x_perm and h unpadded.
+    // layout() with x_perm and h as plain rows x D and rows x H matrices.
     size_t scratch_need(int64_t cap) const;
 
     int64_t D_, H_, E_, k_;

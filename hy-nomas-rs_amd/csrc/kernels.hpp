@@ -97,6 +97,15 @@ constexpr int kStages = 4;  // K steps (K-blocks) per turn of the ring
 template <typename T>
 __host__ __device__ constexpr int kblock_elems() { return kKBlockBytes / (int)sizeof(T); }
 __host__ __device__ constexpr int64_t round_up(int64_t n, int64_t m) { return (n + m - 1) / m * m; }
+// f32 activations (x_perm, h) are stored as their three bf16 planes (mfma.hpp):
+// columns in blocks of 32, each block's planes one after another, each plane's
+// row 64 bytes.  Within a row the 16-byte chunk c holds columns 4c..4c+3 and
+// 16 + 4c..16 + 4c + 3 of the block, the order in which a GEMM lane holds the
+// weights of two 16-column f32 K-blocks.  Element (r, k) of plane p:
+//   ((k / 32 * 3 + p) * R + r) * 32 + (k / 4 % 4) * 8 + (k / 16 % 2) * 4 + k % 4
+constexpr int kActPlanes = 3;
+// Bytes of one element of x_perm or h.
+__host__ __device__ constexpr int act_bytes(DType dt) { return dt == DType::F32 ? 2 * kActPlanes : 2; }
 // Columns of a K-blocked operand with K = `k` columns of es-byte elements.
 __host__ __device__ constexpr int64_t padded_k(int64_t k, int es) {
     return round_up(k, kStages * kKBlockBytes / es);
@@ -117,13 +126,13 @@ struct DispatchArgs {
     TileInfo* tiles;        // max_tiles
     int32_t* tile_total;    // 3: the tile count, then the two GEMMs' tail counters (cleared)
     int32_t* tok_pos;  // rows x k_slots
-    void* x_perm;      // a_cap x Dk, K-blocked (R = a_cap)
+    void* x_perm;      // a_cap x Dk, K-blocked (R = a_cap; f32: planes)
     int Dk;            // padded_k(D): columns D .. Dk - 1 are written as zeros
     int64_t a_cap;     // rows of x_perm (positions must stay below)
 };
 
 struct GemmArgs {
-    const void* X;     // token rows (a_cap x K), expert-contiguous
+    const void* X;     // token rows (a_cap x K), expert-contiguous (f32: planes)
     const void* W;     // expert weights
     const float* bias; // expert biases (f32)
     void* out;

@@ -1,7 +1,7 @@
 // The matrix-core operations and the SwiGLU shared by the grouped GEMMs (device code).
 #pragma once
 
-#include "common.hpp"
+#include "kernels.hpp"
 
 namespace nomas {
 
@@ -9,32 +9,143 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-// A lane's 16-byte operand fragment (one row, 64 bytes of k per stage split
-// over the 4 lane groups) feeds kSub MFMAs: one 16x16x32 for 16-bit types,
-// four 16x16x4 for f32 (MFMA t takes element t; lane group g then holds
-// k = 4 g + t of the stage, the same for both operands).
+// One 16x16x32 MFMA on the lane's 16-byte fragments of 16-bit types (one row,
+// 64 bytes of k split over the 4 lane groups).  For f32, V holds 4 values.
 template <typename T> struct Mfma;
 template <> struct Mfma<__bf16> {
     typedef bf16x8_t V;
-    static constexpr int kSub = 1;
-    static __device__ __forceinline__ f32x4_t run(V a, V b, f32x4_t c, int) {
+    static __device__ __forceinline__ f32x4_t run(V a, V b, f32x4_t c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
     }
 };
 template <> struct Mfma<_Float16> {
     typedef f16x8_t V;
-    static constexpr int kSub = 1;
-    static __device__ __forceinline__ f32x4_t run(V a, V b, f32x4_t c, int) {
+    static __device__ __forceinline__ f32x4_t run(V a, V b, f32x4_t c) {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
     }
 };
 template <> struct Mfma<float> {
     typedef f32x4_t V;
-    static constexpr int kSub = 4;
-    static __device__ __forceinline__ f32x4_t run(V a, V b, f32x4_t c, int t) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], b[t], c, 0, 0, 0);
-    }
 };
+// v_mfma_f32_16x16x4_f32: element t of the fragments, k = 4 (lane group) + t.
+__device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// f32 products on the bf16 matrix cores: each f32 value is the exact sum of
+// three bf16 planes (the value rounded to bf16, the remainder rounded, the
+// rest: 8 + 8 + 8 significant bits), and a product of two values is the six
+// plane products down to 2^-16 of the largest, added smallest first into the
+// f32 accumulator; what is left out is below 2^-26 of the product.  The bf16
+// MFMA does a plane product in 1/16 of the time of the f32 MFMAs.  Weights stay
+// f32 in memory and are split by the GEMM; activations (x_perm, h) are split
+// once, by the kernels that write them (kernels.hpp).
+// (A plane below bf16's smallest normal, 2^-126, may be flushed: values below
+// 2^-110 keep fewer of their bits.)
+// Sums that come out infinite or NaN are made again with f32 MFMAs by the GEMMs
+// (products with the planes of an infinite value, or of a weight that rounds
+// past bf16's largest, are not the product).
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+constexpr int kPlanes = 3;
+constexpr int kProducts = 6;
+__host__ __device__ constexpr int product_a(int p) { return p == 0 ? 0 : p == 1 ? 2 : p == 2 ? 1 : p == 3 ? 0 : p == 4 ? 1 : 0; }
+__host__ __device__ constexpr int product_b(int p) { return p == 0 ? 2 : p == 1 ? 0 : p == 2 ? 1 : p == 3 ? 1 : p == 4 ? 0 : 0; }
+
+// Two f32 to bf16 (round to nearest even), the first in the low half.
+__device__ __forceinline__ uint32_t cvt_pk_bf16(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// The planes of a lane's 8 values, one pair of values at a time in four steps
+// of at most 3 instructions (to be spread between MFMAs).
+struct SplitState {
+    float r0, r1, s0, s1;
+};
+template <int STEP>
+__device__ __forceinline__ void split_step(float x0, float x1, int d, u32x4_t (&pl)[kPlanes], SplitState& t) {
+#pragma clang fp contract(off)
+    if constexpr (STEP == 0) {
+        const uint32_t p = cvt_pk_bf16(x0, x1);
+        pl[0][d] = p;
+        t.s0 = __uint_as_float(p << 16);
+        t.s1 = __uint_as_float(p & 0xffff0000u);
+    } else if constexpr (STEP == 1) {
+        t.r0 = x0 - t.s0;
+        t.r1 = x1 - t.s1;
+        pl[1][d] = cvt_pk_bf16(t.r0, t.r1);
+    } else if constexpr (STEP == 2) {
+        const uint32_t p = pl[1][d];
+        t.s0 = __uint_as_float(p << 16);
+        t.s1 = __uint_as_float(p & 0xffff0000u);
+        t.r0 -= t.s0;
+    } else {
+        t.r1 -= t.s1;
+        pl[2][d] = cvt_pk_bf16(t.r0, t.r1);
+    }
+}
+__device__ __forceinline__ void split_all(const f32x4_t& a, const f32x4_t& b, u32x4_t (&pl)[kPlanes]) {
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const float x0 = d < 2 ? a[2 * d] : b[2 * d - 4], x1 = d < 2 ? a[2 * d + 1] : b[2 * d - 3];
+        SplitState t;
+        split_step<0>(x0, x1, d, pl, t);
+        split_step<1>(x0, x1, d, pl, t);
+        split_step<2>(x0, x1, d, pl, t);
+        split_step<3>(x0, x1, d, pl, t);
+    }
+}
+// The planes of any two values, whose sum (p2 + p1) + p0 is the value again
+// also where it is infinite, NaN or rounds past bf16's largest.
+__device__ __forceinline__ void split_exact(float x0, float x1, uint32_t (&pl)[kPlanes]) {
+#pragma clang fp contract(off)  // the remainders are of the f32 value, not of the product it may come from
+    auto first = [](float x) {  // rounded to bf16, large values truncated
+        const float r = (float)(__bf16)x;
+        return __builtin_isinf(r) ? __uint_as_float(__float_as_uint(x) & 0xffff0000u) : r;
+    };
+    const float a0 = first(x0), a1 = first(x1);
+    const float r0 = __builtin_isfinite(x0) ? x0 - a0 : 0.0f, r1 = __builtin_isfinite(x1) ? x1 - a1 : 0.0f;
+    const float b0 = (float)(__bf16)r0, b1 = (float)(__bf16)r1;
+    pl[0] = cvt_pk_bf16(a0, a1);
+    pl[1] = cvt_pk_bf16(b0, b1);
+    pl[2] = cvt_pk_bf16(r0 - b0, r1 - b1);
+}
+// ... of 4 or 8 values; plane p's bf16s in order in pl[p]
+template <int N>
+__device__ __forceinline__ void split_exact_n(const float* v, uint32_t (&pl)[kPlanes][N / 2]) {
+#pragma unroll
+    for (int d = 0; d < N / 2; ++d) {
+        uint32_t q[kPlanes];
+        split_exact(v[2 * d], v[2 * d + 1], q);
+#pragma unroll
+        for (int p = 0; p < kPlanes; ++p) pl[p][d] = q[p];
+    }
+}
+// Value s (0-7) of a lane's fragment from its planes.
+__device__ __forceinline__ float unsplit(const u32x4_t (&pl)[kPlanes], int s) {
+    float v[kPlanes];
+#pragma unroll
+    for (int p = 0; p < kPlanes; ++p)
+        v[p] = __uint_as_float(s % 2 ? pl[p][s / 2] & 0xffff0000u : pl[p][s / 2] << 16);
+    return v[0] + (v[1] + v[2]);
+}
+__device__ __forceinline__ f32x4_t mfma_plane(const u32x4_t& a, const u32x4_t& b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
+                                                   __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+}
+// NaN if any of the values so far was infinite or NaN, else 0.
+__device__ __forceinline__ float not_finite(const f32x4_t& v, float t) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) t = __builtin_fmaf(v[s], 0.0f, t);
+    return t;
+}
+// The values of v, those that are not finite from `again`.
+__device__ __forceinline__ void keep_finite(f32x4_t& v, const f32x4_t& again) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) v[s] = __builtin_isfinite(v[s]) ? v[s] : again[s];
+}
 
 enum { kGateUp = 0, kDown = 1 };  // the two GEMMs of an expert
 
@@ -44,6 +155,30 @@ template <typename T>
 __device__ __forceinline__ float swiglu(float g, float u) {
     if constexpr (sizeof(T) == 2) return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u;
     else return g / (1.0f + expf(-g)) * u;
+}
+
+// Hidden units hc..hc+3 (hc % 4 == 0) of row r into h, K-blocked (f32: planes).
+template <typename T>
+__device__ __forceinline__ void store_hidden(void* h, int64_t a_cap, int r, int hc, const float (&v)[4]) {
+    unsigned char* dst;
+    if constexpr (sizeof(T) == 4) {
+        uint32_t pl[kPlanes][2];
+        split_exact_n<4>(v, pl);
+        dst = static_cast<unsigned char*>(h) + ((int64_t)(hc / 32 * kPlanes) * a_cap + r) * kKBlockBytes +
+              hc / 4 % 4 * 16 + hc / 16 % 2 * 8;
+#pragma unroll
+        for (int p = 0; p < kPlanes; ++p)
+            *reinterpret_cast<uint2*>(dst + p * a_cap * kKBlockBytes) = make_uint2(pl[p][0], pl[p][1]);
+    } else {
+        constexpr int KB = kblock_elems<T>();
+        T t[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) t[s] = Elt<T>::from_f32(v[s]);
+        uint2 raw;
+        __builtin_memcpy(&raw, t, sizeof(raw));
+        dst = static_cast<unsigned char*>(h) + ((int64_t)(hc / KB) * a_cap + r) * kKBlockBytes + hc % KB * 2;
+        *reinterpret_cast<uint2*>(dst) = raw;
+    }
 }
 
 }  // namespace nomas

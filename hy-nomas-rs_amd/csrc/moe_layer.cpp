@@ -315,6 +315,7 @@ int MoeLayer::upload_f32(const MoeParamsF32& p) {
 // ---- workspace --------------------------------------------------------------
 
 GemmPlan MoeLayer::gemm_plan(int64_t rows) const {
+
     return nomas::gemm_plan(dt_, std::max(rows, plan_rows_) * kslots_, Ecols_, Dk_, Hp_, D_, H_);
 }
 
@@ -359,8 +360,8 @@ size_t MoeLayer::layout(int64_t cap, bool block, uint8_t* base, Workspace* w,
     v.expert_off = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * (Ecols_ + 1)));
     v.tiles = reinterpret_cast<TileInfo*>(take(sizeof(TileInfo) * mt));
     v.tile_total = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * 3));  // + tail counters
-    v.xperm = take(es * A * Dk_);
-    v.h = take(es * A * Hp_);
+    v.xperm = take(act_bytes(dt_) * A * Dk_);
+    v.h = take(act_bytes(dt_) * A * Hp_);
     if (!dense_only_) v.yperm = take(es * A * D_);  // dense: the down GEMM writes y
     if (block) v.block_h = take(es * cap * D_);
     if (w) *w = v;
@@ -368,8 +369,10 @@ size_t MoeLayer::layout(int64_t cap, bool block, uint8_t* base, Workspace* w,
 }
 
 size_t MoeLayer::scratch_need(int64_t cap) const {
-    const int64_t pad = (Dk_ - D_) + (Hp_ - H_);  // zero columns of x_perm and h
-    return layout(cap, false, nullptr, nullptr) - (size_t)(pad * cap * kslots_) * dtype_size(dt_);
+    const int64_t A = cap * kslots_;
+    const int64_t more = (Dk_ + Hp_) * act_bytes(dt_) - (D_ + H_) * (int64_t)dtype_size(dt_);
+    const int64_t tiles = max_gemm_tiles(A, Ecols_) - (A / kMfmaBM + Ecols_);  // of small calls
+    return layout(cap, false, nullptr, nullptr) - (size_t)(more * A + tiles * (int64_t)sizeof(TileInfo));
 }
 
 void MoeLayer::free_workspace() {
@@ -475,8 +478,8 @@ int MoeLayer::forward_noalloc(const void* x, void* y, int64_t rows, hipStream_t 
                          "holds %zu (at most %lld rows for this layer): use nomas_moe_forward",
                          (long long)rows, need, kScratchBytes, (long long)(lo * kRouterRows));
     }
-    // Widths that are padded can need more than the call's own bytes: such a
-    // call runs in row pieces that fit (each an ordinary forward over its
+    // Padded widths and the planes of f32 can need more than the call's own
+    // bytes: such a call runs in row pieces that fit (each an ordinary forward over its
     // rows; the routing of all rows is kept).
     int64_t lo = 0, hi = cap / kRouterRows;
     while (lo < hi) {

@@ -70,6 +70,46 @@ def test_padded_non_finite_rows_stay_apart():
     assert torch.isposinf(yb[3]).all() and torch.isnan(yb[40]).all()
 
 
+# rows, D, H: a call of few rows and one of whole 256-row tiles
+@pytest.mark.parametrize("rows,D,H", [(70, 256, 128), (3000, 512, 256), (3000, 200, 72)])
+def test_f32_values_that_have_no_finite_planes(rows, D, H):
+    """f32 rows with an infinity, a NaN or a value that rounds past bf16's
+    largest, and weights of that size: each row as f32 arithmetic has it, the
+    other rows' bits unchanged.  The bar on the finite values is that of f32
+    sums of one large term and D small ones (a few ulps)."""
+    big = np.float32(3.4e38)
+
+    def ffn(gate):
+        w = {"ffn.gate.weight": gate, "ffn.up.weight": np.full((H, D), 1e-20, np.float32),
+             "ffn.down.weight": np.full((D, H), 1e-3, np.float32)}
+        return nm.FeedForward.from_source(nm.Weights.tensors_(w, "f32"), "ffn", D, H)
+
+    layer = ffn(np.full((H, D), 1e-20, np.float32))
+    x = torch.randn(rows, D, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    y = layer.forward(x)
+    bad = x.clone()
+    bad[3, 5] = float("inf")
+    bad[40, 0] = float("nan")
+    bad[60] = 0.0
+    bad[60, 7] = float(big)
+    yb = layer.forward(bad)
+    keep = [i for i in range(rows) if i not in (3, 40, 60)]
+    assert torch.equal(yb[keep], y[keep])
+    assert torch.isposinf(yb[3]).all() and torch.isnan(yb[40]).all()
+    want = (float(big) * float(np.float32(1e-20))) ** 2 * H * float(np.float32(1e-3))
+    assert torch.allclose(yb[60].double(), torch.full((D,), want, device="cuda", dtype=torch.float64), rtol=2e-6)
+    # one weight of 3.4e38 in every hidden unit's gate, met by x = 1e-30
+    gate = np.full((H, D), 1e-3, np.float32)
+    gate[:, 2] = big
+    x[:, 2] = 1e-30
+    got = ffn(gate).forward(x).double()
+    g = x.double() @ torch.from_numpy(gate).cuda().double().T
+    u = x.double().sum(1, keepdim=True) * float(np.float32(1e-20))
+    want = (g * torch.sigmoid(g) * u).sum(1, keepdim=True) * float(np.float32(1e-3))
+    assert torch.isfinite(got).all()
+    assert (got - want).norm() <= 1e-5 * want.norm() * np.sqrt(D)  # want: (rows, 1), got: its D columns
+
+
 def test_noalloc_in_pieces():
     """A no-allocation call whose padded buffers exceed the scratch array runs
     in row pieces: the same bits and routing as the allocating forward."""
