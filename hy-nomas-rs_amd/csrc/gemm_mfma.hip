@@ -348,6 +348,13 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                         });
                     });
                 });
+                // (keeps the accumulators in place from turn to turn: without it
+                // the down kernel's register allocation moved 576 of them per turn
+                // instead of 272)
+#pragma unroll
+                for (int i = 0; i < SN; ++i)
+#pragma unroll
+                    for (int j = 0; j < SM; ++j) asm volatile("" : "+a"(acc[i][j]));
             }
         }
     };
