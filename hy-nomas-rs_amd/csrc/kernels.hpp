@@ -63,7 +63,6 @@ struct SeamArgs {
     double eps;
     const float* shift;   // sequences x D
     const float* scale;
-    int factor_lds;       // set by the launcher: LDS bytes for the factors
 };
 
 struct RouterArgs {

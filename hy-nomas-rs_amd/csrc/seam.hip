@@ -2,19 +2,24 @@
 //   h = modulate(norm2(x), shift, scale)      (norm.rs:55-65, modulate.rs:69-79)
 // for rows x D activations, row r in sequence r / seq.
 //
-// One block takes 64 rows in two phases.
+// One block of 256 threads takes 16 rows in two phases.
 //  1. The sum of squares of each row, added in the reference's order: x*x
 //     rounded to f32, then one add per element in ascending d -- a serial chain
-//     of D adds per row that no reordering may shorten.  Waves 1..15 make the
-//     squares, 128 columns of the 64 rows at a time, into one half of a double
-//     buffer in LDS (f32, rows padded by 16 bytes so the 64 lanes' 16-byte
-//     reads at one column spread over all banks); meanwhile lane r of wave 0
-//     adds row r's squares out of the other half.  The chain then costs one
-//     add per element and never waits on HBM.
-//  2. h for the 64 rows, 16 bytes per thread, coalesced; norm_w, shift and scale
-//     of the sequences the block touches come from LDS (from global memory
-//     when they do not fit).
-// Bytes per row: D*b read twice (the second pass mostly from cache), D*b written.
+//     of D adds per row that no reordering may shorten.  Waves 1..3 make the
+//     squares, 256 columns of the 16 rows at a time, into one half of a double
+//     buffer in LDS (f32, rows padded by 16 bytes so the lanes' 16-byte reads at
+//     one column spread over all banks); meanwhile lane r of wave 0 adds row
+//     r's squares out of the other half.  The chain then costs one add per
+//     element and never waits on HBM.
+//  2. h: a thread takes a 16-byte column chunk of 8 rows, its norm_w, shift and
+//     scale in registers (read again where the sequence changes).
+// Bytes per row: D*b read twice (the second time mostly from cache), D*b
+// written.  The chain (about 8 us at D = 3072) bounds a call whose blocks run
+// once, so blocks are small: there are enough of them for all CUs from 4,096
+// rows on, and several on a CU hide each other's chains.  Measured against
+// blocks of 64 rows and 1,024 threads (75 blocks for 4,744 rows): 4,744 rows of
+// 3,072 bf16 46 -> 31 us, 4,872 rows of 1,024 f32 19 -> 17 us, 14,232 rows of
+// 1,536 bf16 31 -> 30 us (131 MB, 4.4 TB/s; a large copy reaches 4.9).
 #include <algorithm>
 
 #include "kernels.hpp"
@@ -24,30 +29,25 @@ namespace nomas {
 
 namespace {
 
-constexpr int kSeamRows = 64;
-constexpr int kSeamThreads = 1024;
-constexpr int kStageCols = 128;                           // columns per stage
+constexpr int kSeamRows = 16;
+constexpr int kSeamThreads = 256;
+constexpr int kStageCols = 256;                           // columns per stage
 constexpr int kRowStride = kStageCols * 4 + 16;           // bytes, padded
-constexpr int kStageBytes = kSeamRows * kRowStride;       // 33,792
-constexpr int kBatch = 8;                                 // h chunks per thread in flight
-constexpr size_t kMaxLds = 160 * 1024;
+constexpr int kStageBytes = kSeamRows * kRowStride;       // 16,640
+constexpr int kRowGroup = 8;                              // rows per thread in phase 2
 
 template <typename T>
 __global__ __launch_bounds__(kSeamThreads) void seam_h_kernel(SeamArgs a) {
-    // [2][64][kRowStride] stages (later the factors) in factor_lds bytes,
-    // then inverse RMS [64] and sequence [64] per row
-    extern __shared__ __align__(16) unsigned char s_buf[];
-    float* s_inv = reinterpret_cast<float*>(s_buf + a.factor_lds);
-    int* s_seqidx = reinterpret_cast<int*>(s_inv + kSeamRows);
+    __shared__ __align__(16) unsigned char s_buf[2 * kStageBytes];
+    __shared__ float s_inv[kSeamRows];   // inverse RMS per row
+    __shared__ int s_seqidx[kSeamRows];  // sequence per row, from the block's first
     constexpr int EPC = 16 / sizeof(T);
     constexpr int kChunks = kSeamRows * kStageCols / EPC;   // 16-byte chunks per stage
     constexpr int kRowChunks = kStageCols / EPC;
-    // waves 1..15 produce the squares, wave 0 adds them up
+    // waves 1..3 produce the squares, wave 0 adds them up
     constexpr int kProducers = kSeamThreads - kWave;
-    constexpr int kLoads = (kChunks + kProducers - 1) / kProducers;  // 2 (16-bit) or 3 (f32)
-    // stages of x in flight: ~64 KB per block, what HBM's latency under load
-    // times a CU's share of its bandwidth asks for
-    constexpr int kRing = kLoads == 2 ? 4 : 3;
+    constexpr int kLoads = (kChunks + kProducers - 1) / kProducers;  // 3 (16-bit) or 6 (f32)
+    constexpr int kRing = kLoads == 3 ? 4 : 3;  // stages of x in flight (32 or 48 KB a block)
     const T* x = static_cast<const T*>(a.x);  // h may alias x: no restrict
     T* h = static_cast<T*>(a.h);
     const int D = a.D, nck = D / EPC;  // D % 8 == 0
@@ -111,123 +111,100 @@ __global__ __launch_bounds__(kSeamThreads) void seam_h_kernel(SeamArgs a) {
         stash(ring[0], 0);
         fetch(kRing, ring[0]);
         __syncthreads();
-        // whole ring turns; stage st sits in ring slot st % kRing, LDS half st & 1.
-        // Stages past the end stash zeros nobody reads and load a valid chunk.
+        // stage st sits in ring slot st % kRing, LDS half st & 1.  Stages past the
+        // end stash zeros nobody reads and load a valid chunk.
         for (int st0 = 0; st0 < nstage; st0 += kRing) {
 #pragma unroll
             for (int p = 0; p < kRing; ++p) {
                 const int st = st0 + p;
+                if (st >= nstage) break;
                 stash(ring[(p + 1) % kRing], st + 1);
                 fetch(st + 1 + kRing, ring[(p + 1) % kRing]);
                 __syncthreads();
             }
         }
     } else {
-        s_seqidx[tid] = (int)((row0 + min(tid, nrows - 1)) / a.seq - row0 / a.seq);
+        if (tid < kSeamRows) s_seqidx[tid] = (int)((row0 + min(tid, nrows - 1)) / a.seq - row0 / a.seq);
         __syncthreads();
         for (int st0 = 0; st0 < nstage; st0 += kRing) {
 #pragma unroll
             for (int p = 0; p < kRing; ++p) {
                 const int st = st0 + p;
-                if (st < nstage) {
-                    const unsigned char* rowp = s_buf + (st & 1) * kStageBytes + tid * kRowStride;
-#pragma unroll 8
-                    for (int c = 0; c < kStageCols / 4; ++c) {
-                        const float4 q = *reinterpret_cast<const float4*>(rowp + c * 16);
-                        acc = add_nc(acc, q.x);
-                        acc = add_nc(acc, q.y);
-                        acc = add_nc(acc, q.z);
-                        acc = add_nc(acc, q.w);
+                if (st >= nstage) break;
+                const unsigned char* rowp = s_buf + (st & 1) * kStageBytes + (tid % kSeamRows) * kRowStride;
+                // the reads of the next 8 pieces go out before 8 are added
+                constexpr int kP = 8;
+                float4 q[2][kP];
+#pragma unroll
+                for (int i = 0; i < kP; ++i) q[0][i] = *reinterpret_cast<const float4*>(rowp + i * 16);
+#pragma unroll
+                for (int c = 0; c < kStageCols / 4; c += kP) {
+                    const int b = c / kP % 2;
+                    if (c + kP < kStageCols / 4) {
+#pragma unroll
+                        for (int i = 0; i < kP; ++i)
+                            q[b ^ 1][i] = *reinterpret_cast<const float4*>(rowp + (c + kP + i) * 16);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < kP; ++i) {
+                        acc = add_nc(acc, q[b][i].x);
+                        acc = add_nc(acc, q[b][i].y);
+                        acc = add_nc(acc, q[b][i].z);
+                        acc = add_nc(acc, q[b][i].w);
                     }
                 }
                 __syncthreads();
             }
         }
     }
-    if (tid < kWave) s_inv[tid] = seam_inv_rms(acc, D, a.eps);
+    if (tid < kSeamRows) s_inv[tid] = seam_inv_rms(acc, D, a.eps);
+    __syncthreads();
 
     // ---- phase 2: h ----
-    // norm_w and the scale / shift rows of the sequences the block touches
-    // go to LDS when they fit (the stage buffers are free now), else they are
-    // read from global memory; either way 16 bytes at a time.
+    // Chunk c of rows g kRowGroup .. + kRowGroup - 1, the rows' loads in flight
+    // together; each thread reads only the chunks it writes (h may alias x).
     const int64_t b0 = row0 / a.seq;
-    const int nsq = s_seqidx[nrows - 1] + 1;
-    const bool lds_f = (size_t)(1 + 2 * nsq) * D * 4 <= a.factor_lds;
-    float* f_w = reinterpret_cast<float*>(s_buf);  // D
-    float* f_sc = f_w + D;                          // nsq x D
-    float* f_sh = f_sc + (size_t)nsq * D;           // nsq x D
-    if (lds_f) {
-        for (int i = tid; i < D / 4; i += kSeamThreads) {
-            float4 w = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-            if (a.norm_w) w = reinterpret_cast<const float4*>(a.norm_w)[i];
-            reinterpret_cast<float4*>(f_w)[i] = w;
-        }
-        for (int i = tid; i < nsq * D / 4; i += kSeamThreads) {
-            reinterpret_cast<float4*>(f_sc)[i] = reinterpret_cast<const float4*>(a.scale + b0 * D)[i];
-            reinterpret_cast<float4*>(f_sh)[i] = reinterpret_cast<const float4*>(a.shift + b0 * D)[i];
+    for (int q = tid; q < nck * (kSeamRows / kRowGroup); q += kSeamThreads) {
+        const int g = q / nck, col = (q - g * nck) * EPC, r0 = g * kRowGroup;
+        if (r0 >= nrows) break;
+        uint4 v[kRowGroup];
+#pragma unroll
+        for (int u = 0; u < kRowGroup; ++u)  // past the end: the last row again, not stored
+            v[u] = *reinterpret_cast<const uint4*>(x + (row0 + min(r0 + u, nrows - 1)) * (int64_t)D + col);
+        float w[EPC], sc[EPC], sh[EPC];
+#pragma unroll
+        for (int e = 0; e < EPC; ++e) w[e] = 1.0f;  // norm_w null: gain 1
+        if (a.norm_w) load_f32s<EPC>(a.norm_w + col, w);
+        int seq = -1;
+#pragma unroll
+        for (int u = 0; u < kRowGroup; ++u) {
+            const int r = r0 + u;
+            if (r >= nrows) break;
+            if (s_seqidx[r] != seq) {
+                seq = s_seqidx[r];
+                load_f32s<EPC>(a.scale + (b0 + seq) * D + col, sc);
+                load_f32s<EPC>(a.shift + (b0 + seq) * D + col, sh);
+            }
+            const float inv = s_inv[r];
+            Vec16<T> t;
+            __builtin_memcpy(&t, &v[u], 16);
+#pragma unroll
+            for (int e = 0; e < EPC; ++e)
+                t.v[e] = Elt<T>::from_f32(seam_h<T>(Elt<T>::to_f32(t.v[e]), inv, w[e], sc[e], sh[e]));
+            uint4 o;
+            __builtin_memcpy(&o, &t, 16);
+            *reinterpret_cast<uint4*>(h + (row0 + r) * (int64_t)D + col) = o;
         }
     }
-    __syncthreads();
-    // 16-byte chunks of the block's rows, kBatch per thread in flight; each
-    // thread reads only the chunks it writes (h may alias x).  pw null: gain 1.
-    auto rows_h = [&](const float* pw, const float* psc, const float* psh) {
-        const int total = nrows * nck;
-        for (int i0 = tid; i0 < total; i0 += kSeamThreads * kBatch) {
-            uint4 v[kBatch];
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {  // past the end: the last chunk again, not stored
-                const int i = min(i0 + u * kSeamThreads, total - 1);
-                const int r = i / nck;
-                v[u] = *reinterpret_cast<const uint4*>(x + (row0 + r) * (int64_t)D +
-                                                       (int64_t)(i - r * nck) * EPC);
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const int i = i0 + u * kSeamThreads;
-                if (i >= total) continue;
-                const int r = i / nck, col = (i - r * nck) * EPC;
-                const size_t fo = (size_t)s_seqidx[r] * D + col;
-                const float inv = s_inv[r];
-                float w[EPC], sc[EPC], sh[EPC];
-                if (pw) {
-                    load_f32s<EPC>(pw + col, w);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < EPC; ++e) w[e] = 1.0f;
-                }
-                load_f32s<EPC>(psc + fo, sc);
-                load_f32s<EPC>(psh + fo, sh);
-                Vec16<T> t;
-                __builtin_memcpy(&t, &v[u], 16);
-#pragma unroll
-                for (int e = 0; e < EPC; ++e)
-                    t.v[e] = Elt<T>::from_f32(seam_h<T>(Elt<T>::to_f32(t.v[e]), inv, w[e], sc[e], sh[e]));
-                uint4 o;
-                __builtin_memcpy(&o, &t, 16);
-                *reinterpret_cast<uint4*>(h + (row0 + r) * (int64_t)D + col) = o;
-            }
-        }
-    };
-    if (lds_f)
-        rows_h(f_w, f_sc, f_sh);
-    else
-        rows_h(a.norm_w, a.scale + b0 * D, a.shift + b0 * D);
 }
 
 template <typename T>
 hipError_t launch_seam_h_t(const SeamArgs& a, hipStream_t s) {
     const int64_t nblk = (a.rows + kSeamRows - 1) / kSeamRows;
     if (nblk == 0) return hipSuccess;
-    // LDS: the two stage buffers, which phase 2 reuses for the factors of up
-    // to two sequences when a larger allocation is not needed for them
-    SeamArgs b = a;
-    const size_t want = (size_t)5 * a.D * 4;
-    b.factor_lds = (int)std::max<size_t>(2 * kStageBytes, std::min<size_t>(want, kMaxLds - 512));
-    const size_t lds = (size_t)b.factor_lds + 512;  // + inverse RMS and sequence per row
-    hipError_t err = hipFuncSetAttribute((const void*)seam_h_kernel<T>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (err != hipSuccess) return err;
-    launch_kernel(seam_h_kernel<T>, dim3((unsigned)nblk), dim3(kSeamThreads), lds, s, b);
+    if (nblk > 0x7fffffff) return hipErrorInvalidValue;
+    launch_kernel(seam_h_kernel<T>, dim3((unsigned)nblk), dim3(kSeamThreads), 0, s, a);
     return hipGetLastError();
 }
 
