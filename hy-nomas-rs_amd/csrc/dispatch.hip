@@ -476,9 +476,15 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
     }
 }
 
-// Dense feed-forward: every row goes to expert 0, in order.
-__global__ void dense_tiles_kernel(int64_t rows, int BM, int max_tiles, TileInfo* tiles,
-                                   int32_t* tile_total) {
+// x (rows x D, row-major) to the K-blocked layout of the GEMMs (Dk columns,
+// zeros past D): one 16-byte chunk per thread, coalesced reads, 64-byte runs
+// written.  It also writes the dense feed-forward's tile table (every row goes
+// to expert 0, in order), which as a kernel of its own took 5 us a call.
+template <typename T>
+__global__ __launch_bounds__(256) void kblock_kernel(const T* __restrict__ x, T* __restrict__ xk,
+                                                     int64_t rows, int D, int Dk, int64_t a_cap,
+                                                     int BM, int max_tiles, TileInfo* __restrict__ tiles,
+                                                     int32_t* __restrict__ tile_total) {
     const int64_t ntiles = (rows + BM - 1) / BM;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < max_tiles; i += gridDim.x * blockDim.x) {
         TileInfo t;
@@ -493,14 +499,6 @@ __global__ void dense_tiles_kernel(int64_t rows, int BM, int max_tiles, TileInfo
         tile_total[1] = 0;  // the GEMMs' tail counters
         tile_total[2] = 0;
     }
-}
-
-// x (rows x D, row-major) to the K-blocked layout of the GEMMs (Dk columns,
-// zeros past D): one 16-byte chunk per thread, coalesced reads, 64-byte runs
-// written.
-template <typename T>
-__global__ __launch_bounds__(256) void kblock_kernel(const T* __restrict__ x, T* __restrict__ xk,
-                                                     int64_t rows, int D, int Dk, int64_t a_cap) {
     constexpr int EPC = 16 / sizeof(T);
     const int nchunk = Dk / EPC;
     const int64_t total = rows * nchunk;
@@ -587,33 +585,29 @@ hipError_t launch_dispatch(DType dt, const DispatchArgs& a, hipStream_t s) {
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_dense_tiles(int64_t rows, int BM, int max_tiles, TileInfo* tiles,
-                              int32_t* tile_total, hipStream_t s) {
-    if (max_tiles <= 0) return hipErrorInvalidValue;
-    const int nblk = (max_tiles + 255) / 256;
-    launch_kernel(dense_tiles_kernel, dim3(nblk), dim3(256), 0, s, rows, BM, max_tiles, tiles,
-                  tile_total);
-    return hipGetLastError();
-}
-
 hipError_t launch_kblock(DType dt, const void* x, void* xk, int64_t rows, int D, int Dk,
-                         int64_t a_cap, hipStream_t s) {
+                         int64_t a_cap, int BM, int max_tiles, TileInfo* tiles, int32_t* tile_total,
+                         hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    if (Dk != padded_k(D, (int)dtype_size(dt)) || a_cap < rows) return hipErrorInvalidValue;
+    if (Dk != padded_k(D, (int)dtype_size(dt)) || a_cap < rows || BM < 1 || max_tiles < 1)
+        return hipErrorInvalidValue;
     const int64_t chunks = rows * (Dk / (16 / (int)dtype_size(dt)));
     const unsigned nblk = (unsigned)std::min<int64_t>((chunks + 255) / 256, 65536);
     switch (dt) {
         case DType::BF16:
             launch_kernel(kblock_kernel<__bf16>, dim3(nblk), dim3(256), 0, s,
-                          (const __bf16*)x, (__bf16*)xk, rows, D, Dk, a_cap);
+                          (const __bf16*)x, (__bf16*)xk, rows, D, Dk, a_cap, BM, max_tiles, tiles,
+                          tile_total);
             break;
         case DType::F16:
             launch_kernel(kblock_kernel<_Float16>, dim3(nblk), dim3(256), 0, s,
-                          (const _Float16*)x, (_Float16*)xk, rows, D, Dk, a_cap);
+                          (const _Float16*)x, (_Float16*)xk, rows, D, Dk, a_cap, BM, max_tiles, tiles,
+                          tile_total);
             break;
         case DType::F32:
             launch_kernel(kblock_kernel<float>, dim3(nblk), dim3(256), 0, s,
-                          (const float*)x, (float*)xk, rows, D, Dk, a_cap);
+                          (const float*)x, (float*)xk, rows, D, Dk, a_cap, BM, max_tiles, tiles,
+                          tile_total);
             break;
         default: return hipErrorInvalidValue;
     }

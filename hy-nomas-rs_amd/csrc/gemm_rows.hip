@@ -50,7 +50,7 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
     __shared__ f32x4_t s_part[NW][NB][NT][kWave];
 
     const int N = a.N, K = a.K;
-    const int live = min(*a.tile_total, a.max_tiles);
+    const int live = a.dense_rows ? (int)((a.dense_rows + BM - 1) / BM) : min(*a.tile_total, a.max_tiles);
     // down: weight tiles past the real columns have nothing to store
     const int ntn = (int)((MODE == kDown ? a.n_out + BN - 1 : N) / BN);
     const long long units = (long long)live * ntn;
@@ -58,7 +58,8 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
     const long long q = blockIdx.x / kNumXcd, u = (blockIdx.x % kNumXcd) * share + q;
     if (q >= share || u >= units) return;
     const int mt = (int)(u % live), n0 = (int)(u / live) * BN;
-    const TileInfo ti = a.tiles[mt];
+    TileInfo ti = {0, mt * BM, (int)min<int64_t>(BM, a.dense_rows - (int64_t)mt * BM), 0};
+    if (!a.dense_rows) ti = a.tiles[mt];
     const int e = ti.expert, row0 = ti.row0, nrows = ti.rows;
     if (e < 0 || e >= a.num_experts || nrows < 1 || nrows > BM || row0 < 0 ||
         row0 + (int64_t)nrows > a.a_cap)
@@ -71,14 +72,15 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
     const int kt_all = K / BK, st_all = kt_all / KS;
     const bool pad_tile = MODE == kGateUp && n0 / 2 >= a.n_out;
     const int s0 = pad_tile ? 0 : st_all * wave / NW, s1 = pad_tile ? 0 : st_all * (wave + 1) / NW;
-    const int64_t wstep = (int64_t)N * BK, xstep = a.a_cap * kKBlockBytes;  // (elements, bytes)
+    const int64_t wstep = (int64_t)N * BK, xstep = a.x_row ? kKBlockBytes : a.a_cap * kKBlockBytes;  // (elements, bytes)
+    const int64_t xrow = a.x_row ? a.x_row : kKBlockBytes;
     const T* Wt = static_cast<const T*>(a.W) + ((int64_t)e * kt_all * N + n0) * BK;
-    const char* Xt = static_cast<const char*>(a.X) + (int64_t)row0 * kKBlockBytes;
+    const char* Xt = static_cast<const char*>(a.X) + row0 * xrow;
     const uint32_t woff = (uint32_t)(l16 * kKBlockBytes + lq * 16);
     uint32_t xoff[NT];  // rows past the tile's end read its last row (never stored)
 #pragma unroll
     for (int j = 0; j < NT; ++j)
-        xoff[j] = (uint32_t)(min(j * 16 + l16, nrows - 1) * kKBlockBytes + lq * 16);
+        xoff[j] = (uint32_t)(min(j * 16 + l16, nrows - 1) * xrow + lq * 16);
 
     auto bias = [&](int i) -> f32x4_t {
         const float4 b = *reinterpret_cast<const float4*>(a.bias + (int64_t)e * N + n0 + i * 16 + 4 * lq);
@@ -234,6 +236,8 @@ hipError_t launch_rows_t(const GemmArgs& a, hipStream_t s) {
     const int n_cols = MODE == kGateUp ? a.N / 2 : a.N;
     if (a.N % kMfmaBN != 0 || a.K % (kblock_elems<T>() * kStages) != 0 || a.n_out < 1 || a.n_out > n_cols ||
         (MODE == kDown && a.n_out % 8 != 0))
+        return hipErrorInvalidValue;
+    if (a.x_row && (sizeof(T) != 2 || a.x_row % 16 != 0 || a.x_row < a.K * 2LL || a.x_row > (1LL << 26)))
         return hipErrorInvalidValue;
     if (a.max_tiles <= 0) return hipSuccess;
     const int64_t ntn = (MODE == kDown ? a.n_out + kRowsBN - 1 : a.N) / kRowsBN;

@@ -146,6 +146,12 @@ struct GemmArgs {
     int n_out;
     int num_experts;  // experts with weights (tiles naming others are skipped)
     int64_t a_cap;    // rows of X / out (tiles reaching beyond are skipped)
+    // gemm_rows: where X is not K-blocked (rows of x in place, whole K-blocks
+    // of 16-bit elements): bytes from row to row; 0: K-blocked
+    int64_t x_row = 0;
+    // gemm_rows, dense feed-forward: its rows, all of expert 0, with no tile
+    // table (tiles and tile_total are not read); 0: the table
+    int64_t dense_rows = 0;
     // f32 partial sums of tiles split along K (kSplitUnits units of
     // kSplitUnitFloats each; null: no tile is split) and one arrival counter per
     // split tile (zero between launches: the last part to arrive resets it)
@@ -215,12 +221,11 @@ hipError_t launch_gemm_down(DType dt, const GemmArgs& a, const GemmPlan& plan, h
 hipError_t launch_gemm_mfma(DType dt, bool gate_up, const GemmArgs& a, hipStream_t s);
 hipError_t launch_gemm_rows(DType dt, bool gate_up, const GemmArgs& a, int bm, int waves, hipStream_t s);
 hipError_t launch_combine(DType dt, const CombineArgs& a, hipStream_t s);
-// Dense feed-forward (no routing): the tile table of `rows` rows of one
-// expert in BM-row tiles (max_tiles entries written), and x re-laid out
-// K-blocked with Dk = padded_k(D) columns for the gate/up GEMM.
-hipError_t launch_dense_tiles(int64_t rows, int BM, int max_tiles, TileInfo* tiles,
-                              int32_t* tile_total, hipStream_t s);
+// Dense feed-forward (no routing): x re-laid out K-blocked with Dk =
+// padded_k(D) columns for the gate/up GEMM, and the tile table of `rows` rows
+// of one expert in BM-row tiles (max_tiles entries written).
 hipError_t launch_kblock(DType dt, const void* x, void* xk, int64_t rows, int D, int Dk,
-                         int64_t a_cap, hipStream_t s);
+                         int64_t a_cap, int BM, int max_tiles, TileInfo* tiles, int32_t* tile_total,
+                         hipStream_t s);
 
 }  // namespace nomas

@@ -673,8 +673,11 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
 }
 
 // Dense feed-forward: the stages of the routed forward that remain.  Stage
-// slots for profiling: router (none), scan = tile table, dispatch = K-blocked
-// copy of x, gate/up, down (written straight into y), combine (none).
+// slots for profiling: router (none), scan (none), dispatch = K-blocked copy of
+// x and tile table, gate/up, down (written straight into y), combine (none).
+// Where gemm_rows runs 16-bit rows of whole K turns it reads x in place and
+// needs no table: two kernels (64 rows of 1024 x 2048 in bf16: a call 24.9 ->
+// 19.1 us; f32, without the table kernel, 38.9 -> 36.6 us).
 int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s) {
     int rc;
     const Workspace& w = ws_;
@@ -700,13 +703,17 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     } while (0)
     if ((rc = mark(0))) return rc;
     if ((rc = mark(1))) return rc;
-    STAGE(launch_dense_tiles(rows, plan.bm, mt, w.tiles, w.tile_total, s), "tile table");
     if ((rc = mark(2))) return rc;
-    STAGE(launch_kblock(dt_, x, w.xperm, rows, (int)D_, (int)Dk_, w.cap_rows, s), "K-blocked copy");
+    const bool in_place = plan.waves1 && plan.waves2 && dt_ != DType::F32 && D_ == Dk_;
+    if (!in_place)
+        STAGE(launch_kblock(dt_, x, w.xperm, rows, (int)D_, (int)Dk_, w.cap_rows, plan.bm, mt, w.tiles,
+                            w.tile_total, s), "K-blocked copy");
     if ((rc = mark(3))) return rc;
 
     GemmArgs g1;
-    g1.X = w.xperm;
+    g1.X = in_place ? x : w.xperm;
+    g1.x_row = in_place ? D_ * (int64_t)dtype_size(dt_) : 0;
+    g1.dense_rows = in_place ? rows : 0;
     g1.W = d_w1_;
     g1.bias = d_b1_;
     g1.out = w.h;
@@ -725,6 +732,7 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     if ((rc = mark(4))) return rc;
 
     GemmArgs g2 = g1;
+    g2.x_row = 0;
     g2.X = w.h;
     g2.W = d_w2_;
     g2.bias = d_b2_;

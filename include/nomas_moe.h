@@ -220,7 +220,7 @@ int nomas_ffn_forward_host(nomas_ffn_t *h, const void *x, void *y, int64_t rows)
 /* FeedForward::n_params (mlp.rs:50-58). */
 int64_t nomas_ffn_n_params(const nomas_ffn_t *h);
 
-/* No counterpart: per-stage timing ([0, tile table, K-blocked copy of x,
+/* No counterpart: per-stage timing ([0, 0, K-blocked copy of x (0 where none),
  * gemm_gate_up, gemm_down, 0]) and the GEMM path, as for the MoE handle. */
 int nomas_ffn_set_profiling(nomas_ffn_t *h, int enable);
 int nomas_ffn_stage_times(nomas_ffn_t *h, float *ms6);
