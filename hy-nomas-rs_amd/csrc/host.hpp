@@ -89,19 +89,25 @@ private:
     size_t n_ = 0;
 };
 
-// Pageable host memory <-> device through two pinned staging buffers, the
-// host copies of one chunk overlapping the DMA of the other.
+// Whether host memory is pinned (the DMA engine reads and writes it directly).
+bool is_pinned(const void* p);
+
+// Pageable host memory <-> device through kBufs pinned staging buffers, the
+// host copies of one chunk overlapping the DMA of others.
 class HostStager {
 public:
     ~HostStager();
+    static constexpr int kBufs = 4;
+    void rewind() { next_ = 0; }  // a call starts with the first (cached) buffer
     int to_device(void* dst_dev, const void* src_host, size_t bytes, hipStream_t s);
     int to_host(void* dst_host, const void* src_dev, size_t bytes, hipStream_t s);
 
 private:
     int ensure();
     void release();
-    void* pin_[2] = {nullptr, nullptr};
-    hipEvent_t ev_[2] = {nullptr, nullptr};
+    void* pin_[kBufs] = {};
+    hipEvent_t ev_[kBufs] = {};
+    int next_ = 0;  // the buffer of the next chunk
     std::unique_ptr<CopyPool> pool_;
 };
 
@@ -294,11 +300,12 @@ private:
     size_t hio_bytes_ = 0;  // bytes of each of the two halves
     HostStager stager_;
     // large host-tensor forwards run in row pieces: the copies of one piece
-    // overlap the forward of another (two non-blocking streams of the
-    // default priority, an input-landed and a forward-done event per piece)
-    static constexpr int kHostMaxPieces = 4;
-    static constexpr int64_t kHostPieceRows = 4096;  // at least, per piece
-    hipStream_t hs_copy_ = nullptr, hs_comp_ = nullptr;
+    // overlap the forward of another and the copies of the other direction
+    // (non-blocking streams of the default priority for copies in, forwards
+    // and copies out, an input-landed and a forward-done event per piece)
+    static constexpr int kHostMaxPieces = 8;
+    int host_pieces(int64_t rows) const;
+    hipStream_t hs_copy_ = nullptr, hs_comp_ = nullptr, hs_out_ = nullptr;
     hipEvent_t hev_in_[kHostMaxPieces] = {}, hev_fw_[kHostMaxPieces] = {};
     int host_pipe_setup();
     // the routing of a pieced forward, gathered per piece: idx and w

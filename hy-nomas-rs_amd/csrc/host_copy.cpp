@@ -1,7 +1,8 @@
 // Copies between pageable host memory and the device for the host-tensor
-// forward: through two pinned staging buffers of kChunk bytes, in chunks, so
+// forward: through pinned staging buffers of kChunk bytes, in chunks, so
 // that the host-side memcpy of one chunk (spread over a small pool of worker
-// threads) overlaps the DMA of the previous one.  hipMemcpy from pageable
+// threads) overlaps the DMA of earlier ones.  The first chunk's memcpy is what
+// no DMA hides, so chunks are small: 4 MB, 70 us on either side.  hipMemcpy from pageable
 // memory stages through the runtime's own buffers with one host thread and
 // reached about 19 GB/s here; pinned-to-device DMA runs at about 55 GB/s.
 #include <hip/hip_runtime.h>
@@ -15,7 +16,7 @@
 namespace nomas {
 
 namespace {
-constexpr size_t kChunk = (size_t)16 << 20;  // bytes per staging buffer
+constexpr size_t kChunk = (size_t)4 << 20;  // bytes per staging buffer
 constexpr size_t kMinSplit = (size_t)1 << 20;  // smaller copies stay on the calling thread
 }  // namespace
 
@@ -94,7 +95,7 @@ bool is_pinned(const void* p) {
 HostStager::~HostStager() { release(); }
 
 void HostStager::release() {
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < kBufs; ++b) {
         if (ev_[b]) (void)hipEventDestroy(ev_[b]);
         if (pin_[b]) (void)hipHostFree(pin_[b]);
         ev_[b] = nullptr;
@@ -106,7 +107,7 @@ void HostStager::release() {
 // All or nothing: a failed set-up leaves nothing behind, and the next call tries again.
 int HostStager::ensure() {
     if (pool_) return NOMAS_OK;
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < kBufs; ++b) {
         hipError_t e = hipHostMalloc(&pin_[b], kChunk, hipHostMallocDefault);
         if (e != hipSuccess) {
             pin_[b] = nullptr;
@@ -141,10 +142,10 @@ int HostStager::to_device(void* dst, const void* src, size_t bytes, hipStream_t 
     if (rc != NOMAS_OK) return rc;
     const unsigned char* in = static_cast<const unsigned char*>(src);
     unsigned char* out = static_cast<unsigned char*>(dst);
-    int c = 0;
-    for (size_t off = 0; off < bytes; off += kChunk, ++c) {
+    for (size_t off = 0; off < bytes; off += kChunk) {
         const size_t n = std::min(kChunk, bytes - off);
-        const int b = c & 1;
+        const int b = next_;
+        next_ = (next_ + 1) % kBufs;
         // buffer b drained (its last DMA may belong to an earlier call: the
         // pieces of a host forward stage one after another)
         STAGE_TRY(hipEventSynchronize(ev_[b]), "hipEventSynchronize");
@@ -165,26 +166,27 @@ int HostStager::to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
     if (rc != NOMAS_OK) return rc;
     const unsigned char* in = static_cast<const unsigned char*>(src);
     unsigned char* out = static_cast<unsigned char*>(dst);
-    // DMA chunk c into buffer c & 1, then copy chunk c - 1 out on the host
-    // (the host copy of chunk c - 2 from buffer c & 1 finished before)
-    size_t prev_off = 0, prev_n = 0;
-    int c = 0;
-    for (size_t off = 0; off < bytes; off += kChunk, ++c) {
-        const size_t n = std::min(kChunk, bytes - off);
-        const int b = c & 1;
-        STAGE_TRY(hipMemcpyAsync(pin_[b], in + off, n, hipMemcpyDeviceToHost, s), "hipMemcpyAsync D2H");
-        STAGE_TRY(hipEventRecord(ev_[b], s), "hipEventRecord");
-        if (c >= 1) {
-            STAGE_TRY(hipEventSynchronize(ev_[b ^ 1]), "hipEventSynchronize");
-            pool_->copy(out + prev_off, pin_[b ^ 1], prev_n);
+    // up to kBufs chunks' DMAs in flight; the host copies the oldest one out
+    // when it has landed.  (The buffers' earlier DMAs, into the device, may
+    // still be in flight on the first round.)
+    const int64_t chunks = (int64_t)((bytes + kChunk - 1) / kChunk);
+    const int first = next_;
+    next_ = (int)((next_ + chunks) % kBufs);
+    auto len = [&](int64_t c) { return std::min(kChunk, bytes - (size_t)c * kChunk); };
+    for (int64_t c = 0; c < chunks + kBufs - 1; ++c) {
+        const int64_t done = c - (kBufs - 1);
+        if (done >= 0) {
+            const int b = (int)((first + done) % kBufs);
+            STAGE_TRY(hipEventSynchronize(ev_[b]), "hipEventSynchronize");
+            pool_->copy(out + (size_t)done * kChunk, pin_[b], len(done));
         }
-        prev_off = off;
-        prev_n = n;
-    }
-    if (c >= 1) {
-        const int b = (c - 1) & 1;
-        STAGE_TRY(hipEventSynchronize(ev_[b]), "hipEventSynchronize");
-        pool_->copy(out + prev_off, pin_[b], prev_n);
+        if (c < chunks) {
+            const int b = (int)((first + c) % kBufs);
+            if (c < kBufs) STAGE_TRY(hipEventSynchronize(ev_[b]), "hipEventSynchronize");
+            STAGE_TRY(hipMemcpyAsync(pin_[b], in + (size_t)c * kChunk, len(c), hipMemcpyDeviceToHost, s),
+                      "hipMemcpyAsync D2H");
+            STAGE_TRY(hipEventRecord(ev_[b], s), "hipEventRecord");
+        }
     }
     return NOMAS_OK;
 }
