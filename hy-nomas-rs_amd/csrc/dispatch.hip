@@ -47,7 +47,7 @@ __host__ __device__ inline bool dispatch_fits(int E_cols, int k) {
 //     wave sums every 16th chunk, the waves' partials added in LDS);
 //  2. expert offsets (exclusive scan over experts, ascending) and the chunk's
 //     own per-expert slot offsets; block 0 also publishes the expert counts
-//     and offsets and the GEMM tile table (ceil(count / BM) tiles of BM rows
+//     and offsets and the GEMM tile tables (ceil(count / BM) tiles of BM rows
 //     per expert);
 //  3. the waves rank the chunk's slots, each taking every 16th expert: a
 //     ballot over the 64 rows gives every row its rank among the chunk's rows
@@ -213,26 +213,50 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_kernel(DispatchArgs a) 
             a.expert_count[e] = s_tot[e];
             a.expert_off[e] = s_off[e];
         }
-        const int total_tiles = s_ts[Ec];
+        if (tid == 0) a.expert_off[Ec] = s_off[Ec];
+        auto table = [&](int BM, int max_tiles, TileInfo* tiles, int32_t* total) {
+            const int total_tiles = s_ts[Ec];
+            if (tid == 0) *total = min(total_tiles, max_tiles);
+            for (int i = tid; i < total_tiles && i < max_tiles; i += kDispThreads) {
+                int lo = 0, hi = Ec - 1;  // last expert with s_ts <= i (skipping empty ones)
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (s_ts[mid] <= i) lo = mid; else hi = mid - 1;
+                }
+                const int j = i - s_ts[lo];
+                TileInfo t;
+                t.expert = lo;
+                t.row0 = s_off[lo] + j * BM;
+                t.rows = min(BM, s_tot[lo] - j * BM);
+                t.pad = 0;
+                tiles[i] = t;
+            }
+        };
+        table(a.BM, a.max_tiles, a.tiles, &a.tile_total[0]);
         if (tid == 0) {
-            a.expert_off[Ec] = s_off[Ec];
-            a.tile_total[0] = min(total_tiles, a.max_tiles);
             a.tile_total[1] = 0;  // the GEMMs' tail counters
             a.tile_total[2] = 0;
         }
-        for (int i = tid; i < total_tiles && i < a.max_tiles; i += kDispThreads) {
-            int lo = 0, hi = Ec - 1;  // last expert with s_ts <= i (skipping empty ones)
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (s_ts[mid] <= i) lo = mid; else hi = mid - 1;
+        if (a.BM2 != a.BM) {  // the down GEMM's own table
+            __syncthreads();
+            if (wave == 0) {
+                int carry = 0;
+                for (int e0 = 0; e0 < Ec; e0 += kWave) {
+                    const int e = e0 + lane;
+                    const int v = e < Ec ? (s_tot[e] + a.BM2 - 1) / a.BM2 : 0;
+                    int inc = v;
+#pragma unroll
+                    for (int o = 1; o < kWave; o <<= 1) {
+                        const int t = __shfl_up(inc, o);
+                        if (lane >= o) inc += t;
+                    }
+                    if (e < Ec) s_ts[e] = carry + inc - v;
+                    carry += __shfl(inc, kWave - 1);
+                }
+                if (lane == 0) s_ts[Ec] = carry;
             }
-            const int j = i - s_ts[lo];
-            TileInfo t;
-            t.expert = lo;
-            t.row0 = s_off[lo] + j * a.BM;
-            t.rows = min(a.BM, s_tot[lo] - j * a.BM);
-            t.pad = 0;
-            a.tiles[i] = t;
+            __syncthreads();
+            table(a.BM2, a.max_tiles2, a.tiles2, &a.tile_total[3]);
         }
     }
     // 3. ranks and positions.  Every wave holds each row's experts as a bit
@@ -531,7 +555,7 @@ hipError_t launch_dispatch_t(const DispatchArgs& a, hipStream_t s) {
     if (nblk == 0) return hipSuccess;
     if (a.nchunks != nblk || a.count_rows < kMinRouterBlockRows || a.count_rows > kRouterRows ||
         kRouterRows % a.count_rows != 0 || a.E_cols < 1 || a.E_cols > kMaxExperts + 1 || a.k_slots < 1 ||
-        a.k_slots > a.E_cols || a.BM < 1 || !dispatch_fits(a.E_cols, a.k_slots) ||
+        a.k_slots > a.E_cols || a.BM < 1 || a.BM2 < 1 || !dispatch_fits(a.E_cols, a.k_slots) ||
         a.Dk != padded_k(a.D, sizeof(T)))
         return hipErrorInvalidValue;
     const size_t lds = dispatch_lds(a.E_cols, a.k_slots);

@@ -753,12 +753,12 @@ hipError_t launch_gemm_mfma(DType dt, bool gate_up, const GemmArgs& a, hipStream
 }
 
 hipError_t launch_gemm_gate_up(DType dt, const GemmArgs& a, const GemmPlan& plan, hipStream_t s) {
-    return plan.waves1 ? launch_gemm_rows(dt, true, a, plan.bm, plan.waves1, s)
+    return plan.waves1 ? launch_gemm_rows(dt, true, a, plan.bm1, plan.waves1, s)
                        : launch_gemm_mfma(dt, true, a, s);
 }
 
 hipError_t launch_gemm_down(DType dt, const GemmArgs& a, const GemmPlan& plan, hipStream_t s) {
-    return plan.waves2 ? launch_gemm_rows(dt, false, a, plan.bm, plan.waves2, s)
+    return plan.waves2 ? launch_gemm_rows(dt, false, a, plan.bm2, plan.waves2, s)
                        : launch_gemm_mfma(dt, false, a, s);
 }
 

@@ -152,8 +152,9 @@ struct Workspace {
     int32_t* chunk_counts = nullptr; // chunks x E_cols
     int32_t* expert_count = nullptr; // E_cols, for each piece of the forward
     int32_t* expert_off = nullptr;   // E_cols + 1
-    TileInfo* tiles = nullptr;       // max_tiles
-    int32_t* tile_total = nullptr;   // 3: tile count, the GEMMs' tail counters
+    TileInfo* tiles = nullptr;       // max_gemm_tiles
+    TileInfo* tiles2 = nullptr;      // max_gemm_tiles: the down GEMM's where its tiles differ
+    int32_t* tile_total = nullptr;   // 4: tile count, the GEMMs' tail counters, second tile count
     void* xperm = nullptr;           // a_cap x Dk (D padded, K-blocked; f32: planes)
     void* h = nullptr;               // a_cap x Hp (H padded, likewise)
     void* yperm = nullptr;           // a_cap x D (MoE only)
@@ -251,7 +252,7 @@ private:
     // summed as in one forward.
     GemmPlan gemm_plan(int64_t rows) const;
     int64_t plan_rows_ = 0;  // rows of the pieced call in progress, else 0
-    int max_tiles(int64_t rows) const;
+    int max_tiles(int64_t rows, int bm) const;
     // Lays out the buffers of a forward on up to `cap` rows (a multiple of
     // 64) from `base` (nullptr: sizes only) and returns the bytes used.
     // `route_cap` (0: cap): rows of the routing, when the forward runs in

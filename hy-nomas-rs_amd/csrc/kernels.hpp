@@ -118,12 +118,13 @@ struct DispatchArgs {
     const int32_t* chunk_counts;  // ceil(rows / count_rows) x E_cols, from the router
     int nchunks;            // 64-row chunks
     int count_rows;         // rows per histogram (the router's rows per block: 64 or 32)
-    int BM;                 // GEMM tile rows
-    int max_tiles;
+    int BM, BM2;            // GEMM tile rows: gate/up, down
+    int max_tiles, max_tiles2;
     int32_t* expert_count;  // E_cols
     int32_t* expert_off;    // E_cols + 1
     TileInfo* tiles;        // max_tiles
-    int32_t* tile_total;    // 3: the tile count, then the two GEMMs' tail counters (cleared)
+    TileInfo* tiles2;       // max_tiles2 (written where BM2 != BM)
+    int32_t* tile_total;    // 4: the tile count, the two GEMMs' tail counters (cleared), the second count
     int32_t* tok_pos;  // rows x k_slots
     void* x_perm;      // a_cap x Dk, K-blocked (R = a_cap; f32: planes)
     int Dk;            // padded_k(D): columns D .. Dk - 1 are written as zeros
@@ -176,8 +177,10 @@ constexpr int kSplitUnits = 256;
 
 // Which kernels run a forward's two GEMMs (gemm_plan.hpp).
 struct GemmPlan {
-    int bm;              // token rows per tile of the tile table
-    int waves1, waves2;  // gate/up, down: waves per block of gemm_rows, 0: gemm_mfma
+    // gate/up and down: token rows per tile, and waves per block of gemm_rows
+    // (0: gemm_mfma, with its 256 rows)
+    int bm1, waves1;
+    int bm2, waves2;
 };
 
 struct CombineArgs {
@@ -214,8 +217,8 @@ hipError_t launch_gated_residual(DType dt, const void* x, const void* y, const f
                                  void* out, int64_t rows, int D, int64_t seq, hipStream_t s);
 hipError_t launch_router(DType dt, const RouterArgs& a, hipStream_t s);
 hipError_t launch_dispatch(DType dt, const DispatchArgs& a, hipStream_t s);
-// Grouped GEMMs: W packed as described in moe_layer.cpp, the tile table in
-// tiles of plan.bm rows.
+// Grouped GEMMs: W packed as described in moe_layer.cpp, the tile tables in
+// tiles of plan.bm1 and plan.bm2 rows.
 hipError_t launch_gemm_gate_up(DType dt, const GemmArgs& a, const GemmPlan& plan, hipStream_t s);
 hipError_t launch_gemm_down(DType dt, const GemmArgs& a, const GemmPlan& plan, hipStream_t s);
 hipError_t launch_gemm_mfma(DType dt, bool gate_up, const GemmArgs& a, hipStream_t s);

@@ -321,9 +321,8 @@ GemmPlan MoeLayer::gemm_plan(int64_t rows) const {
     return nomas::gemm_plan(dt_, std::max(rows, plan_rows_) * kslots_, Ecols_, Dk_, Hp_, D_, H_);
 }
 
-int MoeLayer::max_tiles(int64_t rows) const {
+int MoeLayer::max_tiles(int64_t rows, int bm) const {
     const int64_t A = rows * kslots_;
-    const int bm = gemm_plan(rows).bm;
     return (int)((A + bm - 1) / bm + Ecols_);
 }
 
@@ -361,7 +360,8 @@ size_t MoeLayer::layout(int64_t cap, bool block, uint8_t* base, Workspace* w,
     v.expert_count = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * pieces * Ecols_));
     v.expert_off = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * (Ecols_ + 1)));
     v.tiles = reinterpret_cast<TileInfo*>(take(sizeof(TileInfo) * mt));
-    v.tile_total = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * 3));  // + tail counters
+    v.tiles2 = reinterpret_cast<TileInfo*>(take(sizeof(TileInfo) * mt));
+    v.tile_total = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * 4));  // + tail counters, second count
     v.xperm = take(act_bytes(dt_) * A * Dk_);
     v.h = take(act_bytes(dt_) * A * Hp_);
     if (!dense_only_) v.yperm = take(es * A * D_);  // dense: the down GEMM writes y
@@ -373,7 +373,7 @@ size_t MoeLayer::layout(int64_t cap, bool block, uint8_t* base, Workspace* w,
 size_t MoeLayer::scratch_need(int64_t cap) const {
     const int64_t A = cap * kslots_;
     const int64_t more = (Dk_ + Hp_) * act_bytes(dt_) - (D_ + H_) * (int64_t)dtype_size(dt_);
-    const int64_t tiles = max_gemm_tiles(A, Ecols_) - (A / kMfmaBM + Ecols_);  // of small calls
+    const int64_t tiles = 2 * max_gemm_tiles(A, Ecols_) - (A / kMfmaBM + Ecols_);  // of small calls
     return layout(cap, false, nullptr, nullptr) - (size_t)(more * A + tiles * (int64_t)sizeof(TileInfo));
 }
 
@@ -489,7 +489,9 @@ int MoeLayer::forward_noalloc(const void* x, void* y, int64_t rows, hipStream_t 
         if (layout(mid * kRouterRows, false, nullptr, nullptr, cap) <= kScratchBytes) lo = mid;
         else hi = mid - 1;
     }
-    const int64_t piece = lo * kRouterRows;
+    // (pieces of equal size: the fewest that fit)
+    const int64_t n = lo > 0 ? (cap + lo * kRouterRows - 1) / (lo * kRouterRows) : 0;
+    const int64_t piece = n > 0 ? round_up((cap + n - 1) / n, kRouterRows) : 0;
     if (piece == 0)
         return set_error(NOMAS_ERR_INVALID_ARGUMENT,
                          "rows=%lld do not fit the no-allocation forward's device scratch of %zu "
@@ -541,7 +543,8 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
                          const BlockArgs* blk, const Workspace& w) {
     int rc;
     const int nch = (int)((rows + kRouterRows - 1) / kRouterRows);
-    const int mt = max_tiles(rows);
+    const GemmPlan plan = gemm_plan(rows);
+    const int mt = max_tiles(rows, plan.bm1), mt2 = max_tiles(rows, plan.bm2);
     const int64_t a_cap = w.cap_rows * kslots_;
     hipEvent_t* ev = nullptr;
     uint8_t* empty = nullptr;
@@ -609,12 +612,14 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     da.chunk_counts = w.chunk_counts;
     da.nchunks = nch;
     da.count_rows = ra.block_rows;
-    const GemmPlan plan = gemm_plan(rows);
-    da.BM = plan.bm;
+    da.BM = plan.bm1;
+    da.BM2 = plan.bm2;
     da.max_tiles = mt;
+    da.max_tiles2 = mt2;
     da.expert_count = w.expert_count;
     da.expert_off = w.expert_off;
     da.tiles = w.tiles;
+    da.tiles2 = w.tiles2;
     da.tile_total = w.tile_total;
     da.tok_pos = w.pos;
     da.x_perm = w.xperm;
@@ -648,6 +653,11 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     g2.bias = d_b2_;
     g2.out = w.yperm;
     g2.tail_cnt = w.tile_total + 2;
+    if (plan.bm2 != plan.bm1) {
+        g2.tiles = w.tiles2;
+        g2.tile_total = w.tile_total + 3;
+        g2.max_tiles = mt2;
+    }
     g2.N = (int)Dn_;
     g2.K = (int)Hp_;
     g2.n_out = (int)D_;
@@ -684,7 +694,7 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     int rc;
     const Workspace& w = ws_;
     const GemmPlan plan = gemm_plan(rows);
-    const int mt = max_tiles(rows);
+    const int mt = max_tiles(rows, kMfmaBM);
     hipEvent_t* ev = nullptr;
     uint8_t* empty = nullptr;
     if (profiling_) {
@@ -708,20 +718,20 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     if ((rc = mark(2))) return rc;
     const bool in_place = plan.waves1 && plan.waves2 && dt_ != DType::F32 && D_ == Dk_;
     if (!in_place)
-        STAGE(launch_kblock(dt_, x, w.xperm, rows, (int)D_, (int)Dk_, w.cap_rows, plan.bm, mt, w.tiles,
+        STAGE(launch_kblock(dt_, x, w.xperm, rows, (int)D_, (int)Dk_, w.cap_rows, kMfmaBM, mt, w.tiles,
                             w.tile_total, s), "K-blocked copy");
     if ((rc = mark(3))) return rc;
 
     GemmArgs g1;
     g1.X = in_place ? x : w.xperm;
     g1.x_row = in_place ? D_ * (int64_t)dtype_size(dt_) : 0;
-    g1.dense_rows = in_place ? rows : 0;
+    g1.dense_rows = plan.waves1 ? rows : 0;  // (gemm_mfma: the table)
     g1.W = d_w1_;
     g1.bias = d_b1_;
     g1.out = w.h;
     g1.tiles = w.tiles;
     g1.tile_total = w.tile_total;
-    g1.max_tiles = mt;
+    g1.max_tiles = max_tiles(rows, plan.bm1);
     g1.N = (int)(2 * Hp_);
     g1.K = (int)Dk_;
     g1.n_out = (int)H_;
@@ -740,6 +750,8 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     g2.bias = d_b2_;
     g2.out = y;  // rows stay in order: the output is y itself
     g2.tail_cnt = w.tile_total + 2;
+    g2.max_tiles = max_tiles(rows, plan.bm2);
+    g2.dense_rows = plan.waves2 ? rows : 0;
     g2.N = (int)Dn_;
     g2.K = (int)Hp_;
     g2.n_out = (int)D_;

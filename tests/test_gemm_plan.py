@@ -19,7 +19,7 @@ PROG = r"""
 #include <cstdio>
 using namespace nomas;
 int main() {
-  long n = 0, used[4] = {0, 0, 0, 0};
+  long n = 0, mixed = 0, used[4] = {0, 0, 0, 0};
   const int64_t widths[] = {8, 64, 72, 256, 264, 1000, 1024, 1536, 3072};
   const int64_t hiddens[] = {1, 96, 128, 640, 2667, 4096, 8192};
   for (DType dt : {DType::F32, DType::BF16, DType::F16})
@@ -30,17 +30,23 @@ int main() {
           int64_t most = 0;  // tiles of any call so far (A ascending)
           for (int64_t A = 1; A < 40000000; A += 1 + A / 7) {
             const GemmPlan p = gemm_plan(dt, A, E, Dk, Hp, D, H);
-            const bool rows = p.bm == 16 || p.bm == 32 || p.bm == 64;
-            if (!rows && p.bm != kMfmaBM) { printf("tile of %d rows\n", p.bm); return 1; }
-            if (rows != (p.waves1 > 0) || rows != (p.waves2 > 0)) { printf("waves\n"); return 1; }
-            if (rows && (D % 256 || H % 128) && (p.waves1 != 1 || p.waves2 != 1)) { printf("order\n"); return 1; }
-            const int64_t tiles = (A + p.bm - 1) / p.bm + E;
-            most = tiles > most ? tiles : most;
-            if (most > max_gemm_tiles(A, E)) { printf("bound: A %ld E %ld\n", (long)A, (long)E); return 1; }
-            used[p.bm == 16 ? 0 : p.bm == 32 ? 1 : p.bm == 64 ? 2 : 3]++;
+            const int bms[2] = {p.bm1, p.bm2}, waves[2] = {p.waves1, p.waves2};
+            for (int g = 0; g < 2; ++g) {
+              const int bm = bms[g];
+              const bool rows = bm == 16 || bm == 32 || bm == 64;
+              if (!rows && bm != kMfmaBM) { printf("tile of %d rows\n", bm); return 1; }
+              if (rows != (waves[g] > 0)) { printf("waves\n"); return 1; }
+              if (rows && (D % 256 || H % 128) && waves[g] != 1) { printf("order\n"); return 1; }
+              const int64_t tiles = (A + bm - 1) / bm + E;
+              most = tiles > most ? tiles : most;
+              if (most > max_gemm_tiles(A, E)) { printf("bound: A %ld E %ld\n", (long)A, (long)E); return 1; }
+              used[bm == 16 ? 0 : bm == 32 ? 1 : bm == 64 ? 2 : 3]++;
+            }
+            mixed += p.bm1 != p.bm2;
             ++n;
           }
         }
+  if (!mixed) { printf("the GEMMs never differ\n"); return 1; }
   for (long u : used) if (!u) { printf("a choice is never taken\n"); return 1; }
   printf("ok %ld\n", n);
   return 0;

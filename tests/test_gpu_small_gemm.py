@@ -41,6 +41,12 @@ def test_padded_widths(rows, D, H, dtype):
     run_case(rows, D, 3, 2, H, dtype, 600 + D + H, 0.5 if D == 72 else 0.0)
 
 
+# gate/up on 256-row tiles and down on 64-row ones (two tile tables)
+@pytest.mark.parametrize("D,H,dtype", [(1024, 2688, "bf16"), (1000, 2667, "bf16"), (512, 2048, "f32")])
+def test_gemms_of_different_tile_heights(D, H, dtype):
+    run_case(1111, D, 6, 2, H, dtype, 700 + D)
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 def test_padded_rows_do_not_depend_on_the_call(dtype):
     """Every row of a padded-width layer is the same bits in a call of 9,000 rows and of 3."""
