@@ -223,8 +223,10 @@ int MoeLayer::upload(const void* router_w, const void* gate_w, const void* gate_
     auto pack_row = [&](std::vector<uint8_t>& w, int64_t e, int64_t nkb, int64_t nrows, int64_t row,
                         const uint8_t* src, int64_t k) {
         uint8_t* dst = &w[(size_t)((e * nkb * nrows + row) * KB) * es];
-        for (int64_t k0 = 0; k0 < k; k0 += KB, dst += (size_t)(nrows * KB) * es)
-            std::memcpy(dst, src + k0 * es, (size_t)std::min(KB, k - k0) * es);
+        const int64_t full = k / KB;
+        for (int64_t b = 0; b < full; ++b)
+            std::memcpy(dst + b * nrows * kKBlockBytes, src + b * kKBlockBytes, kKBlockBytes);
+        if (k % KB) std::memcpy(dst + full * nrows * kKBlockBytes, src + full * kKBlockBytes, (size_t)(k % KB) * es);
     };
     // gate/up: rows 64g..64g+31 gate 32g.., rows 64g+32.. up 32g..
     std::vector<uint8_t> w1((size_t)(Ecols_ * 2 * Hp_ * Dk_) * es);
