@@ -784,7 +784,11 @@ int MoeLayer::forward_host(const void* x, void* y, int64_t rows) {
     }
     void* dx = d_hio_;
     void* dy = static_cast<uint8_t*>(d_hio_) + hio_bytes_;
-    const int np = host_pieces(rows);
+    // x and y that overlap without being the same: all of x is read before any
+    // of y is written, in one piece
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
+    const bool apart = xa == ya || xa + bytes <= ya || ya + bytes <= xa;
+    const int np = apart ? host_pieces(rows) : 1;
     stager_.rewind();
     if (np == 1) {
         host_pieces_ = 0;

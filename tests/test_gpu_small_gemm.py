@@ -116,6 +116,21 @@ def test_f32_values_that_have_no_finite_planes(rows, D, H):
     assert (got - want).norm() <= 1e-5 * want.norm() * np.sqrt(D)  # want: (rows, 1), got: its D columns
 
 
+@pytest.mark.parametrize("shift", [0, 64, -64])
+def test_host_output_over_the_input(shift):
+    """A pinned host output that is the input, or overlaps it some rows on."""
+    rows, D = 20_000, 264
+    t, x = small_case(rows, D, 4, 1, 96, 82)
+    layer = layer_from_tensors(t, "f32", D, 96, 4, 1)
+    want = layer.forward(to_device(x, "f32")).cpu()
+    buf = torch.empty(rows + 64, D, pin_memory=True)
+    src = buf[64:] if shift < 0 else buf[:rows]
+    dst = buf[:rows] if shift < 0 else buf[shift:shift + rows]
+    src.copy_(torch.from_numpy(x))
+    layer.forward(src, out=dst)
+    assert torch.equal(dst, want)
+
+
 def test_noalloc_in_pieces():
     """A no-allocation call whose padded buffers exceed the scratch array runs
     in row pieces: the same bits and routing as the allocating forward."""
