@@ -509,13 +509,17 @@ int MoeLayer::forward_noalloc(const void* x, void* y, int64_t rows, hipStream_t 
     layout(piece, false, static_cast<uint8_t*>(base), &w, cap);
     if (done_recorded_ && s != last_stream_) HIP_TRY(hipStreamWaitEvent(s, done_, 0));
     const Scoped whole(plan_rows_, rows);
-    int pieces = 0;
-    for (int64_t off = 0; off < rows; off += piece, ++pieces) {
+    // A piece writes its rows of y before the next one reads its rows of x:
+    // where y overlaps x from above, the pieces run from the last one down.
+    const int pieces = (int)((rows + piece - 1) / piece);
+    const bool down = reinterpret_cast<uintptr_t>(y) > reinterpret_cast<uintptr_t>(x);
+    for (int i = 0; i < pieces; ++i) {
+        const int64_t at = down ? pieces - 1 - i : i, off = at * piece;
         Workspace p = w;
         p.idx += off * kslots_;
         p.w += off * kslots_;
         p.gap += off;
-        p.expert_count += pieces * Ecols_;
+        p.expert_count += at * Ecols_;
         const size_t o = (size_t)off * D_ * dtype_size(dt_);
         rc = run_routed(static_cast<const uint8_t*>(x) + o, static_cast<uint8_t*>(y) + o,
                         std::min(piece, rows - off), s, nullptr, p);

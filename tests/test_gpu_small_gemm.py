@@ -148,3 +148,26 @@ def test_noalloc_in_pieces():
     assert torch.equal(y, y_ref)
     for a, b in zip(layer.routing(rows), ref):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("shift", [0, 64, -64])
+def test_noalloc_in_pieces_output_over_the_input(shift):
+    """y is x, or overlaps it some rows on: every piece reads rows of x that
+    no earlier piece has written."""
+    rows, D, E, k, H = 2_000_000, 8, 3, 1, 4
+    t, _ = small_case(8, D, E, k, H, 83, router_std=0.5)
+    layer = layer_from_tensors(t, "bf16", D, H, E, k)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x = torch.randn(rows, D, device="cuda", generator=g).to(torch.bfloat16)
+    want = layer.forward(x)
+    ref = layer.routing(rows)
+    buf = torch.empty(rows + 64, D, dtype=torch.bfloat16, device="cuda")
+    src = buf[64:] if shift < 0 else buf[:rows]
+    dst = buf[:rows] if shift < 0 else buf[shift:shift + rows]
+    src.copy_(x)
+    rc, msg = _noalloc(layer, src, dst)
+    assert rc == 0, msg
+    torch.cuda.synchronize()
+    assert torch.equal(dst, want)
+    for a, b in zip(layer.routing(rows), ref):
+        assert np.array_equal(a, b)
