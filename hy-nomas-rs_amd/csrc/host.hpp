@@ -161,10 +161,16 @@ struct Workspace {
     void* block_h = nullptr;         // forward_block: rows x D
 };
 
-// The device scratch array of the no-allocation forward (scratch.hip):
-// 512 MiB per GPU, enough for one 4,744-row segment of the 8B preset
-// (dim 3072, 8 experts, top-2, hidden 8192: 8,128 rows).
+// The no-allocation forward takes calls of up to kScratchBytes of plain
+// buffers: enough for one 4,744-row segment of the 8B preset (dim 3072, 8
+// experts, top-2, hidden 8192: 8,128 rows).
 constexpr size_t kScratchBytes = (size_t)512 << 20;
+// Its device scratch array (scratch.hip) per GPU.  f32 planes take 6 bytes an
+// element instead of 4: x_perm and h of whole-tile widths, and with them every
+// such call, need at most half as much again (of the call's own 8 D + 4 H bytes
+// a routed row, 4 (D + H) grow by 2 (D + H); the tile tables' 4 bytes a row and
+// 32 an expert are within what the other 4 D leave).
+constexpr size_t kScratchArrayBytes = kScratchBytes / 2 * 3;
 // Its address on `device` (looked up once per device; the first call also
 // clears the split-tile counters with a kernel on `s`).  Never allocates.
 // Each call counts as one use of the array: *gen receives that use's number
@@ -248,8 +254,10 @@ private:
     int ensure_workspace(int64_t rows);
     void free_workspace();
     // The GEMM kernels of a forward on `rows` rows.  The pieces of one call all
-    // take the plan of the whole call (plan_rows_), so that its rows are
-    // summed as in one forward.
+    // take the plan of the whole call (plan_rows_): the same kernels as in one
+    // forward.  (Rows of padded widths then have the same bits.  At whole-tile
+    // widths a piece's own last round decides which of its tiles gemm_mfma
+    // splits along K.)
     GemmPlan gemm_plan(int64_t rows) const;
     int64_t plan_rows_ = 0;  // rows of the pieced call in progress, else 0
     int max_tiles(int64_t rows, int bm) const;

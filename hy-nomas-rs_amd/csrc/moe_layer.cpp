@@ -482,13 +482,15 @@ int MoeLayer::forward_noalloc(const void* x, void* y, int64_t rows, hipStream_t 
                          "holds %zu (at most %lld rows for this layer): use nomas_moe_forward",
                          (long long)rows, need, kScratchBytes, (long long)(lo * kRouterRows));
     }
-    // Padded widths and the planes of f32 can need more than the call's own
-    // bytes: such a call runs in row pieces that fit (each an ordinary forward over its
-    // rows; the routing of all rows is kept).
+    // Padded widths can need more than the array holds: such a call runs in row
+    // pieces that fit (each an ordinary forward over its rows; the routing of
+    // all rows is kept), whose rows have the bits of one forward.  Whole-tile
+    // widths always fit (kScratchArrayBytes) and run as one forward does, K-split
+    // tiles included.
     int64_t lo = 0, hi = cap / kRouterRows;
     while (lo < hi) {
         const int64_t mid = (lo + hi + 1) / 2;
-        if (layout(mid * kRouterRows, false, nullptr, nullptr, cap) <= kScratchBytes) lo = mid;
+        if (layout(mid * kRouterRows, false, nullptr, nullptr, cap) <= kScratchArrayBytes) lo = mid;
         else hi = mid - 1;
     }
     // (pieces of equal size: the fewest that fit)
@@ -498,7 +500,7 @@ int MoeLayer::forward_noalloc(const void* x, void* y, int64_t rows, hipStream_t 
         return set_error(NOMAS_ERR_INVALID_ARGUMENT,
                          "rows=%lld do not fit the no-allocation forward's device scratch of %zu "
                          "bytes with this layer's padded widths: use nomas_moe_forward",
-                         (long long)rows, kScratchBytes);
+                         (long long)rows, kScratchArrayBytes);
     DeviceGuard g(device_);
     if (!g.ok) return set_error(NOMAS_ERR_HIP, "hipSetDevice(%d) failed", device_);
     void* base = nullptr;

@@ -1,5 +1,5 @@
 // The device scratch array of the no-allocation forward
-// (nomas_moe_forward_noalloc): a fixed kScratchBytes of device memory per GPU,
+// (nomas_moe_forward_noalloc): a fixed kScratchArrayBytes of device memory per GPU,
 // in the library's code object, so that a forward can run without any
 // allocation (callers under HIP graph capture or in tight serving loops).
 //
@@ -15,7 +15,7 @@
 
 namespace nomas {
 
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kScratchArrayBytes];
 
 namespace {
 

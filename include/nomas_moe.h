@@ -105,10 +105,10 @@ int nomas_moe_forward(nomas_moe_t *h, const void *x, void *y, int64_t rows, void
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  Same arguments and results, but every device buffer of
  * the forward (routing, permuted rows, the SwiGLU intermediate, K-split
- * partials) lives in a static device array of 512 MiB per GPU, held until
- * the process ends: the call allocates nothing.  `rows` beyond what fits (it
- * depends on dim, hidden and top_k; 8,128 rows at dim 3072, hidden 8192,
- * top-2, so one 4,744-row segment of the 8B preset) is
+ * partials) lives in a static device array of 768 MiB per GPU, held until
+ * the process ends: the call allocates nothing.  `rows` whose plain buffers
+ * pass 512 MiB (it depends on dim, hidden and top_k; 8,128 rows at dim 3072,
+ * hidden 8192, top-2, so one 4,744-row segment of the 8B preset) are
  * NOMAS_ERR_INVALID_ARGUMENT with the limit in the message.  The
  * first call on a device looks up the array's address and clears its
  * counters with a kernel on `stream`.  All such calls on one GPU share the

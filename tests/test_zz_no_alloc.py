@@ -111,6 +111,21 @@ def test_noalloc_rejects_rows_beyond_the_array():
     assert rc == 0
 
 
+def test_noalloc_f32_splits_k_as_forward_does():
+    """24,000 f32 rows of 1024 x 2048, one expert: the down GEMM has 376 tiles,
+    whose last round of 120 is split along K.  The no-allocation forward, whose
+    buffers take 580 MiB, runs the same tiles: the same bits."""
+    rows, dim, hidden = 24000, 1024, 2048
+    layer, _ = _layer(dim, 1, 1, hidden, "f32", 86)
+    x = torch.randn(rows, dim, device="cuda", generator=torch.Generator(device="cuda").manual_seed(7))
+    want = layer.forward(x)
+    y = torch.full_like(want, float("nan"))
+    rc, msg = _noalloc(layer, x, y)
+    assert rc == 0, msg
+    torch.cuda.synchronize()
+    assert torch.equal(y, want)
+
+
 def test_noalloc_runs_one_8b_segment():
     # dim 3072, 8 experts, top-2, hidden 8192, bf16: the reference's
     # per-branch forward_segment call
