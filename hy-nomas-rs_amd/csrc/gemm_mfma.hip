@@ -522,6 +522,20 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
             bad |= (t != t ? 1u : 0u) << j;
         }
     }
+    // gate/up: which hidden units (bit 4 j + s of gate block 4 p + b in word 2 p + b)
+    uint32_t bad_units[SN / 2] = {};
+    if constexpr (kSplit && MODE == kGateUp) {
+        if (bad) {
+#pragma unroll
+            for (int i = 0; i < SN / 2; ++i)
+#pragma unroll
+                for (int j = 0; j < SM; ++j)
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        bad_units[i] |= (unit_finite(acc[i / 2 * 4 + i % 2][j][s], acc[i / 2 * 4 + i % 2 + 2][j][s]) ? 0u : 1u)
+                                        << (4 * j + s);
+        }
+    }
 
     // Epilogue (the accumulators include the bias).  Lane (l16, lq) of block
     // (i, j) holds token row wm*WM + j*16 + l16 and weight rows
@@ -665,9 +679,9 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
     }
 
     if constexpr (kSplit) {
-        // Rows whose sums came out infinite or NaN (which may be the planes'
-        // doing, mfma.hpp), once more with f32 MFMAs on operands read from
-        // memory, over the rows stored above.
+        // Sums that came out infinite or NaN (which may be the planes' doing,
+        // mfma.hpp), once more with f32 MFMAs on operands read from memory, over
+        // the values stored above.  (A row at a time; its other values stay.)
         wait_vmcnt<0>();
         __syncthreads();  // everyone's stores of the tile are done
         bad |= __shfl_xor(bad, 16);
@@ -705,13 +719,19 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                 if constexpr (MODE == kGateUp) {
                     if (i % 4 >= 2) continue;  // (with its gate block)
                     const int hc = (n0 + wn * WN + i / 4 * 64) / 2 + i % 2 * 16 + 4 * lq;
+                    const uint32_t units = bad_units[(i / 4 * 2 + i % 2) % (SN / 2)] >> (4 * j) & 15u;
+                    if (!units) continue;
                     float hv[4];
+                    load_hidden(a.out, a.a_cap, row0 + m, hc, hv);
 #pragma unroll
                     for (int s = 0; s < 4; ++s)
-                        hv[s] = hc + s < a.n_out ? swiglu<T>(again[i][s], again[(i + 2) % SN][s]) : 0.0f;
+                        if (units >> s & 1) hv[s] = hc + s < a.n_out ? swiglu<T>(again[i][s], again[(i + 2) % SN][s]) : 0.0f;
                     store_hidden<T>(a.out, a.a_cap, row0 + m, hc, hv);
                 } else if (n < a.n_out) {
-                    *reinterpret_cast<f32x4_t*>(out + (int64_t)(row0 + m) * a.n_out + n) = again[i];
+                    f32x4_t* y = reinterpret_cast<f32x4_t*>(out + (int64_t)(row0 + m) * a.n_out + n);
+                    f32x4_t v = *y;
+                    keep_finite(v, again[i]);
+                    *y = v;
                 }
             }
         }

@@ -168,9 +168,21 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
                 }
             }
 #pragma unroll
-            for (int i = 0; i < NB; ++i)
+            for (int j = 0; j < NT; ++j) {
+                if constexpr (MODE == kDown) {
 #pragma unroll
-                for (int j = 0; j < NT; ++j) keep_finite(acc[i][j], again[i][j]);
+                    for (int i = 0; i < NB; ++i) keep_finite(acc[i][j], again[i][j]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) {
+                            const bool ok = unit_finite(acc[i][j][s], acc[i + 2][j][s]);
+                            acc[i][j][s] = ok ? acc[i][j][s] : again[i][j][s];
+                            acc[i + 2][j][s] = ok ? acc[i + 2][j][s] : again[i + 2][j][s];
+                        }
+                }
+            }
         }
     }
     // Epilogue.  Lane (l16, lq) of block (i, j) holds token row 16 j + l16 and

@@ -123,13 +123,14 @@ __device__ __forceinline__ void split_exact_n(const float* v, uint32_t (&pl)[kPl
         for (int p = 0; p < kPlanes; ++p) pl[p][d] = q[p];
     }
 }
-// Value s (0-7) of a lane's fragment from its planes.
+// A value from its planes: the low (0) or high (1) half of each plane's word.
+__device__ __forceinline__ float unsplit1(uint32_t p0, uint32_t p1, uint32_t p2, int half) {
+    auto v = [&](uint32_t p) { return __uint_as_float(half ? p & 0xffff0000u : p << 16); };
+    return v(p0) + (v(p1) + v(p2));
+}
+// Value s (0-7) of a lane's fragment.
 __device__ __forceinline__ float unsplit(const u32x4_t (&pl)[kPlanes], int s) {
-    float v[kPlanes];
-#pragma unroll
-    for (int p = 0; p < kPlanes; ++p)
-        v[p] = __uint_as_float(s % 2 ? pl[p][s / 2] & 0xffff0000u : pl[p][s / 2] << 16);
-    return v[0] + (v[1] + v[2]);
+    return unsplit1(pl[0][s / 2], pl[1][s / 2], pl[2][s / 2], s % 2);
 }
 __device__ __forceinline__ f32x4_t mfma_plane(const u32x4_t& a, const u32x4_t& b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
@@ -141,10 +142,16 @@ __device__ __forceinline__ float not_finite(const f32x4_t& v, float t) {
     for (int s = 0; s < 4; ++s) t = __builtin_fmaf(v[s], 0.0f, t);
     return t;
 }
-// The values of v, those that are not finite from `again`.
+// Which values are taken from the f32 MFMAs: in the down GEMM each sum that is
+// not finite, in gate/up both sums of a hidden unit where one is not (h alone
+// does not say which).  Both GEMM kernels keep all other values as they are, so
+// that a row's bits do not depend on the kernel.
 __device__ __forceinline__ void keep_finite(f32x4_t& v, const f32x4_t& again) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) v[s] = __builtin_isfinite(v[s]) ? v[s] : again[s];
+}
+__device__ __forceinline__ bool unit_finite(float g, float u) {
+    return __builtin_isfinite(g) && __builtin_isfinite(u);
 }
 
 enum { kGateUp = 0, kDown = 1 };  // the two GEMMs of an expert
@@ -157,6 +164,21 @@ __device__ __forceinline__ float swiglu(float g, float u) {
     else return g / (1.0f + expf(-g)) * u;
 }
 
+// Where hidden units hc..hc+3 (hc % 4 == 0) of row r are in the first plane of an f32 h.
+__device__ __forceinline__ unsigned char* hidden_at(void* h, int64_t a_cap, int r, int hc) {
+    return static_cast<unsigned char*>(h) + ((int64_t)(hc / 32 * kPlanes) * a_cap + r) * kKBlockBytes +
+           hc / 4 % 4 * 16 + hc / 16 % 2 * 8;
+}
+// ... and their values.
+__device__ __forceinline__ void load_hidden(void* h, int64_t a_cap, int r, int hc, float (&v)[4]) {
+    const unsigned char* src = hidden_at(h, a_cap, r, hc);
+    uint2 p[kPlanes];
+#pragma unroll
+    for (int t = 0; t < kPlanes; ++t) p[t] = *reinterpret_cast<const uint2*>(src + t * a_cap * kKBlockBytes);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+        v[s] = s < 2 ? unsplit1(p[0].x, p[1].x, p[2].x, s % 2) : unsplit1(p[0].y, p[1].y, p[2].y, s % 2);
+}
 // Hidden units hc..hc+3 (hc % 4 == 0) of row r into h, K-blocked (f32: planes).
 template <typename T>
 __device__ __forceinline__ void store_hidden(void* h, int64_t a_cap, int r, int hc, const float (&v)[4]) {
@@ -164,8 +186,7 @@ __device__ __forceinline__ void store_hidden(void* h, int64_t a_cap, int r, int 
     if constexpr (sizeof(T) == 4) {
         uint32_t pl[kPlanes][2];
         split_exact_n<4>(v, pl);
-        dst = static_cast<unsigned char*>(h) + ((int64_t)(hc / 32 * kPlanes) * a_cap + r) * kKBlockBytes +
-              hc / 4 % 4 * 16 + hc / 16 % 2 * 8;
+        dst = hidden_at(h, a_cap, r, hc);
 #pragma unroll
         for (int p = 0; p < kPlanes; ++p)
             *reinterpret_cast<uint2*>(dst + p * a_cap * kKBlockBytes) = make_uint2(pl[p][0], pl[p][1]);

@@ -116,6 +116,40 @@ def test_f32_values_that_have_no_finite_planes(rows, D, H):
     assert (got - want).norm() <= 1e-5 * want.norm() * np.sqrt(D)  # want: (rows, 1), got: its D columns
 
 
+def test_f32_repaired_rows_do_not_depend_on_the_call():
+    """A gate weight and a down weight of 3.4e38 make one hidden unit and one
+    output column of every row sums that the planes cannot hold.  Those values
+    are made again, every other one keeps its bits: a row is the same in a call
+    of 9,000 rows (256-row tiles in both GEMMs) and in small ones."""
+    rows, D, H = 9000, 1000, 2667
+    g = torch.Generator(device="cuda").manual_seed(9)
+
+    def randn(*shape, std):
+        return (torch.randn(*shape, generator=g, device="cuda") * std).cpu().numpy()
+
+    w = {"ffn.gate.weight": randn(H, D, std=D ** -0.5), "ffn.up.weight": randn(H, D, std=D ** -0.5),
+         "ffn.down.weight": randn(D, H, std=H ** -0.5), "ffn.up.bias": randn(H, std=0.1)}
+    w["ffn.gate.weight"][5, 2] = 3.4e38
+    w["ffn.up.weight"][9] = 0.0
+    w["ffn.up.bias"][9] = 1e-30
+    w["ffn.down.weight"][7, 9] = 3.4e38
+    zeros = {"ffn.gate.bias": np.zeros(H, np.float32), "ffn.down.bias": np.zeros(D, np.float32)}
+    layer = nm.FeedForward.from_source(nm.Weights.tensors_({**w, **zeros}, "f32"), "ffn", D, H)
+    x = torch.randn(rows, D, generator=g, device="cuda")
+    x[:, 2] = 1e-30
+    y = layer.forward(x)
+    for n in (40, 700):
+        assert torch.equal(layer.forward(x[:n]), y[:n]), n
+    # and right: every column to f32 sums of about 3,000 terms
+    t = {k: torch.from_numpy(v).cuda().double() for k, v in w.items()}
+    xd = x[:200].double()
+    gate, up = xd @ t["ffn.gate.weight"].T, xd @ t["ffn.up.weight"].T + t["ffn.up.bias"]
+    want = (gate * torch.sigmoid(gate) * up) @ t["ffn.down.weight"].T
+    err = (y[:200].double() - want).norm(dim=0) / want.norm(dim=0)
+    print(f"  worst column {float(err.max()):.2e}", flush=True)
+    assert err.max() <= 5e-6
+
+
 @pytest.mark.parametrize("shift", [0, 64, -64])
 def test_host_output_over_the_input(shift):
     """A pinned host output that is the input, or overlaps it some rows on."""
