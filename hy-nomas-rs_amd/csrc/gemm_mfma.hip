@@ -290,7 +290,7 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                 float4 b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
                 if (wu.part == 0) b = *reinterpret_cast<const float4*>(bias + i * 16);
 #pragma unroll
-                for (int j = 0; j < SM; ++j) acc[i][j] = f32x4_t{b.x, b.y, b.z, b.w};
+                for (int j = 0; j < SM; ++j) acc[i][j] = f32x4_t{b.x, b.y, b.z, b.w} * a.sum_up;
             }
             wait_vmcnt<QS>();
             __builtin_amdgcn_s_barrier();
@@ -521,6 +521,7 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
             for (int i = 0; i < SN; ++i) t = not_finite(acc[i][j], t);
             bad |= (t != t ? 1u : 0u) << j;
         }
+        if (a.all_f32) bad = (1u << SM) - 1;
     }
     // gate/up: which hidden units (bit 4 j + s of gate block 4 p + b in word 2 p + b)
     uint32_t bad_units[SN / 2] = {};
@@ -532,7 +533,8 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                 for (int j = 0; j < SM; ++j)
 #pragma unroll
                     for (int s = 0; s < 4; ++s)
-                        bad_units[i] |= (unit_finite(acc[i / 2 * 4 + i % 2][j][s], acc[i / 2 * 4 + i % 2 + 2][j][s]) ? 0u : 1u)
+                        bad_units[i] |= (unit_finite(acc[i / 2 * 4 + i % 2][j][s], acc[i / 2 * 4 + i % 2 + 2][j][s]) &&
+                                                 !a.all_f32 ? 0u : 1u)
                                         << (4 * j + s);
         }
     }
@@ -574,7 +576,7 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                     for (int b = 0; b < 2; ++b)
 #pragma unroll
                         for (int s = 0; s < 4; ++s)
-                            v[b * 4 + s] = swiglu<T>(acc[4 * p + b][j][s], acc[4 * p + b + 2][j][s]);
+                            v[b * 4 + s] = swiglu<T>(acc[4 * p + b][j][s] * a.sum_down, acc[4 * p + b + 2][j][s] * a.sum_down);
                     uint32_t pl[kPlanes][4];
                     split_exact_n<8>(v, pl);
 #pragma unroll
@@ -633,7 +635,8 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                 for (int jj = 0; jj < kJR; ++jj) {
                     T ov[4];
 #pragma unroll
-                    for (int s = 0; s < 4; ++s) ov[s] = Elt<T>::from_f32(acc[i][rd * kJR + jj][s]);
+                    for (int s = 0; s < 4; ++s)
+                        ov[s] = Elt<T>::from_f32(kSplit ? acc[i][rd * kJR + jj][s] * a.sum_down : acc[i][rd * kJR + jj][s]);
                     Raw4 raw;
                     __builtin_memcpy(&raw, ov, sizeof(raw));
                     *reinterpret_cast<Raw4*>(sO + (wm * kWR + jj * 16 + l16) * kOS + nl * (int)sizeof(T)) = raw;
@@ -709,7 +712,7 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                         const f32x4_t fa = *reinterpret_cast<const f32x4_t*>(w + i * 16 * BK);
 #pragma unroll
                         for (int k4 = 0; k4 < 4; ++k4)
-                            again[i] = mfma_f32(fa[k4], unsplit(pl, c * 4 + k4), again[i]);
+                            again[i] = mfma_f32(fa[k4] * a.w_down, unsplit(pl, c * 4 + k4), again[i]);
                     }
             }
             if (!mine) continue;
@@ -729,8 +732,11 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                     store_hidden<T>(a.out, a.a_cap, row0 + m, hc, hv);
                 } else if (n < a.n_out) {
                     f32x4_t* y = reinterpret_cast<f32x4_t*>(out + (int64_t)(row0 + m) * a.n_out + n);
-                    f32x4_t v = *y;
-                    keep_finite(v, again[i]);
+                    f32x4_t v = again[i];
+                    if (!a.all_f32) {
+                        v = *y;
+                        keep_finite(v, again[i]);
+                    }
                     *y = v;
                 }
             }

@@ -91,6 +91,12 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
     for (int i = 0; i < NB; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = NW == 1 ? bias(i) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (kSplit && NW == 1) {  // f32: the sums are scaled (mfma.hpp)
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] *= a.sum_up;
+    }
     V fa[P][KS][NB], fb[P][XS][NT];
     auto load = [&](int st, V (&wa)[KS][NB], V (&xb)[XS][NT]) {  // the fragments of step st
 #pragma unroll
@@ -146,7 +152,11 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
         for (int i = 0; i < NB; ++i)
 #pragma unroll
             for (int j = 0; j < NT; ++j) t = not_finite(acc[i][j], t);
-        if (__any(t != t)) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] *= a.sum_down;
+        if (a.all_f32 || __any(t != t)) {
             f32x4_t again[NB][NT];
 #pragma unroll
             for (int i = 0; i < NB; ++i)
@@ -164,12 +174,15 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
                     for (int k8 = 0; k8 < 8; ++k8)
 #pragma unroll
                         for (int i = 0; i < NB; ++i)
-                            again[i][j] = mfma_f32(wa[k8 / 4][i][k8 % 4], unsplit(pl, k8), again[i][j]);
+                            again[i][j] = mfma_f32(wa[k8 / 4][i][k8 % 4] * a.w_down, unsplit(pl, k8), again[i][j]);
                 }
             }
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                if constexpr (MODE == kDown) {
+                if (a.all_f32) {
+#pragma unroll
+                    for (int i = 0; i < NB; ++i) acc[i][j] = again[i][j];
+                } else if constexpr (MODE == kDown) {
 #pragma unroll
                     for (int i = 0; i < NB; ++i) keep_finite(acc[i][j], again[i][j]);
                 } else {

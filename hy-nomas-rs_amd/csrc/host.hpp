@@ -295,6 +295,10 @@ private:
     float* d_b1_ = nullptr;   // [Ecols][2 Hp], f32
     void* d_w2_ = nullptr;    // down, K-blocked: [Ecols][Hp / KB][Dn][KB]
     float* d_b2_ = nullptr;   // [Ecols][Dn]
+    // f32: what the device weights were multiplied by, and whether the GEMM
+    // makes all its sums with f32 MFMAs (GemmArgs)
+    float w1_scale_ = 1.0f, w2_scale_ = 1.0f;
+    bool w1_all_f32_ = false, w2_all_f32_ = false;
 
     // the handle's workspace (sized for ws_.cap_rows rows)
     void* d_ws_ = nullptr;

@@ -103,6 +103,7 @@ __host__ __device__ constexpr int64_t round_up(int64_t n, int64_t m) { return (n
 // weights of two 16-column f32 K-blocks.  Element (r, k) of plane p:
 //   ((k / 32 * 3 + p) * R + r) * 32 + (k / 4 % 4) * 8 + (k / 16 % 2) * 4 + k % 4
 constexpr int kActPlanes = 3;
+constexpr float kPlaneScale = 0x1p24f;  // the planes add up to the value times this (mfma.hpp)
 // Bytes of one element of x_perm or h.
 __host__ __device__ constexpr int act_bytes(DType dt) { return dt == DType::F32 ? 2 * kActPlanes : 2; }
 // Columns of a K-blocked operand with K = `k` columns of es-byte elements.
@@ -158,6 +159,11 @@ struct GemmArgs {
     // split tile (zero between launches: the last part to arrive resets it)
     float* split_ws;
     int32_t* split_cnt;
+    // f32: W holds the weights times a power of two (kPlaneScale or 1) and the sums
+    // of planes come out times sum_up; their inverses; and whether every sum is
+    // made with f32 MFMAs (weights too large to be scaled, others too small not to be)
+    float w_down = 1.0f, sum_up = 1.0f, sum_down = 1.0f;
+    bool all_f32 = false;
     // the ticket counter of the tail units handed out at run time
     // (zero before the launch: the kernel that writes the tile table clears it)
     int32_t* tail_cnt = nullptr;

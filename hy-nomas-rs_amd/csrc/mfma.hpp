@@ -40,14 +40,20 @@ __device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
 // MFMA does a plane product in 1/16 of the time of the f32 MFMAs.  Weights stay
 // f32 in memory and are split by the GEMM; activations (x_perm, h) are split
 // once, by the kernels that write them (kernels.hpp).
-// (A plane below bf16's smallest normal, 2^-126, may be flushed: values below
-// 2^-110 keep fewer of their bits.)
-// Sums that come out infinite or NaN are made again with f32 MFMAs by the GEMMs
-// (products with the planes of an infinite value, or of a weight that rounds
-// past bf16's largest, are not the product).
+// The matrix cores flush planes below bf16's smallest normal, 2^-126: a value
+// below 2^-107 would lose bits (of weights of 2^-115 the product kept 16).  So
+// both operands are taken times 2^24, where the last bit of every f32 value
+// is a normal bf16: activations when they are split, weights once at upload (but
+// not a layer that holds a weight of 2^103 or more).  The sums are scaled back
+// by the epilogue, exactly (partial sums overflow from 2^80 on instead of 2^128).
+// Sums that come out infinite or NaN are made again with f32 MFMAs by the GEMMs:
+// those, and products with a value that has no planes (2^103 and more, infinite,
+// NaN: the mark below) or with a weight that rounds past bf16's largest.
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kPlanes = 3;
 constexpr int kProducts = 6;
+constexpr float kPlaneMax = 0x1p127f;  // of a value times kPlaneScale
+constexpr uint32_t kRawMark = 0x7f80;  // plane 1 (infinite) of a value stored as its raw halves in planes 0 and 2
 __host__ __device__ constexpr int product_a(int p) { return p == 0 ? 0 : p == 1 ? 2 : p == 2 ? 1 : p == 3 ? 0 : p == 4 ? 1 : 0; }
 __host__ __device__ constexpr int product_b(int p) { return p == 0 ? 2 : p == 1 ? 0 : p == 2 ? 1 : p == 3 ? 1 : p == 4 ? 0 : 0; }
 
@@ -97,20 +103,23 @@ __device__ __forceinline__ void split_all(const f32x4_t& a, const f32x4_t& b, u3
         split_step<3>(x0, x1, d, pl, t);
     }
 }
-// The planes of any two values, whose sum (p2 + p1) + p0 is the value again
-// also where it is infinite, NaN or rounds past bf16's largest.
+// The planes of any two values times kPlaneScale, or the values themselves
+// where they are too large.
 __device__ __forceinline__ void split_exact(float x0, float x1, uint32_t (&pl)[kPlanes]) {
 #pragma clang fp contract(off)  // the remainders are of the f32 value, not of the product it may come from
-    auto first = [](float x) {  // rounded to bf16, large values truncated
-        const float r = (float)(__bf16)x;
-        return __builtin_isinf(r) ? __uint_as_float(__float_as_uint(x) & 0xffff0000u) : r;
-    };
-    const float a0 = first(x0), a1 = first(x1);
-    const float r0 = __builtin_isfinite(x0) ? x0 - a0 : 0.0f, r1 = __builtin_isfinite(x1) ? x1 - a1 : 0.0f;
-    const float b0 = (float)(__bf16)r0, b1 = (float)(__bf16)r1;
-    pl[0] = cvt_pk_bf16(a0, a1);
-    pl[1] = cvt_pk_bf16(b0, b1);
-    pl[2] = cvt_pk_bf16(r0 - b0, r1 - b1);
+    const float s0 = x0 * kPlaneScale, s1 = x1 * kPlaneScale;
+    pl[0] = cvt_pk_bf16(s0, s1);
+    const float r0 = s0 - __uint_as_float(pl[0] << 16), r1 = s1 - __uint_as_float(pl[0] & 0xffff0000u);
+    pl[1] = cvt_pk_bf16(r0, r1);
+    pl[2] = cvt_pk_bf16(r0 - __uint_as_float(pl[1] << 16), r1 - __uint_as_float(pl[1] & 0xffff0000u));
+    const bool ok0 = __builtin_fabsf(s0) < kPlaneMax, ok1 = __builtin_fabsf(s1) < kPlaneMax;
+    if (!(ok0 && ok1)) {
+        const uint32_t b0 = __float_as_uint(x0), b1 = __float_as_uint(x1);
+        const uint32_t m = (ok0 ? 0 : 0xffffu) | (ok1 ? 0 : 0xffff0000u);
+        pl[0] = (pl[0] & ~m) | ((b0 >> 16 | (b1 & 0xffff0000u)) & m);
+        pl[1] = (pl[1] & ~m) | ((kRawMark | kRawMark << 16) & m);
+        pl[2] = (pl[2] & ~m) | (((b0 & 0xffffu) | b1 << 16) & m);
+    }
 }
 // ... of 4 or 8 values; plane p's bf16s in order in pl[p]
 template <int N>
@@ -125,8 +134,10 @@ __device__ __forceinline__ void split_exact_n(const float* v, uint32_t (&pl)[kPl
 }
 // A value from its planes: the low (0) or high (1) half of each plane's word.
 __device__ __forceinline__ float unsplit1(uint32_t p0, uint32_t p1, uint32_t p2, int half) {
-    auto v = [&](uint32_t p) { return __uint_as_float(half ? p & 0xffff0000u : p << 16); };
-    return v(p0) + (v(p1) + v(p2));
+    auto bits = [&](uint32_t p) { return half ? p & 0xffff0000u : p << 16; };
+    auto v = [&](uint32_t p) { return __uint_as_float(bits(p)); };
+    if (bits(p1) == kRawMark << 16) return __uint_as_float(bits(p0) | bits(p2) >> 16);
+    return (v(p0) + (v(p1) + v(p2))) * (1.0f / kPlaneScale);
 }
 // Value s (0-7) of a lane's fragment.
 __device__ __forceinline__ float unsplit(const u32x4_t (&pl)[kPlanes], int s) {

@@ -13,6 +13,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -70,6 +71,43 @@ void over_rows(int64_t n, size_t bytes, const F& fn) {
     }
     fn(0, n / parts);
     for (std::thread& t : ts) t.join();
+}
+
+// f32 weights times kPlaneScale, so that the bf16 planes hold all of their
+// bits (mfma.hpp): in place, unless one of them is too large for it.  Sets the
+// scale taken, and whether some are then too small for their planes.
+void scale_f32(std::vector<uint8_t>& w, float* scale, bool* all_f32) {
+    float* v = reinterpret_cast<float*>(w.data());
+    const int64_t n = (int64_t)(w.size() / sizeof(float));
+    std::mutex mu;
+    bool large = false, small = false;
+    over_rows(n, w.size(), [&](int64_t b, int64_t e) {
+        uint32_t most = 0, least = 0xffffffffu;  // of the magnitudes' bits, in their values' order
+        for (int64_t i = b; i < e; ++i) {
+            uint32_t m;
+            std::memcpy(&m, &v[i], 4);
+            m &= 0x7fffffffu;
+            most = std::max(most, m);
+            least = std::min(least, m - 1);  // (zero: the largest)
+        }
+        std::lock_guard<std::mutex> lk(mu);
+        large |= most >= (103u + 127) << 23;      // 2^103, infinite, NaN
+        small |= least < ((127u - 102) << 23) - 1;  // nonzero below 2^-102
+    });
+    *scale = large ? 1.0f : kPlaneScale;
+    *all_f32 = large && small;
+    if (!large)
+        over_rows(n, w.size(), [&](int64_t b, int64_t e) {
+            for (int64_t i = b; i < e; ++i) v[i] *= kPlaneScale;
+        });
+}
+
+// The scales of a GEMM's operands (all of them powers of two).
+void set_scale(GemmArgs& g, float w_scale, bool all_f32) {
+    g.w_down = 1.0f / w_scale;
+    g.sum_up = kPlaneScale * w_scale;
+    g.sum_down = 1.0f / g.sum_up;
+    g.all_f32 = all_f32;
 }
 
 inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -252,6 +290,11 @@ int MoeLayer::upload(const void* router_w, const void* gate_w, const void* gate_
             b2[(size_t)(e * Dn_ + n)] = bsrc(down_b, dd_b, e, D, n);
         }
     });
+
+    if (dt_ == DType::F32) {
+        scale_f32(w1, &w1_scale_, &w1_all_f32_);
+        scale_f32(w2, &w2_scale_, &w2_all_f32_);
+    }
 
     for (void* p : {d_wr_, d_w1_, (void*)d_b1_, d_w2_, (void*)d_b2_})
         if (p) (void)hipFree(p);
@@ -640,6 +683,7 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     g1.X = w.xperm;
     g1.W = d_w1_;
     g1.bias = d_b1_;
+    set_scale(g1, w1_scale_, w1_all_f32_);
     g1.out = w.h;
     g1.tiles = w.tiles;
     g1.tile_total = w.tile_total;
@@ -659,6 +703,7 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     g2.X = w.h;
     g2.W = d_w2_;
     g2.bias = d_b2_;
+    set_scale(g2, w2_scale_, w2_all_f32_);
     g2.out = w.yperm;
     g2.tail_cnt = w.tile_total + 2;
     if (plan.bm2 != plan.bm1) {
@@ -736,6 +781,7 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     g1.dense_rows = plan.waves1 ? rows : 0;  // (gemm_mfma: the table)
     g1.W = d_w1_;
     g1.bias = d_b1_;
+    set_scale(g1, w1_scale_, w1_all_f32_);
     g1.out = w.h;
     g1.tiles = w.tiles;
     g1.tile_total = w.tile_total;
@@ -756,6 +802,7 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     g2.X = w.h;
     g2.W = d_w2_;
     g2.bias = d_b2_;
+    set_scale(g2, w2_scale_, w2_all_f32_);
     g2.out = y;  // rows stay in order: the output is y itself
     g2.tail_cnt = w.tile_total + 2;
     g2.max_tiles = max_tiles(rows, plan.bm2);

@@ -150,6 +150,41 @@ def test_f32_repaired_rows_do_not_depend_on_the_call():
     assert err.max() <= 5e-6
 
 
+# calls of few rows (whole tiles and padded), and of 256-row tiles
+@pytest.mark.parametrize("rows,D,H", [(70, 256, 128), (70, 264, 100), (9000, 1024, 2048), (9000, 1000, 2667)])
+@pytest.mark.parametrize("exp", [-112, -119, -126])
+@pytest.mark.parametrize("tiny", ["x", "up", "down", "up, one large", "down, one large"])
+def test_f32_tiny_values(tiny, exp, rows, D, H):
+    """Activations or weights around 2^exp, down to subnormal ones: as exact as f32
+    sums of values near 1 (TIGHT's 5e-6; at 2^-126 the results' own last
+    place is up to 2^-22 of them, 2.4e-7).  One weight of 3e38 among them, on
+    an input that is zero, changes nothing."""
+    g = torch.Generator(device="cuda").manual_seed(10)
+
+    def randn(*shape, std):
+        return (torch.randn(*shape, generator=g, device="cuda", dtype=torch.float64) * std).float().cpu().numpy()
+
+    sc = 2.0 ** exp
+    w = {"ffn.gate.weight": np.zeros((H, D), np.float32), "ffn.gate.bias": np.ones(H, np.float32),
+         "ffn.up.weight": randn(H, D, std=D ** -0.5 * (sc if tiny[:2] == "up" else 1)),
+         "ffn.up.bias": np.zeros(H, np.float32),
+         "ffn.down.weight": randn(D, H, std=H ** -0.5 * (sc if tiny[:4] == "down" else 1)),
+         "ffn.down.bias": np.zeros(D, np.float32)}
+    x = torch.from_numpy(randn(rows, D, std=sc if tiny == "x" else 1)).cuda()
+    if tiny == "up, one large":
+        w["ffn.up.weight"][3, 4] = 3e38
+        x[:, 4] = 0.0
+    if tiny == "down, one large":
+        w["ffn.up.weight"][6] = 0.0
+        w["ffn.down.weight"][5, 6] = 3e38
+    y = nm.FeedForward.from_source(nm.Weights.tensors_(w, "f32"), "ffn", D, H).forward(x)[:200].double()
+    t = {k: torch.from_numpy(v).cuda().double() for k, v in w.items()}
+    want = (x[:200].double() @ t["ffn.up.weight"].T * torch.sigmoid(torch.ones(1).double().cuda())) @ t["ffn.down.weight"].T
+    err = float((y - want).norm() / want.norm())
+    print(f"  {tiny} 2^{exp} {rows} x {D} x {H}: {err:.2e}", flush=True)
+    assert err <= 5e-6
+
+
 @pytest.mark.parametrize("shift", [0, 64, -64])
 def test_host_output_over_the_input(shift):
     """A pinned host output that is the input, or overlaps it some rows on."""
