@@ -341,6 +341,8 @@ private:
     static constexpr int kRing = 512;
     std::vector<hipEvent_t> events_;
     std::vector<uint8_t> stage_empty_;  // kProfStages flags per event set
+    std::vector<uint8_t> later_piece_;  // per event set: a piece of the call that the set before belongs to
+    int64_t piece_ = 0;                 // the pieced call in progress: pieces run before this one
     int recorded_ = 0;
 };
 

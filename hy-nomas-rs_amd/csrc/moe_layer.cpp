@@ -553,13 +553,14 @@ int MoeLayer::forward_noalloc(const void* x, void* y, int64_t rows, hipStream_t 
     Workspace w;
     layout(piece, false, static_cast<uint8_t*>(base), &w, cap);
     if (done_recorded_ && s != last_stream_) HIP_TRY(hipStreamWaitEvent(s, done_, 0));
-    const Scoped whole(plan_rows_, rows);
+    const Scoped whole(plan_rows_, rows), part(piece_, 0);
     // A piece writes its rows of y before the next one reads its rows of x:
     // where y overlaps x from above, the pieces run from the last one down.
     const int pieces = (int)((rows + piece - 1) / piece);
     const bool down = reinterpret_cast<uintptr_t>(y) > reinterpret_cast<uintptr_t>(x);
     for (int i = 0; i < pieces; ++i) {
         const int64_t at = down ? pieces - 1 - i : i, off = at * piece;
+        piece_ = i;
         Workspace p = w;
         p.idx += off * kslots_;
         p.w += off * kslots_;
@@ -602,6 +603,7 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     if (profiling_) {
         ev = &events_[(size_t)(recorded_ % kRing) * kProfEvents];
         empty = &stage_empty_[(size_t)(recorded_ % kRing) * kProfStages];
+        later_piece_[(size_t)(recorded_ % kRing)] = piece_ > 0;
         ++recorded_;
     }
     StageClock clock(ev, empty, s);
@@ -753,6 +755,7 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     if (profiling_) {
         ev = &events_[(size_t)(recorded_ % kRing) * kProfEvents];
         empty = &stage_empty_[(size_t)(recorded_ % kRing) * kProfStages];
+        later_piece_[(size_t)(recorded_ % kRing)] = piece_ > 0;
         ++recorded_;
     }
     StageClock clock(ev, empty, s);
@@ -922,12 +925,13 @@ int MoeLayer::forward_host_pieces(const void* x, void* y, int64_t rows, int np, 
         return code;
     };
     const bool out_pinned = is_pinned(y);
-    const Scoped whole(plan_rows_, rows);
+    const Scoped whole(plan_rows_, rows), part(piece_, 0);
     int n_pieces = 0;
     for (int p = 0; p < np; ++p) {
         const int64_t off = p * per, n = std::min(per, rows - off);
         if (n <= 0) break;
         n_pieces = p + 1;
+        piece_ = p;
         const size_t o = (size_t)off * rb;
         rc = stager_.to_device(static_cast<uint8_t*>(dx) + o, static_cast<const uint8_t*>(x) + o,
                                (size_t)n * rb, hs_copy_);
@@ -1029,6 +1033,7 @@ int MoeLayer::set_profiling(bool on) {
     if (on && events_.empty()) {
         events_.resize((size_t)kRing * kProfEvents);
         stage_empty_.assign((size_t)kRing * kProfStages, 0);
+        later_piece_.assign((size_t)kRing, 0);
         for (hipEvent_t& e : events_) HIP_TRY(hipEventCreateWithFlags(&e, hipEventReleaseToDevice));
     }
     profiling_ = on;
@@ -1042,7 +1047,10 @@ int MoeLayer::stage_times(float* ms6) {
         return set_error(NOMAS_ERR_STATE, "no profiled forward recorded");
     DeviceGuard g(device_);
     const int n = std::min(recorded_, kRing);
-    double sum[6] = {0, 0, 0, 0, 0, 0};
+    // from the newest set back; a call in pieces is the sum of its sets (one that
+    // the ring has lost the first of is left out)
+    double sum[6] = {0, 0, 0, 0, 0, 0}, call[6] = {0, 0, 0, 0, 0, 0};
+    int calls = 0;
     for (int i = 0; i < n; ++i) {
         const int set = (recorded_ - 1 - i) % kRing;
         hipEvent_t* ev = &events_[(size_t)set * kProfEvents];
@@ -1053,10 +1061,16 @@ int MoeLayer::stage_times(float* ms6) {
             if (empty[st]) continue;  // no kernel: zero
             float ms = 0.0f;
             HIP_TRY(hipEventElapsedTime(&ms, ev[2 * st], ev[2 * st + 1]));
-            sum[st] += ms;
+            call[st] += ms;
+        }
+        if (later_piece_[(size_t)set]) continue;
+        ++calls;
+        for (int st = 0; st < 6; ++st) {
+            sum[st] += call[st];
+            call[st] = 0.0;
         }
     }
-    for (int st = 0; st < 6; ++st) ms6[st] = (float)(sum[st] / n);
+    for (int st = 0; st < 6; ++st) ms6[st] = calls ? (float)(sum[st] / calls) : 0.0f;
     recorded_ = 0;
     return NOMAS_OK;
 }

@@ -170,7 +170,8 @@ int nomas_moe_dims(const nomas_moe_t *h, int64_t *dim, int64_t *hidden, int64_t 
  * of a stage's first kernel and the end of its last, so a stage's time is its
  * kernels' own (no launch gap); a stage without a kernel reads zero.
  * nomas_moe_stage_times returns the mean over the forwards recorded since the
- * last call, in milliseconds: [router, scan, dispatch, gemm_gate_up,
+ * last call (the last 512; one that ran in row pieces is the sum of its
+ * pieces), in milliseconds: [router, scan, dispatch, gemm_gate_up,
  * gemm_down, combine] ("scan" is part of the dispatch kernel and reads zero).
  * Synchronises. */
 int nomas_moe_set_profiling(nomas_moe_t *h, int enable);

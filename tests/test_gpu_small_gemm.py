@@ -219,6 +219,33 @@ def test_noalloc_in_pieces():
         assert np.array_equal(a, b)
 
 
+def test_stage_times_of_a_call_in_pieces():
+    """The stage times of a call in row pieces are those of the whole call: about a
+    forward's in one piece (a mean over the pieces would be half of it or less)."""
+    rows, D, E, k, H = 2_000_000, 8, 3, 1, 4
+    t, _ = small_case(8, D, E, k, H, 84, router_std=0.5)
+    layer = layer_from_tensors(t, "bf16", D, H, E, k)
+    x = torch.randn(rows, D, device="cuda", generator=torch.Generator(device="cuda").manual_seed(8)).to(torch.bfloat16)
+    y = torch.empty_like(x)
+    host = x.cpu()
+
+    def gemm_ms(call):
+        call()
+        layer.set_profiling(True)
+        for _ in range(3):
+            call()
+        torch.cuda.synchronize()
+        st = layer.stage_times()
+        layer.set_profiling(False)
+        return st["gemm_gate_up"] + st["gemm_down"] + st["router"]
+
+    one = gemm_ms(lambda: layer.forward(x, out=y))
+    for name, call in (("no allocation", lambda: _noalloc(layer, x, y)), ("host tensor", lambda: layer.forward(host))):
+        ms = gemm_ms(call)
+        print(f"  {name}: {ms:.3f} ms, in one piece {one:.3f} ms", flush=True)
+        assert ms >= 0.75 * one, name
+
+
 @pytest.mark.parametrize("shift", [0, 64, -64])
 def test_noalloc_in_pieces_output_over_the_input(shift):
     """y is x, or overlaps it some rows on: every piece reads rows of x that
