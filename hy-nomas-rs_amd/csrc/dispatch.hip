@@ -556,7 +556,7 @@ hipError_t launch_dispatch_t(const DispatchArgs& a, hipStream_t s) {
     if (a.nchunks != nblk || a.count_rows < kMinRouterBlockRows || a.count_rows > kRouterRows ||
         kRouterRows % a.count_rows != 0 || a.E_cols < 1 || a.E_cols > kMaxExperts + 1 || a.k_slots < 1 ||
         a.k_slots > a.E_cols || a.BM < 1 || a.BM2 < 1 || !dispatch_fits(a.E_cols, a.k_slots) ||
-        a.Dk != padded_k(a.D, sizeof(T)))
+        (a.Dk != padded_k(a.D, sizeof(T)) && a.Dk != step_k(a.D)))
         return hipErrorInvalidValue;
     const size_t lds = dispatch_lds(a.E_cols, a.k_slots);
     // the load hint and the padding as compile-time choices: no test in the copy loop.
@@ -613,7 +613,7 @@ hipError_t launch_kblock(DType dt, const void* x, void* xk, int64_t rows, int D,
                          int64_t a_cap, int BM, int max_tiles, TileInfo* tiles, int32_t* tile_total,
                          hipStream_t s) {
     if (rows <= 0) return hipSuccess;
-    if (Dk != padded_k(D, (int)dtype_size(dt)) || a_cap < rows || BM < 1 || max_tiles < 1)
+    if ((Dk != padded_k(D, (int)dtype_size(dt)) && Dk != step_k(D)) || a_cap < rows || BM < 1 || max_tiles < 1)
         return hipErrorInvalidValue;
     const int64_t chunks = rows * (Dk / (16 / (int)dtype_size(dt)));
     const unsigned nblk = (unsigned)std::min<int64_t>((chunks + 255) / 256, 65536);

@@ -46,7 +46,8 @@ inline GemmPlan gemm_plan(DType dt, int64_t A, int64_t E, int64_t Dk, int64_t Hp
     const bool padded = D % kMfmaBN != 0 || H != Hp;
     const bool f32 = dt == DType::F32;
     const double kb = kKBlockBytes / (double)dtype_size(dt);
-    const double kt1 = Dk / kb, kt2 = Hp / kb;  // k steps of gate/up and down
+    // k steps of gate/up and down: gemm_mfma's, and gemm_rows' (kernels.hpp)
+    const double kt1 = Dk / kb, kt2 = Hp / kb, kr1 = step_k(D) / kb, kr2 = step_k(H) / kb;
     const double live = (double)std::max<int64_t>(1, std::min(A, E)), mean = A / live;
     auto tiles = [&](int bm) { return live * std::max(1.0, mean / bm + 0.5); };  // row tiles, about
     auto cost_mfma = [&](double cols, double kt) {
@@ -60,11 +61,11 @@ inline GemmPlan gemm_plan(DType dt, int64_t A, int64_t E, int64_t Dk, int64_t Hp
     const struct { int bm; double ns, ns_kt, ns_f32, ns_kt_f32; } opts[] = {
         {16, 3.8, 0.27, 12, 0.25}, {32, 5, 0.31, 7.5, 0.44}, {64, 5.3, 0.47, 8, 0.8}};
     // the least cost of a GEMM over the choices (all of them, or those of one tile height)
-    auto pick = [&](double cols_mfma, double cols, double kt, int only, int* bm, int* waves) {
+    auto pick = [&](double cols_mfma, double kt_mfma, double cols, double kt, int only, int* bm, int* waves) {
         double least = 1e30;
         *bm = kMfmaBM;
         if (!only || only == kMfmaBM) {
-            least = cost_mfma(cols_mfma, kt);
+            least = cost_mfma(cols_mfma, kt_mfma);
             *waves = 0;
         }
         for (const auto& o : opts) {
@@ -82,8 +83,8 @@ inline GemmPlan gemm_plan(DType dt, int64_t A, int64_t E, int64_t Dk, int64_t Hp
         return least;
     };
     auto both = [&](int only, GemmPlan* p) {
-        const double c = pick(2.0 * Hp, 2.0 * Hp, kt1, only, &p->bm1, &p->waves1);
-        return c + pick((double)round_up(D, kMfmaBN), (double)D, kt2, only, &p->bm2, &p->waves2);
+        const double c = pick(2.0 * Hp, kt1, 2.0 * step_k(H), kr1, only, &p->bm1, &p->waves1);
+        return c + pick((double)round_up(D, kMfmaBN), kt2, (double)round_up(D, 64), kr2, only, &p->bm2, &p->waves2);
     };
     GemmPlan plan, one;
     double least = both(0, &plan);

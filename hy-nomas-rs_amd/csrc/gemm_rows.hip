@@ -52,7 +52,7 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
     const int N = a.N, K = a.K;
     const int live = a.dense_rows ? (int)((a.dense_rows + BM - 1) / BM) : min(*a.tile_total, a.max_tiles);
     // down: weight tiles past the real columns have nothing to store
-    const int ntn = (int)((MODE == kDown ? a.n_out + BN - 1 : N) / BN);
+    const int ntn = (MODE == kDown ? a.n_out + BN - 1 : a.n_used) / BN;
     const long long units = (long long)live * ntn;
     const long long share = (units + kNumXcd - 1) / kNumXcd;
     const long long q = blockIdx.x / kNumXcd, u = (blockIdx.x % kNumXcd) * share + q;
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
     const int l16 = lane & 15, lq = lane >> 4;
 
     // this wave's k steps (none in gate/up tiles that hold padding only)
-    const int kt_all = K / BK, st_all = kt_all / KS;
+    const int kt_all = K / BK, st_all = a.k_used / (BK * KS);
     const bool pad_tile = MODE == kGateUp && n0 / 2 >= a.n_out;
     const int s0 = pad_tile ? 0 : st_all * wave / NW, s1 = pad_tile ? 0 : st_all * (wave + 1) / NW;
     const int64_t wstep = (int64_t)N * BK, xstep = a.x_row ? kKBlockBytes : a.a_cap * kKBlockBytes;  // (elements, bytes)
@@ -262,10 +262,13 @@ hipError_t launch_rows_t(const GemmArgs& a, hipStream_t s) {
     if (a.N % kMfmaBN != 0 || a.K % (kblock_elems<T>() * kStages) != 0 || a.n_out < 1 || a.n_out > n_cols ||
         (MODE == kDown && a.n_out % 8 != 0))
         return hipErrorInvalidValue;
+    if (a.k_used < 1 || a.k_used % 32 != 0 || a.k_used > a.K ||
+        (MODE == kGateUp && (a.n_used < a.n_out * 2LL || a.n_used % kRowsBN != 0 || a.n_used > a.N)))
+        return hipErrorInvalidValue;
     if (a.x_row && (sizeof(T) != 2 || a.x_row % 16 != 0 || a.x_row < a.K * 2LL || a.x_row > (1LL << 26)))
         return hipErrorInvalidValue;
     if (a.max_tiles <= 0) return hipSuccess;
-    const int64_t ntn = (MODE == kDown ? a.n_out + kRowsBN - 1 : a.N) / kRowsBN;
+    const int64_t ntn = (MODE == kDown ? a.n_out + kRowsBN - 1 : a.n_used) / kRowsBN;
     const int64_t grid = round_up((int64_t)a.max_tiles * ntn, kNumXcd);
     if (grid > 0x7fffffff) return hipErrorInvalidValue;
     launch_kernel((gemm_rows_kernel<T, MODE, NT, NW>), dim3((unsigned)grid), dim3(NW * kWave), 0, s, a);

@@ -90,7 +90,9 @@ struct RouterArgs {
 // Any dim and hidden width run on the same GEMMs: the operands are padded with
 // zeros when they are laid out (weights at upload, x_perm by the dispatch, h
 // by the gate/up epilogue), K to whole turns of the GEMM's LDS ring and the
-// weight rows to whole tiles, so no GEMM loop has a remainder.
+// weight rows to whole tiles, so no GEMM loop has a remainder.  gemm_rows needs
+// whole steps of 32 only (step_k), and neither computes nor reads the rest of the
+// padding; where it runs the GEMM that reads an operand, the rest is not written.
 constexpr int kKBlockBytes = 64;
 constexpr int kStages = 4;  // K steps (K-blocks) per turn of the ring
 template <typename T>
@@ -111,6 +113,9 @@ __host__ __device__ constexpr int64_t padded_k(int64_t k, int es) {
     return round_up(k, kStages * kKBlockBytes / es);
 }
 
+// Columns that gemm_rows reads of an operand of `k` columns.
+__host__ __device__ constexpr int64_t step_k(int64_t k) { return round_up(k, 32); }
+
 struct DispatchArgs {
     const void* x;
     int64_t rows;
@@ -128,7 +133,7 @@ struct DispatchArgs {
     int32_t* tile_total;    // 4: the tile count, the two GEMMs' tail counters (cleared), the second count
     int32_t* tok_pos;  // rows x k_slots
     void* x_perm;      // a_cap x Dk, K-blocked (R = a_cap; f32: planes)
-    int Dk;            // padded_k(D): columns D .. Dk - 1 are written as zeros
+    int Dk;            // padded_k(D) or step_k(D): columns D .. Dk - 1 are written as zeros
     int64_t a_cap;     // rows of x_perm (positions must stay below)
 };
 
@@ -148,6 +153,10 @@ struct GemmArgs {
     int n_out;
     int num_experts;  // experts with weights (tiles naming others are skipped)
     int64_t a_cap;    // rows of X / out (tiles reaching beyond are skipped)
+    // gemm_rows: the columns of K that it walks (step_k of the real ones), and in
+    // gate/up the weight rows that it computes (those of step_k(H) hidden units,
+    // or N where gemm_mfma reads h)
+    int k_used = 0, n_used = 0;
     // gemm_rows: where X is not K-blocked (rows of x in place, whole K-blocks
     // of 16-bit elements): bytes from row to row; 0: K-blocked
     int64_t x_row = 0;
@@ -230,8 +239,8 @@ hipError_t launch_gemm_down(DType dt, const GemmArgs& a, const GemmPlan& plan, h
 hipError_t launch_gemm_mfma(DType dt, bool gate_up, const GemmArgs& a, hipStream_t s);
 hipError_t launch_gemm_rows(DType dt, bool gate_up, const GemmArgs& a, int bm, int waves, hipStream_t s);
 hipError_t launch_combine(DType dt, const CombineArgs& a, hipStream_t s);
-// Dense feed-forward (no routing): x re-laid out K-blocked with Dk =
-// padded_k(D) columns for the gate/up GEMM, and the tile table of `rows` rows
+// Dense feed-forward (no routing): x re-laid out K-blocked with Dk columns
+// (padded_k(D) or step_k(D)) for the gate/up GEMM, and the tile table of `rows` rows
 // of one expert in BM-row tiles (max_tiles entries written).
 hipError_t launch_kblock(DType dt, const void* x, void* xk, int64_t rows, int D, int Dk,
                          int64_t a_cap, int BM, int max_tiles, TileInfo* tiles, int32_t* tile_total,

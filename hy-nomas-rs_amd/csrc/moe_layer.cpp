@@ -676,7 +676,7 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     da.tile_total = w.tile_total;
     da.tok_pos = w.pos;
     da.x_perm = w.xperm;
-    da.Dk = (int)Dk_;
+    da.Dk = (int)(plan.waves1 ? step_k(D_) : Dk_);
     da.a_cap = a_cap;
     STAGE(launch_dispatch(dt_, da, s), "dispatch");
     if ((rc = mark(3))) return rc;
@@ -693,6 +693,8 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     g1.N = (int)(2 * Hp_);
     g1.K = (int)Dk_;
     g1.n_out = (int)H_;
+    g1.k_used = (int)step_k(D_);
+    g1.n_used = (int)(2 * (plan.waves2 ? step_k(H_) : Hp_));
     g1.num_experts = (int)Ecols_;
     g1.a_cap = a_cap;
     g1.split_ws = w.split_ws;
@@ -716,6 +718,7 @@ int MoeLayer::run_routed(const void* x, void* y, int64_t rows, hipStream_t s,
     g2.N = (int)Dn_;
     g2.K = (int)Hp_;
     g2.n_out = (int)D_;
+    g2.k_used = (int)step_k(H_);
     g2.out_nt = rows * kslots_ * D_ * (int64_t)dtype_size(dt_) > kLastLevelCacheBytes;
     STAGE(launch_gemm_down(dt_, g2, plan, s), "down GEMM");
     if ((rc = mark(5))) return rc;
@@ -774,7 +777,7 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     if ((rc = mark(2))) return rc;
     const bool in_place = plan.waves1 && plan.waves2 && dt_ != DType::F32 && D_ == Dk_;
     if (!in_place)
-        STAGE(launch_kblock(dt_, x, w.xperm, rows, (int)D_, (int)Dk_, w.cap_rows, kMfmaBM, mt, w.tiles,
+        STAGE(launch_kblock(dt_, x, w.xperm, rows, (int)D_, (int)(plan.waves1 ? step_k(D_) : Dk_), w.cap_rows, kMfmaBM, mt, w.tiles,
                             w.tile_total, s), "K-blocked copy");
     if ((rc = mark(3))) return rc;
 
@@ -792,6 +795,8 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     g1.N = (int)(2 * Hp_);
     g1.K = (int)Dk_;
     g1.n_out = (int)H_;
+    g1.k_used = (int)step_k(D_);
+    g1.n_used = (int)(2 * (plan.waves2 ? step_k(H_) : Hp_));
     g1.num_experts = 1;
     g1.a_cap = w.cap_rows;  // the K-blocked buffers' row capacity
     g1.split_ws = w.split_ws;
@@ -813,6 +818,7 @@ int MoeLayer::forward_dense(const void* x, void* y, int64_t rows, hipStream_t s)
     g2.N = (int)Dn_;
     g2.K = (int)Hp_;
     g2.n_out = (int)D_;
+    g2.k_used = (int)step_k(H_);
     STAGE(launch_gemm_down(dt_, g2, plan, s), "down GEMM");
     if ((rc = mark(5))) return rc;
     if ((rc = mark(6))) return rc;

@@ -41,6 +41,15 @@ def test_padded_widths(rows, D, H, dtype):
     run_case(rows, D, 3, 2, H, dtype, 600 + D + H, 0.5 if D == 72 else 0.0)
 
 
+# widths at the edges of the 32-wide steps that gemm_rows walks and of the 32 hidden
+# units of its gate/up tiles: it skips all other padding
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("D,H", [(24, 31), (32, 32), (40, 33), (96, 64), (136, 65), (160, 224)])
+@pytest.mark.parametrize("rows", [3, 700])
+def test_padding_that_is_skipped(rows, D, H, dtype):
+    run_case(rows, D, 3, 2, H, dtype, 650 + D + H, 0.5 if D == 40 else 0.0)
+
+
 # gate/up on 256-row tiles and down on 64-row ones (two tile tables)
 @pytest.mark.parametrize("D,H,dtype", [(1024, 2688, "bf16"), (1000, 2667, "bf16"), (512, 2048, "f32")])
 def test_gemms_of_different_tile_heights(D, H, dtype):
