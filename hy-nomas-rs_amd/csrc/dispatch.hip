@@ -68,8 +68,9 @@ __host__ __device__ inline bool dispatch_fits(int E_cols, int k) {
 //     rows are loaded with that hint too (no later kernel of the forward reads
 //     them); a smaller x is still in L2 from the router and loads faster
 //     without it.
-template <typename T, bool kNtX, bool kPad>
-__global__ __launch_bounds__(kDispThreads) void dispatch_kernel(DispatchArgs a) {
+//     kTwo: 64 registers a lane instead of 65, so that two blocks share a CU.
+template <typename T, bool kNtX, bool kPad, bool kTwo>
+__global__ __launch_bounds__(kDispThreads) __attribute__((amdgpu_waves_per_eu(kTwo ? 8 : 4))) void dispatch_kernel(DispatchArgs a) {
     extern __shared__ __align__(16) unsigned char s_raw[];
     // parts > 1: blocks b * parts .. b * parts + parts - 1 share chunk b, each
     // doing the bookkeeping and copying its own contiguous range of slabs
@@ -564,8 +565,20 @@ hipError_t launch_dispatch_t(const DispatchArgs& a, hipStream_t s) {
     // 41.9 -> 40.2 us; one 4,680-row segment (29 MB, in L2 after the router)
     // 17.6 -> 19.5 us (A/B on one box, two repeats each).
     const bool nt_x = a.rows * (int64_t)a.D * (int64_t)sizeof(T) > kL2TotalBytes;
-    auto kern = a.Dk == a.D ? (nt_x ? dispatch_kernel<T, true, false> : dispatch_kernel<T, false, false>)
-                            : (nt_x ? dispatch_kernel<T, true, true> : dispatch_kernel<T, false, true>);
+    // Two blocks per CU where there are more blocks than CUs, two fit the LDS and a
+    // row is one slab, so that the bookkeeping is most of a block's time: 65,536
+    // f32 rows of dim 8, 2 experts 38.5 -> 29.1 us; 400,000 bf16 rows of dim 8
+    // 778 -> 647 us; f32 rows of dim 128, 64 experts top-8, 17,000 to 400,000: 0.82-0.95
+    // of the time.  Longer rows gain less or lose (f32 dim 256, 64 experts
+    // top-8: 0.91-1.04; bf16 dim 1024, 8 experts top-2: 0.89-1.05).
+    const bool two = nblk > kDispCUs && 2 * lds <= 160 * 1024 && a.Dk * (int)sizeof(T) <= kSlabBytes;
+    auto pick = [&](auto nt, auto pad) {
+        constexpr bool kNt = decltype(nt)::value, kPad = decltype(pad)::value;
+        return two ? dispatch_kernel<T, kNt, kPad, true> : dispatch_kernel<T, kNt, kPad, false>;
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    auto kern = a.Dk == a.D ? (nt_x ? pick(yes, no) : pick(no, no)) : (nt_x ? pick(yes, yes) : pick(no, yes));
     hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                          (int)lds);
     if (err != hipSuccess) return err;

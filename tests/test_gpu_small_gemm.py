@@ -228,6 +228,18 @@ def test_noalloc_in_pieces():
         assert np.array_equal(a, b)
 
 
+# more 64-row chunks than CUs: two dispatch blocks share a CU (rows of one 512-byte
+# slab: padded, whole, and more x than the L2 caches hold), next to one of two slabs
+@pytest.mark.parametrize("rows,D,E,k,dtype", [(16448, 72, 6, 2, "f32"), (17000, 128, 40, 5, "bf16"), (16500, 128, 3, 1, "f32"),
+                                              (70000, 256, 4, 1, "bf16"), (70001, 248, 4, 2, "bf16"), (17000, 288, 6, 2, "bf16")])
+def test_dispatch_two_blocks_a_cu(rows, D, E, k, dtype):
+    t, x = small_case(rows, D, E, k, 24, 690 + D, router_std=0.5)
+    layer = layer_from_tensors(t, dtype, D, 24, E, k)
+    rt, rx = rounded(t, x, dtype)
+    p, dn = nm.workloads.oracle_params(rt, E)
+    compare(layer, to_device(x, dtype), rx, p, k, dtype, rows=np.unique(np.r_[np.arange(0, rows, 61), rows - 1]))
+
+
 def test_stage_times_of_a_call_in_pieces():
     """The stage times of a call in row pieces are those of the whole call: about a
     forward's in one piece (a mean over the pieces would be half of it or less)."""
