@@ -68,9 +68,11 @@ __host__ __device__ inline bool dispatch_fits(int E_cols, int k) {
 //     rows are loaded with that hint too (no later kernel of the forward reads
 //     them); a smaller x is still in L2 from the router and loads faster
 //     without it.
-//     kTwo: 64 registers a lane instead of 65, so that two blocks share a CU.
-template <typename T, bool kNtX, bool kPad, bool kTwo>
-__global__ __launch_bounds__(kDispThreads) __attribute__((amdgpu_waves_per_eu(kTwo ? 8 : 4))) void dispatch_kernel(DispatchArgs a) {
+// 64 registers a lane, so that two blocks share a CU where there are more
+// chunks than CUs: at 65, 400,000 bf16 rows of dim 8 took 778 us instead of 640,
+// 40,000 rows of dim 1024, 8 experts top-2, 52.6 instead of 49.
+template <typename T, bool kNtX, bool kPad>
+__global__ __launch_bounds__(kDispThreads) __attribute__((amdgpu_waves_per_eu(8))) void dispatch_kernel(DispatchArgs a) {
     extern __shared__ __align__(16) unsigned char s_raw[];
     // parts > 1: blocks b * parts .. b * parts + parts - 1 share chunk b, each
     // doing the bookkeeping and copying its own contiguous range of slabs
@@ -210,11 +212,17 @@ __global__ __launch_bounds__(kDispThreads) __attribute__((amdgpu_waves_per_eu(kT
     }
     __syncthreads();
     if (b == 0 && part == 0) {
+        // (its own arguments are read here: held from the start with all the
+        // others they spill scalar registers into a 65th vector register, one
+        // more than two blocks on a CU allow)
+        typedef const __attribute__((address_space(4))) DispatchArgs* Args;
+        Args late = (Args)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(late));
         for (int e = tid; e < Ec; e += kDispThreads) {
-            a.expert_count[e] = s_tot[e];
-            a.expert_off[e] = s_off[e];
+            late->expert_count[e] = s_tot[e];
+            late->expert_off[e] = s_off[e];
         }
-        if (tid == 0) a.expert_off[Ec] = s_off[Ec];
+        if (tid == 0) late->expert_off[Ec] = s_off[Ec];
         auto table = [&](int BM, int max_tiles, TileInfo* tiles, int32_t* total) {
             const int total_tiles = s_ts[Ec];
             if (tid == 0) *total = min(total_tiles, max_tiles);
@@ -233,18 +241,18 @@ __global__ __launch_bounds__(kDispThreads) __attribute__((amdgpu_waves_per_eu(kT
                 tiles[i] = t;
             }
         };
-        table(a.BM, a.max_tiles, a.tiles, &a.tile_total[0]);
+        table(late->BM, late->max_tiles, late->tiles, &late->tile_total[0]);
         if (tid == 0) {
-            a.tile_total[1] = 0;  // the GEMMs' tail counters
-            a.tile_total[2] = 0;
+            late->tile_total[1] = 0;  // the GEMMs' tail counters
+            late->tile_total[2] = 0;
         }
-        if (a.BM2 != a.BM) {  // the down GEMM's own table
+        if (late->BM2 != late->BM) {  // the down GEMM's own table
             __syncthreads();
             if (wave == 0) {
                 int carry = 0;
                 for (int e0 = 0; e0 < Ec; e0 += kWave) {
                     const int e = e0 + lane;
-                    const int v = e < Ec ? (s_tot[e] + a.BM2 - 1) / a.BM2 : 0;
+                    const int v = e < Ec ? (s_tot[e] + late->BM2 - 1) / late->BM2 : 0;
                     int inc = v;
 #pragma unroll
                     for (int o = 1; o < kWave; o <<= 1) {
@@ -257,7 +265,7 @@ __global__ __launch_bounds__(kDispThreads) __attribute__((amdgpu_waves_per_eu(kT
                 if (lane == 0) s_ts[Ec] = carry;
             }
             __syncthreads();
-            table(a.BM2, a.max_tiles2, a.tiles2, &a.tile_total[3]);
+            table(late->BM2, late->max_tiles2, late->tiles2, &late->tile_total[3]);
         }
     }
     // 3. ranks and positions.  Every wave holds each row's experts as a bit
@@ -565,20 +573,8 @@ hipError_t launch_dispatch_t(const DispatchArgs& a, hipStream_t s) {
     // 41.9 -> 40.2 us; one 4,680-row segment (29 MB, in L2 after the router)
     // 17.6 -> 19.5 us (A/B on one box, two repeats each).
     const bool nt_x = a.rows * (int64_t)a.D * (int64_t)sizeof(T) > kL2TotalBytes;
-    // Two blocks per CU where there are more blocks than CUs, two fit the LDS and a
-    // row is one slab, so that the bookkeeping is most of a block's time: 65,536
-    // f32 rows of dim 8, 2 experts 38.5 -> 29.1 us; 400,000 bf16 rows of dim 8
-    // 778 -> 647 us; f32 rows of dim 128, 64 experts top-8, 17,000 to 400,000: 0.82-0.95
-    // of the time.  Longer rows gain less or lose (f32 dim 256, 64 experts
-    // top-8: 0.91-1.04; bf16 dim 1024, 8 experts top-2: 0.89-1.05).
-    const bool two = nblk > kDispCUs && 2 * lds <= 160 * 1024 && a.Dk * (int)sizeof(T) <= kSlabBytes;
-    auto pick = [&](auto nt, auto pad) {
-        constexpr bool kNt = decltype(nt)::value, kPad = decltype(pad)::value;
-        return two ? dispatch_kernel<T, kNt, kPad, true> : dispatch_kernel<T, kNt, kPad, false>;
-    };
-    const std::true_type yes;
-    const std::false_type no;
-    auto kern = a.Dk == a.D ? (nt_x ? pick(yes, no) : pick(no, no)) : (nt_x ? pick(yes, yes) : pick(no, yes));
+    auto kern = a.Dk == a.D ? (nt_x ? dispatch_kernel<T, true, false> : dispatch_kernel<T, false, false>)
+                            : (nt_x ? dispatch_kernel<T, true, true> : dispatch_kernel<T, false, true>);
     hipError_t err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                          (int)lds);
     if (err != hipSuccess) return err;

@@ -228,8 +228,8 @@ def test_noalloc_in_pieces():
         assert np.array_equal(a, b)
 
 
-# more 64-row chunks than CUs: two dispatch blocks share a CU (rows of one 512-byte
-# slab: padded, whole, and more x than the L2 caches hold), next to one of two slabs
+# more 64-row chunks than CUs, two dispatch blocks on a CU: rows of one 512-byte slab
+# (padded, whole, and more x than the L2 caches hold) and of two
 @pytest.mark.parametrize("rows,D,E,k,dtype", [(16448, 72, 6, 2, "f32"), (17000, 128, 40, 5, "bf16"), (16500, 128, 3, 1, "f32"),
                                               (70000, 256, 4, 1, "bf16"), (70001, 248, 4, 2, "bf16"), (17000, 288, 6, 2, "bf16")])
 def test_dispatch_two_blocks_a_cu(rows, D, E, k, dtype):
