@@ -157,42 +157,44 @@ __global__ __launch_bounds__(NW * kWave) void gemm_rows_kernel(GemmArgs a) {
 #pragma unroll
             for (int j = 0; j < NT; ++j) acc[i][j] *= a.sum_down;
         if (a.all_f32 || __any(t != t)) {
-            f32x4_t again[NB][NT];
-#pragma unroll
-            for (int i = 0; i < NB; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) again[i][j] = NW == 1 ? bias(i) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            for (int st = s0; st < s1; ++st) {
-                V wa[KS][NB], xb[XS][NT];
-                load(st, wa, xb);
-#pragma unroll
-                for (int j = 0; j < NT; ++j) {
-                    u32x4_t pl[kPlanes];
-#pragma unroll
-                    for (int c = 0; c < kPlanes; ++c) pl[c] = __builtin_bit_cast(u32x4_t, xb[c][j]);
-#pragma unroll
-                    for (int k8 = 0; k8 < 8; ++k8)
-#pragma unroll
-                        for (int i = 0; i < NB; ++i)
-                            again[i][j] = mfma_f32(wa[k8 / 4][i][k8 % 4] * a.w_down, unsplit(pl, k8), again[i][j]);
-                }
-            }
+            // (16 token rows at a time: all of them at once took 260 to 288
+            // registers, which leaves a SIMD one wave)
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
+                f32x4_t again[NB];
+#pragma unroll
+                for (int i = 0; i < NB; ++i) again[i] = NW == 1 ? bias(i) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+                for (int st = s0; st < s1; ++st) {
+                    u32x4_t pl[kPlanes];
+#pragma unroll
+                    for (int c = 0; c < kPlanes; ++c)
+                        pl[c] = *reinterpret_cast<const u32x4_t*>(Xt + (st * XS + c) * xstep + xoff[j]);
+#pragma unroll
+                    for (int c = 0; c < KS; ++c)
+#pragma unroll
+                        for (int i = 0; i < NB; ++i) {
+                            const f32x4_t w = *reinterpret_cast<const f32x4_t*>(
+                                reinterpret_cast<const char*>(Wt + (st * KS + c) * wstep) + i * 16 * kKBlockBytes + woff);
+#pragma unroll
+                            for (int k4 = 0; k4 < 4; ++k4)
+                                again[i] = mfma_f32(w[k4] * a.w_down, unsplit(pl, c * 4 + k4), again[i]);
+                        }
+                }
                 if (a.all_f32) {
 #pragma unroll
-                    for (int i = 0; i < NB; ++i) acc[i][j] = again[i][j];
+                    for (int i = 0; i < NB; ++i) acc[i][j] = again[i];
                 } else if constexpr (MODE == kDown) {
 #pragma unroll
-                    for (int i = 0; i < NB; ++i) keep_finite(acc[i][j], again[i][j]);
+                    for (int i = 0; i < NB; ++i) keep_finite(acc[i][j], again[i]);
                 } else {
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
 #pragma unroll
                         for (int s = 0; s < 4; ++s) {
                             const bool ok = unit_finite(acc[i][j][s], acc[i + 2][j][s]);
-                            acc[i][j][s] = ok ? acc[i][j][s] : again[i][j][s];
-                            acc[i + 2][j][s] = ok ? acc[i + 2][j][s] : again[i + 2][j][s];
+                            acc[i][j][s] = ok ? acc[i][j][s] : again[i][s];
+                            acc[i + 2][j][s] = ok ? acc[i + 2][j][s] : again[i + 2][s];
                         }
                 }
             }

@@ -163,16 +163,16 @@ struct GemmArgs {
     // gemm_rows, dense feed-forward: its rows, all of expert 0, with no tile
     // table (tiles and tile_total are not read); 0: the table
     int64_t dense_rows = 0;
-    // f32 partial sums of tiles split along K (kSplitUnits units of
-    // kSplitUnitFloats each; null: no tile is split) and one arrival counter per
-    // split tile (zero between launches: the last part to arrive resets it)
-    float* split_ws;
-    int32_t* split_cnt;
     // f32: W holds the weights times a power of two (kPlaneScale or 1) and the sums
     // of planes come out times sum_up; their inverses; and whether every sum is
     // made with f32 MFMAs (weights too large to be scaled, others too small not to be)
     float w_down = 1.0f, sum_up = 1.0f, sum_down = 1.0f;
     bool all_f32 = false;
+    // f32 partial sums of tiles split along K (kSplitUnits units of
+    // kSplitUnitFloats each; null: no tile is split) and one arrival counter per
+    // split tile (zero between launches: the last part to arrive resets it)
+    float* split_ws;
+    int32_t* split_cnt;
     // the ticket counter of the tail units handed out at run time
     // (zero before the launch: the kernel that writes the tile table clears it)
     int32_t* tail_cnt = nullptr;
