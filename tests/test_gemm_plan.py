@@ -3,7 +3,8 @@
 For a wide range of routed rows, expert counts and widths: the choice is one
 the kernels have, the tile table's bound holds the tiles of every choice at
 any row count up to the bound's, and padded widths never split K over waves
-(so that their results do not depend on the row count).
+(so that their results do not depend on the row count).  At sizes where one
+kernel measured far ahead of the other the choice is that one.
 """
 import os
 import shutil
@@ -29,7 +30,9 @@ int main() {
           const int64_t Dk = padded_k(D, (int)dtype_size(dt)), Hp = round_up(H, 128);
           int64_t most = 0;  // tiles of any call so far (A ascending)
           for (int64_t A = 1; A < 40000000; A += 1 + A / 7) {
-            const GemmPlan p = gemm_plan(dt, A, E, Dk, Hp, D, H);
+           for (double copy : {-1.0, 0.0, 20.0}) {  // routed; dense without and with a copy of x to save
+            if (copy >= 0 && E != 1) continue;
+            const GemmPlan p = gemm_plan(dt, A, E, Dk, Hp, D, H, copy);
             const int bms[2] = {p.bm1, p.bm2}, waves[2] = {p.waves1, p.waves2};
             for (int g = 0; g < 2; ++g) {
               const int bm = bms[g];
@@ -44,6 +47,7 @@ int main() {
             }
             mixed += p.bm1 != p.bm2;
             ++n;
+           }
           }
         }
   if (!mixed) { printf("the GEMMs never differ\n"); return 1; }
@@ -66,3 +70,59 @@ def test_gemm_plan(tmp_path):
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0, out.stdout + out.stderr
     assert out.stdout.startswith("ok")
+
+
+# (dtype, routed rows, experts, dim, hidden, GEMM, tile rows): stage times on one
+# MI355X in us, 256-row tiles against the best of gemm_rows
+MEASURED = [
+    ("bf16", 5539, 1, 512, 768, "up", 256),        # 20.0 against 38.7
+    ("bf16", 2836, 1, 512, 1408, "up", 256),       # 20.1 against 36.6
+    ("bf16", 2567, 1, 768, 1536, "up", 256),       # 24.4 against 43.3
+    ("bf16", 19116, 4, 256, 256, "up", 256),       # 16.5 against 30.3
+    ("bf16", 16000, 32, 256, 640, "up", 256),      # a forward 76 against 104
+    ("bf16", 4000, 32, 512, 2048, "up", 256),      # 42.3 against 68.1
+    ("f32", 7322, 16, 1024, 1024, "up", 256),      # 161 against 259
+    ("bf16", 14560, 64, 616, 616, "down", 256),    # 27.7 against 45.5
+    ("bf16", 15361, 64, 1216, 304, "up", 256),     # 48.9 against 76.3
+    ("bf16", 32, 8, 1536, 4096, "up", 16),         # 37 against 28
+    ("bf16", 2222, 6, 1000, 2667, "down", 64),     # 53 against 35
+    ("f32", 416, 4, 64, 128, "up", 16),            # a forward 59 against 31
+]
+
+PICKS = r"""
+#include "gemm_plan.hpp"
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+using namespace nomas;
+int main(int argc, char** argv) {
+  for (int i = 1; i + 4 < argc; i += 5) {
+    const DType dt = !strcmp(argv[i], "f32") ? DType::F32 : !strcmp(argv[i], "bf16") ? DType::BF16 : DType::F16;
+    const int64_t A = atol(argv[i + 1]), E = atol(argv[i + 2]), D = atol(argv[i + 3]), H = atol(argv[i + 4]);
+    const GemmPlan p = gemm_plan(dt, A, E, padded_k(D, (int)dtype_size(dt)), round_up(H, 128), D, H);
+    printf("%d %d %d %d\n", p.bm1, p.waves1, p.bm2, p.waves2);
+  }
+  return 0;
+}
+"""
+
+
+def picks(tmp_path, calls):
+    """(bm1, waves1, bm2, waves2) of each (dtype, routed rows, experts, dim, hidden)."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not available")
+    src = tmp_path / "picks.cpp"
+    src.write_text(PICKS)
+    exe = tmp_path / "picks"
+    subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "-O2", "-std=c++17", "-I", CSRC,
+                    str(src), "-o", str(exe)], check=True, capture_output=True)
+    out = subprocess.run([str(exe)] + [str(v) for c in calls for v in c], capture_output=True,
+                         text=True, timeout=60, check=True).stdout.split("\n")
+    return [tuple(int(v) for v in line.split()) for line in out if line]
+
+
+def test_measured_choices(tmp_path):
+    got = picks(tmp_path, [c[:5] for c in MEASURED])
+    for c, p in zip(MEASURED, got):
+        assert (p[0] if c[5] == "up" else p[2]) == c[6], (c, p)
