@@ -205,7 +205,13 @@ __device__ __forceinline__ void store_hidden(void* h, int64_t a_cap, int r, int 
         constexpr int KB = kblock_elems<T>();
         T t[4];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) t[s] = Elt<T>::from_f32(v[s]);
+        for (int s = 0; s < 4; ++s) {
+            // rounded to f32 and then to T, as gemm_mfma does (the compiler made one
+            // operation with a single rounding of the last product and the f16)
+            float f = v[s];
+            asm("" : "+v"(f));
+            t[s] = Elt<T>::from_f32(f);
+        }
         uint2 raw;
         __builtin_memcpy(&raw, t, sizeof(raw));
         dst = static_cast<unsigned char*>(h) + ((int64_t)(hc / KB) * a_cap + r) * kKBlockBytes + hc % KB * 2;

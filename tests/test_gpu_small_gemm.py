@@ -56,7 +56,7 @@ def test_gemms_of_different_tile_heights(D, H, dtype):
     run_case(1111, D, 6, 2, H, dtype, 700 + D)
 
 
-@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
 def test_padded_rows_do_not_depend_on_the_call(dtype):
     """Every row of a padded-width layer is the same bits in a call of 9,000 rows and of 3."""
     t, x = small_case(9000, 264, 2, 1, 700, 77)
