@@ -20,10 +20,10 @@ CASES = {
     # the same shape with biases everywhere and the additive dense branch
     "tiny_f32_bias_dense": dict(rows=208, dim=64, E=4, k=2, H=128, dtype="f32", seed=0x5EED0100,
                                 bias=True, shared_dense=0.5, router_std=0.3),
-    # bf16, a shape the MFMA kernels tile (D % 256 == 0, H % 128 == 0)
+    # bf16, widths of whole tiles (D % 256 == 0, H % 128 == 0)
     "bf16_mfma": dict(rows=64, dim=256, E=8, k=2, H=128, dtype="bf16", seed=0x5EED0101,
                       bias=True, shared_dense=0.0, router_std=0.1),
-    # f16, general path (D and H not tiled by the MFMA kernels), k = 3
+    # f16, widths that run padded, k = 3
     "f16_general": dict(rows=50, dim=72, E=6, k=3, H=100, dtype="f16", seed=0x5EED0102,
                         bias=True, shared_dense=0.0, router_std=0.2),
     # k = E: every expert selected

@@ -12,6 +12,8 @@ import subprocess
 
 import pytest
 
+from gemm_cases import DENSE, EXPERTS, ONE_EXPERT
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "hy-nomas-rs_amd", "csrc")
 
@@ -96,11 +98,17 @@ PICKS = r"""
 #include <cstring>
 using namespace nomas;
 int main(int argc, char** argv) {
-  for (int i = 1; i + 4 < argc; i += 5) {
+  for (int i = 1; i + 5 < argc; i += 6) {
     const DType dt = !strcmp(argv[i], "f32") ? DType::F32 : !strcmp(argv[i], "bf16") ? DType::BF16 : DType::F16;
     const int64_t A = atol(argv[i + 1]), E = atol(argv[i + 2]), D = atol(argv[i + 3]), H = atol(argv[i + 4]);
-    const GemmPlan p = gemm_plan(dt, A, E, padded_k(D, (int)dtype_size(dt)), round_up(H, 128), D, H);
-    printf("%d %d %d %d\n", p.bm1, p.waves1, p.bm2, p.waves2);
+    const int64_t Dk = padded_k(D, (int)dtype_size(dt)), Hp = round_up(H, 128), mt = (A + 255) / 256;
+    const GemmPlan p = gemm_plan(dt, A, E, Dk, Hp, D, H, atof(argv[i + 5]));
+    // the K-split parts of one expert's last tiles (tile_map.hpp)
+    const int turn = kStages * kKBlockBytes / (int)dtype_size(dt);
+    const bool padded = D % 256 || H != Hp;
+    const int s1 = padded ? 1 : split_parts(mt * (2 * Hp / 256), (int)(Dk / turn));
+    const int s2 = padded ? 1 : split_parts(mt * (round_up(D, 256) / 256), (int)(Hp / turn));
+    printf("%d %d %d %d %d %d\n", p.bm1, p.waves1, p.bm2, p.waves2, s1, s2);
   }
   return 0;
 }
@@ -108,7 +116,8 @@ int main(int argc, char** argv) {
 
 
 def picks(tmp_path, calls):
-    """(bm1, waves1, bm2, waves2) of each (dtype, routed rows, experts, dim, hidden)."""
+    """(bm1, waves1, bm2, waves2, parts1, parts2) of each (dtype, routed rows, experts, dim,
+    hidden, dense_copy); the parts are those of one expert."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         pytest.skip("hipcc not available")
@@ -123,6 +132,18 @@ def picks(tmp_path, calls):
 
 
 def test_measured_choices(tmp_path):
-    got = picks(tmp_path, [c[:5] for c in MEASURED])
+    got = picks(tmp_path, [c[:5] + (-1,) for c in MEASURED])
     for c, p in zip(MEASURED, got):
         assert (p[0] if c[5] == "up" else p[2]) == c[6], (c, p)
+
+
+def test_calls_reach_gemm_mfma(tmp_path):
+    """The calls of gemm_cases.py run the 256-row kernel in the forms they name."""
+    one = [(dt, rows, 1, D, H, copy) for cases, copy in ((ONE_EXPERT, -1), (DENSE, 0))
+           for dt, rows, D, H, _, _ in cases]
+    want = [c[4:] for c in ONE_EXPERT + DENSE]
+    for call, parts, p in zip(one, want, picks(tmp_path, one)):
+        assert p[0] == 256 and p[2] == 256 and p[4:] == parts, (call, p)
+    several = [(dt, rows * k, E, D, H, -1) for dt, rows, D, E, k, H in EXPERTS]
+    for call, p in zip(several, picks(tmp_path, several)):
+        assert p[0] == 256 and p[2] == 256, (call, p)

@@ -65,7 +65,7 @@ def test_mfma_path(dtype):
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_general_path(dtype):
-    # shapes the MFMA kernels do not tile take the general path
+    # widths that are no whole tiles run padded
     ffn, _, _ = run(130, 72, 100, dtype, seed=42)
     assert not ffn.uses_mfma
 
@@ -104,10 +104,11 @@ def test_host_tensors_and_leading_dims():
     assert torch.equal(yh.reshape(96, 256).float(), torch.from_numpy(got))
 
 
-def test_host_tensors_in_pieces():
-    # 9,000 host rows: two pieces of 4,544 and 4,456 rows whose copies overlap the other's forward;
+@pytest.mark.parametrize("rows", [9000, 40000])
+def test_host_tensors_in_pieces(rows):
+    # 9,000 host rows run in one piece, 40,000 in three whose copies overlap the others' forwards;
     # against the oracle and a device forward of all rows (a K-split tile may round differently)
-    t, x = ffn_case(9000, 256, 256, 46)
+    t, x = ffn_case(rows, 256, 256, 46)
     ffn = nm.FeedForward.from_source(nm.Weights.from_tensors(t, "bf16"), PATH, 256, 256)
     raw = nm.to_model_dtype(x, "bf16")
     xh = torch.from_numpy(raw.view(np.int16)).view(torch.bfloat16)

@@ -40,9 +40,11 @@ def _noalloc(layer, x, out):
 
 @pytest.mark.parametrize("entry", ["forward", "forward_noalloc"])
 @pytest.mark.parametrize("dim,E,k,hidden,dtype,rows", [
-    (256, 8, 2, 256, "bf16", 1500),   # MFMA path
-    (256, 8, 2, 128, "f32", 700),     # MFMA path, f32
-    (192, 4, 2, 96, "bf16", 400),     # general grouped GEMM
+    (256, 8, 2, 256, "bf16", 1500),   # whole tiles, gemm_rows
+    (256, 8, 2, 128, "f32", 700),
+    (192, 4, 2, 96, "bf16", 400),     # padded widths
+    (1280, 1, 1, 512, "bf16", 6100),  # gemm_mfma, both GEMMs split along K
+    (1024, 1, 1, 256, "f32", 8150),
 ])
 def test_graph_replays_match_eager(entry, dim, E, k, hidden, dtype, rows):
     layer = _layer(dim, E, k, hidden, dtype, 90 + rows % 7)
@@ -138,8 +140,9 @@ def _replay_check(run, y, eager, other_run, y_other, eager_other, s, reps=3):
 
 
 @pytest.mark.parametrize("dim,hidden,dtype,rows", [
-    (256, 256, "bf16", 1500),   # MFMA path
-    (192, 96, "f32", 300),      # general path
+    (256, 256, "bf16", 1500),   # whole tiles
+    (192, 96, "f32", 300),      # padded widths
+    (1024, 512, "f32", 9000),   # gemm_mfma
 ])
 def test_graph_of_dense_ffn(dim, hidden, dtype, rows):
     # the dense feed-forward (mlp.rs:39-48): tile table, K-blocked copy of x

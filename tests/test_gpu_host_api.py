@@ -51,9 +51,9 @@ def test_host_tensor_forward_equals_device_forward():
 
 
 def test_host_tensor_forward_in_several_staging_chunks():
-    # 33,333 rows x 264 f32 = 35.2 MB each way: three 16 MB staging chunks, the
-    # last one partial and not a multiple of 64 bytes, each split over the copy
-    # threads; then a small call on the same handle
+    # 33,333 rows x 264 f32 = 35.2 MB each way, in four row pieces of 8.8 MB: 4 MB
+    # staging chunks, each split over the copy threads, the last of a piece partial;
+    # then a small call on the same handle
     t, x = small_case(33_333, 264, 4, 1, 96, 32)
     layer = layer_from_tensors(t, "f32", 264, 96, 4, 1)
     xd = to_device(x, "f32")
@@ -66,12 +66,13 @@ def test_host_tensor_forward_in_several_staging_chunks():
     assert torch.equal(layer.forward(xd[:5].cpu()), yd[:5])
 
 
-def test_host_tensor_forward_in_pieces():
-    # 10,000 bf16 rows of 256 (the MFMA path): two pieces of 5,056 and 4,944 rows, the copies of one
-    # overlapping the other's forward.  The routing of the whole call is kept (the pieces are whole
+@pytest.mark.parametrize("rows", [10_000, 40_000])
+def test_host_tensor_forward_in_pieces(rows):
+    # bf16 rows of 256: 10,000 run in one piece, 40,000 in three, the copies of one
+    # overlapping the others' forwards.  The routing of the whole call is kept (the pieces are whole
     # 64-row router chunks, so it equals a device forward's bit for bit); outputs against the oracle
     # and the device forward (a K-split tile may round differently in a piece).
-    rows, D, E, k, H = 10_000, 256, 8, 2, 128
+    D, E, k, H = 256, 8, 2, 128
     t, x = small_case(rows, D, E, k, H, 33)
     layer = layer_from_tensors(t, "bf16", D, H, E, k)
     rt, rx = rounded(t, x, "bf16")

@@ -73,7 +73,7 @@ def test_golden_fixture(name):
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 def test_general_path(dtype):
-    # D=72, H=100 are not tiled by the MFMA kernels: the general path for every dtype
+    # widths that are no whole tiles (D=72, H=100) run padded, for every dtype
     assert not run_case(150, 72, 6, 2, 100, dtype, seed=11).uses_mfma
 
 
@@ -83,14 +83,13 @@ def test_mfma_path(dtype):
 
 
 def test_mfma_f32_ragged_split_tiles():
-    # f32 on the matrix cores (16x16x4 MFMAs): ragged expert tiles, several
-    # column tiles, a K long enough for the K-split tail, the quarter-tile
-    # staging of the down GEMM's output
+    # f32, k = 3, on gemm_rows' 32-row tiles (its planes on gemm_mfma's tiles, split
+    # along K too, are in test_gpu_gemm_mfma.py)
     run_case(900, 512, 4, 3, 384, "f32", seed=14)
 
 
 def test_mfma_multi_tile_ragged():
-    # several row tiles per expert, ragged last tiles, several column tiles, k = 3
+    # several row tiles per expert (of 64 rows), ragged last tiles, several column tiles, k = 3
     run_case(1000, 512, 4, 3, 384, "bf16", seed=13)
 
 

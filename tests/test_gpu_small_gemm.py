@@ -10,6 +10,7 @@ import torch
 
 from _common import rounded, small_case
 from _gpu import compare, layer_from_tensors, to_device
+from gemm_cases import DENSE
 import nomas_moe as nm
 from test_zz_no_alloc import _noalloc
 
@@ -58,7 +59,8 @@ def test_gemms_of_different_tile_heights(D, H, dtype):
 
 @pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
 def test_padded_rows_do_not_depend_on_the_call(dtype):
-    """Every row of a padded-width layer is the same bits in a call of 9,000 rows and of 3."""
+    """Every row of a padded-width layer is the same bits in a call of 9,000 rows (gate/up on
+    256-row tiles) and of 3."""
     t, x = small_case(9000, 264, 2, 1, 700, 77)
     layer = layer_from_tensors(t, dtype, 264, 700, 2, 1)
     xd = to_device(x, dtype)
@@ -85,8 +87,10 @@ def test_padded_non_finite_rows_stay_apart():
     assert torch.isposinf(yb[3]).all() and torch.isnan(yb[40]).all()
 
 
-# rows, D, H: a call of few rows and one of whole 256-row tiles
-@pytest.mark.parametrize("rows,D,H", [(70, 256, 128), (3000, 512, 256), (3000, 200, 72)])
+# rows, D, H: gemm_rows' tiles (32 and 64 rows; padded) and gemm_mfma's (whole, gate/up or
+# down split along K, padded)
+@pytest.mark.parametrize("rows,D,H", [(70, 256, 128), (3000, 512, 256), (3000, 200, 72)] +
+                         [c[1:4] for c in DENSE])
 def test_f32_values_that_have_no_finite_planes(rows, D, H):
     """f32 rows with an infinity, a NaN or a value that rounds past bf16's
     largest, and weights of that size: each row as f32 arithmetic has it, the
@@ -112,7 +116,9 @@ def test_f32_values_that_have_no_finite_planes(rows, D, H):
     assert torch.equal(yb[keep], y[keep])
     assert torch.isposinf(yb[3]).all() and torch.isnan(yb[40]).all()
     want = (float(big) * float(np.float32(1e-20))) ** 2 * H * float(np.float32(1e-3))
-    assert torch.allclose(yb[60].double(), torch.full((D,), want, device="cuda", dtype=torch.float64), rtol=2e-6)
+    # (H equal terms: each of at most H adds rounds by 2^-24 of the sum)
+    assert torch.allclose(yb[60].double(), torch.full((D,), want, device="cuda", dtype=torch.float64),
+                          rtol=max(2e-6, H * 2.0 ** -24))
     # one weight of 3.4e38 in every hidden unit's gate, met by x = 1e-30
     gate = np.full((H, D), 1e-3, np.float32)
     gate[:, 2] = big

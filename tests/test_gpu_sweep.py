@@ -1,7 +1,7 @@
 """GPU parity over a fixed, seeded sample of random configurations.
 
 Each case draws dim, hidden, experts, top-k, rows, dtype, router scale and
-the shared dense branch from fixed lists (MFMA-tiled and general shapes, one
+the shared dense branch from fixed lists (whole-tile and padded widths, one
 to 256 experts, up to top-20), builds the layer from seeded checkpoint
 tensors and compares routing and outputs with the oracle to the usual bars
 (tests/_gpu.py: compare).  Configurations the library rejects at
@@ -97,7 +97,7 @@ def test_random_block_configuration(B, S, D, E, k, H, dt, s, affine, seed):
     (2, 64, 512, 16, 8, 128, "bf16", 0.0, True, 4100),   # one group of 8 slots
     (1, 300, 256, 40, 10, 256, "f16", 0.5, False, 4101),  # 8 + 3 (dense slot)
     (3, 17, 512, 64, 8, 128, "f32", 0.5, True, 4102),    # 8 + 1 (dense slot)
-    (1, 64, 264, 17, 9, 96, "bf16", 0.0, True, 4103),    # 8 + 1, general GEMM path
+    (1, 64, 264, 17, 9, 96, "bf16", 0.0, True, 4103),    # 8 + 1, padded widths
 ])
 def test_block_many_slots(B, S, D, E, k, H, dt, s, affine, seed):
     """forward_block with 8 or more slots per row: the gated-residual combine

@@ -35,8 +35,8 @@ def test_workload(name):
 def test_one_segment_in_other_model_dtypes(dt):
     # The one-segment 8B shape (4,680 rows, dim 3072, 8 experts, top-2, hidden
     # 8192) for f16 and f32 models: their own router and MFMA GEMM
-    # instantiations (16x16x32 f16 MFMAs; for f32, f64 router MFMAs and four
-    # 16x16x4 f32 MFMAs per 16-byte fragment) at full size.
+    # instantiations (16x16x32 f16 MFMAs; for f32, f64 router MFMAs and six
+    # products of bf16 planes) at full size.
     check_workload(dataclasses.replace(wl.WORKLOADS["seg8b"], dtype=dt))
 
 

@@ -4,9 +4,9 @@ Both entry points run the same kernels; the no-allocation one lays every device
 buffer out in the library's static scratch array instead of the handle's own
 workspace.  The same input must give the same expert indices, counts, gates
 and bit-identical outputs, on two calls in a row (the second smaller), across
-layers on the MFMA and the general path sharing the one array, with a K-split
-GEMM tail (its arrival counters live in the array and must be back at zero
-after each call), and a row count beyond the array is a clear error.  One
+layers of whole-tile and of padded widths sharing the one array, with tiles
+split along K (their arrival counters live in the array and must be back at
+zero after each call), and a row count beyond the array is a clear error.  One
 4,744-row segment of the 8B preset (one guidance branch: 4,680 video + 64
 text rows) fits.  Reading the routing back after another handle's
 no-allocation forward has reused the array is a state error, not stale data.
@@ -74,16 +74,20 @@ def _check_pair(layer, t, x_f32, dtype, label):
 
 
 def test_noalloc_matches_forward_on_two_calls_and_two_layers():
-    mf, tm = _layer(1024, 8, 2, 1024, "bf16", 71)     # MFMA path, K-split tail at 1500 rows
-    gen, tg = _layer(64, 4, 2, 96, "f32", 72)         # general path (dim not a multiple of 256)
+    mf, tm = _layer(1024, 8, 2, 1024, "bf16", 71)     # whole tiles
+    ks, tk = _layer(1280, 1, 1, 512, "bf16", 79)      # both GEMMs' last tiles split along K
+    gen, tg = _layer(64, 4, 2, 96, "f32", 72)         # padded widths
     assert mf.uses_mfma and not gen.uses_mfma
     _, x1 = small_case(1500, 1024, 8, 2, 1024, 73)
     _, x2 = small_case(700, 1024, 8, 2, 1024, 74)
     _, xg = small_case(300, 64, 4, 2, 96, 75)
-    _check_pair(mf, tm, x1, "bf16", "mfma call 1")
-    _check_pair(mf, tm, x2, "bf16", "mfma call 2 (smaller)")
-    _check_pair(gen, tg, xg, "f32", "general-path layer on the same array")
-    _check_pair(mf, tm, x1, "bf16", "mfma again after the general-path layer")
+    _, xk = small_case(6100, 1280, 1, 1, 512, 78)
+    _check_pair(mf, tm, x1, "bf16", "whole tiles, call 1")
+    _check_pair(mf, tm, x2, "bf16", "call 2 (smaller)")
+    _check_pair(gen, tg, xg, "f32", "padded layer on the same array")
+    _check_pair(ks, tk, xk, "bf16", "K-split tiles")
+    _check_pair(mf, tm, x1, "bf16", "again after the other layers")
+    _check_pair(ks, tk, xk, "bf16", "K-split tiles again")
 
 
 def test_noalloc_rejects_rows_beyond_the_array():
