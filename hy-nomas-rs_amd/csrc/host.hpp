@@ -98,7 +98,8 @@ class HostStager {
 public:
     ~HostStager();
     static constexpr int kBufs = 4;
-    void rewind() { next_ = 0; }  // a call starts with the first (cached) buffer
+    // A call that copies `bytes` each way starts: with the first (cached) buffer.
+    void begin(size_t bytes);
     int to_device(void* dst_dev, const void* src_host, size_t bytes, hipStream_t s);
     int to_host(void* dst_host, const void* src_dev, size_t bytes, hipStream_t s);
 
@@ -108,6 +109,7 @@ private:
     void* pin_[kBufs] = {};
     hipEvent_t ev_[kBufs] = {};
     int next_ = 0;  // the buffer of the next chunk
+    size_t chunk_ = 0, cap_ = 0;  // bytes per chunk of this call, and of each buffer
     std::unique_ptr<CopyPool> pool_;
 };
 

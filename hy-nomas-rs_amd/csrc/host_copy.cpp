@@ -1,8 +1,11 @@
 // Copies between pageable host memory and the device for the host-tensor
-// forward: through pinned staging buffers of kChunk bytes, in chunks, so
+// forward: through pinned staging buffers of one chunk each, so
 // that the host-side memcpy of one chunk (spread over a small pool of worker
 // threads) overlaps the DMA of earlier ones.  The first chunk's memcpy is what
-// no DMA hides, so chunks are small: 4 MB, 70 us on either side.  hipMemcpy from pageable
+// no DMA hides, and every chunk wakes the workers: 4 MB, 70 us on either side, and
+// 8 MB where there are many (123 MB each way, both pageable: 4 MB 5,800, 8 MB 5,430, 16 MB
+// 5,660 us; 55 MB 2,600 / 2,240 / 2,280; 29 MB 1,320 / 1,310 / 1,500, and 8 MB buffers take
+// 1.2 ms more to allocate on a handle's first call).  hipMemcpy from pageable
 // memory stages through the runtime's own buffers with one host thread and
 // reached about 19 GB/s here; pinned-to-device DMA runs at about 55 GB/s.
 #include <hip/hip_runtime.h>
@@ -16,7 +19,8 @@
 namespace nomas {
 
 namespace {
-constexpr size_t kChunk = (size_t)4 << 20;  // bytes per staging buffer
+// bytes per chunk (and staging buffer) of calls of up to kLongCall bytes, and of longer ones
+constexpr size_t kChunk = (size_t)4 << 20, kLongChunk = (size_t)8 << 20, kLongCall = (size_t)40 << 20;
 constexpr size_t kMinSplit = (size_t)1 << 20;  // smaller copies stay on the calling thread
 }  // namespace
 
@@ -94,6 +98,11 @@ bool is_pinned(const void* p) {
 
 HostStager::~HostStager() { release(); }
 
+void HostStager::begin(size_t bytes) {
+    chunk_ = bytes > kLongCall ? kLongChunk : kChunk;
+    next_ = 0;
+}
+
 void HostStager::release() {
     for (int b = 0; b < kBufs; ++b) {
         if (ev_[b]) (void)hipEventDestroy(ev_[b]);
@@ -106,9 +115,12 @@ void HostStager::release() {
 
 // All or nothing: a failed set-up leaves nothing behind, and the next call tries again.
 int HostStager::ensure() {
-    if (pool_) return NOMAS_OK;
+    if (pool_ && cap_ >= chunk_) return NOMAS_OK;
+    for (int b = 0; pool_ && b < kBufs; ++b) (void)hipEventSynchronize(ev_[b]);  // larger ones are needed
+    release();
+    cap_ = chunk_;
     for (int b = 0; b < kBufs; ++b) {
-        hipError_t e = hipHostMalloc(&pin_[b], kChunk, hipHostMallocDefault);
+        hipError_t e = hipHostMalloc(&pin_[b], cap_, hipHostMallocDefault);
         if (e != hipSuccess) {
             pin_[b] = nullptr;
             release();
@@ -142,8 +154,8 @@ int HostStager::to_device(void* dst, const void* src, size_t bytes, hipStream_t 
     if (rc != NOMAS_OK) return rc;
     const unsigned char* in = static_cast<const unsigned char*>(src);
     unsigned char* out = static_cast<unsigned char*>(dst);
-    for (size_t off = 0; off < bytes; off += kChunk) {
-        const size_t n = std::min(kChunk, bytes - off);
+    for (size_t off = 0; off < bytes; off += chunk_) {
+        const size_t n = std::min(chunk_, bytes - off);
         const int b = next_;
         next_ = (next_ + 1) % kBufs;
         // buffer b drained (its last DMA may belong to an earlier call: the
@@ -169,21 +181,21 @@ int HostStager::to_host(void* dst, const void* src, size_t bytes, hipStream_t s)
     // up to kBufs chunks' DMAs in flight; the host copies the oldest one out
     // when it has landed.  (The buffers' earlier DMAs, into the device, may
     // still be in flight on the first round.)
-    const int64_t chunks = (int64_t)((bytes + kChunk - 1) / kChunk);
+    const int64_t chunks = (int64_t)((bytes + chunk_ - 1) / chunk_);
     const int first = next_;
     next_ = (int)((next_ + chunks) % kBufs);
-    auto len = [&](int64_t c) { return std::min(kChunk, bytes - (size_t)c * kChunk); };
+    auto len = [&](int64_t c) { return std::min(chunk_, bytes - (size_t)c * chunk_); };
     for (int64_t c = 0; c < chunks + kBufs - 1; ++c) {
         const int64_t done = c - (kBufs - 1);
         if (done >= 0) {
             const int b = (int)((first + done) % kBufs);
             STAGE_TRY(hipEventSynchronize(ev_[b]), "hipEventSynchronize");
-            pool_->copy(out + (size_t)done * kChunk, pin_[b], len(done));
+            pool_->copy(out + (size_t)done * chunk_, pin_[b], len(done));
         }
         if (c < chunks) {
             const int b = (int)((first + c) % kBufs);
             if (c < kBufs) STAGE_TRY(hipEventSynchronize(ev_[b]), "hipEventSynchronize");
-            STAGE_TRY(hipMemcpyAsync(pin_[b], in + (size_t)c * kChunk, len(c), hipMemcpyDeviceToHost, s),
+            STAGE_TRY(hipMemcpyAsync(pin_[b], in + (size_t)c * chunk_, len(c), hipMemcpyDeviceToHost, s),
                       "hipMemcpyAsync D2H");
             STAGE_TRY(hipEventRecord(ev_[b], s), "hipEventRecord");
         }

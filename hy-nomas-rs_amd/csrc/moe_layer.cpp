@@ -855,7 +855,7 @@ int MoeLayer::forward_host(const void* x, void* y, int64_t rows) {
     const uintptr_t xa = reinterpret_cast<uintptr_t>(x), ya = reinterpret_cast<uintptr_t>(y);
     const bool apart = xa == ya || xa + bytes <= ya || ya + bytes <= xa;
     const int np = apart ? host_pieces(rows) : 1;
-    stager_.rewind();
+    stager_.begin(bytes);
     if (np == 1) {
         host_pieces_ = 0;
         int rc = stager_.to_device(dx, x, bytes, nullptr);

@@ -64,6 +64,12 @@ def test_host_tensor_forward_in_several_staging_chunks():
     layer.forward(xd.cpu(), out=yp)
     assert torch.equal(yd, yp)
     assert torch.equal(layer.forward(xd[:5].cpu()), yd[:5])
+    # 50,000 rows, 53 MB: 8 MB chunks, for which the buffers grow; and small ones again
+    xl = torch.cat([xd, xd.flip(0)[:16_667]])
+    yl = torch.empty(xl.shape)
+    layer.forward(xl.cpu(), out=yl)
+    assert torch.equal(yl, layer.forward(xl).cpu())
+    assert torch.equal(layer.forward(xd.cpu()), yd)
 
 
 @pytest.mark.parametrize("rows", [10_000, 40_000])
