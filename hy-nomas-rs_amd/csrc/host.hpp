@@ -255,11 +255,11 @@ public:
 private:
     int ensure_workspace(int64_t rows);
     void free_workspace();
-    // The GEMM kernels of a forward on `rows` rows.  The pieces of one call all
-    // take the plan of the whole call (plan_rows_): the same kernels as in one
-    // forward.  (Rows of padded widths then have the same bits.  At whole-tile
-    // widths a piece's own last round decides which of its tiles gemm_mfma
-    // splits along K.)
+    // The GEMM kernels of a forward on `rows` rows.  At whole-tile widths the
+    // pieces of one call all take the plan of the whole call (plan_rows_), so that
+    // their rows are summed as in one forward but for the tiles that gemm_mfma
+    // splits along K (a piece's own last round decides which).  Rows of padded
+    // widths have the same bits whichever kernel runs: a piece takes its own plan.
     GemmPlan gemm_plan(int64_t rows) const;
     int64_t plan_rows_ = 0;  // rows of the pieced call in progress, else 0
     int max_tiles(int64_t rows, int bm) const;

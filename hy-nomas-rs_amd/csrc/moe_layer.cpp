@@ -362,7 +362,7 @@ int MoeLayer::upload_f32(const MoeParamsF32& p) {
 // ---- workspace --------------------------------------------------------------
 
 GemmPlan MoeLayer::gemm_plan(int64_t rows) const {
-    rows = std::max(rows, plan_rows_);
+    if (tiled_) rows = std::max(rows, plan_rows_);
     // dense, 16-bit rows of whole K turns: gemm_rows reads them in place, and the
     // copy (5 us and both ways of x at 5 TB/s) is saved
     const bool copy = dt_ != DType::F32 && D_ == Dk_;
