@@ -20,8 +20,8 @@
 //    Bound by the matrix cores: 384 MFMAs per wave and step against 352 vector
 //    instructions that split the weights (the f32 MFMAs take 2.7 times as long).
 //    4,680 rows of dim 1536, hidden 4096, 8 experts: gate/up + down 1,955 +
-//    1,091 -> 1,270 + 579 us in a trace (a forward 3,035 -> 1,768 us), the
-//    error against f64 1.6e-6 -> 1.4e-6.  The
+//    1,091 us on the f32 MFMAs, 1,154 + 572 in a trace (a forward 3,035 -> 1,645
+//    us), the error against f64 1.6e-6 -> 1.4e-6.  The
 //    weights are split here and not in memory (6 bytes an element, 1.5 times
 //    the traffic of a call of few rows); splitting the token rows here too
 //    needs 192 registers of planes and ran 1.36 times slower.
@@ -350,8 +350,8 @@ __global__ __launch_bounds__(NWM * 2 * kWave, 1) void gemm_mfma_kernel(GemmArgs 
                     });
                 });
                 // (keeps the accumulators in place from turn to turn: without it
-                // the down kernel's register allocation moved 576 of them per turn
-                // instead of 272)
+                // the down kernel's register allocation moved 576 of them per turn;
+                // it now moves 152, the padded gate/up kernel 244)
 #pragma unroll
                 for (int i = 0; i < SN; ++i)
 #pragma unroll

@@ -19,11 +19,14 @@
 //    each other, in eight contiguous shares, one per XCD (block i runs on XCD
 //    i % 8): the row tiles of an expert then find its weights in their XCD's
 //    L2.
-// Measured (gate/up + down, one MI355X, against gemm_mfma's 256 x 256 tiles or,
-// for padded widths, the earlier vector-unit kernel): 16 rows of 8 experts of
-// 1536 x 4096 in bf16 37 + 47 -> 28 + 16 us (7.0 and 6.2 TB/s of weights); 64
-// rows 41 + 52 -> 34 + 20 us; 512 rows of 512 x 1024, 4 experts, 36 + 29 -> 13 +
-// 9 us; 208 rows of 64 x 128 in f32, 4 experts, 19 + 20 -> 5 + 5 us.
+//  - Padding past a step of 32 columns, past the real columns (down) and past 32
+//    hidden units that hold a real one (gate/up) is neither read nor computed.
+// Measured (stage times of gate/up + down, one MI355X, against gemm_mfma's 256 x
+// 256 tiles or, for padded widths, the earlier vector-unit kernel): 16 rows of 8
+// experts of 1536 x 4096 in bf16 42 + 51 -> 33 + 18.5 us (6.1 and 5.4 TB/s of
+// weights); 64 rows 43 + 53 -> 36 + 21 us; 512 rows of 512 x 1024, 4 experts, 37 +
+// 29 -> 13 + 8 us; 208 rows of 64 x 128 in f32, 4 experts, 18 + 20 -> 5.5 + 6 us;
+// 1,111 rows of 1000 x 2667, 6 experts, down 555 -> 35 us.
 #include <type_traits>
 
 #include "kernels.hpp"

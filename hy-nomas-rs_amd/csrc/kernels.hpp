@@ -104,7 +104,7 @@ __host__ __device__ constexpr int64_t round_up(int64_t n, int64_t m) { return (n
 // 16 + 4c..16 + 4c + 3 of the block, the order in which a GEMM lane holds the
 // weights of two 16-column f32 K-blocks.  Element (r, k) of plane p:
 //   ((k / 32 * 3 + p) * R + r) * 32 + (k / 4 % 4) * 8 + (k / 16 % 2) * 4 + k % 4
-constexpr int kActPlanes = 3;
+constexpr int kActPlanes = 3;  // mfma.hpp's kPlanes
 constexpr float kPlaneScale = 0x1p24f;  // the planes add up to the value times this (mfma.hpp)
 // Bytes of one element of x_perm or h.
 __host__ __device__ constexpr int act_bytes(DType dt) { return dt == DType::F32 ? 2 * kActPlanes : 2; }

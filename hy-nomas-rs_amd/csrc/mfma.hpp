@@ -36,7 +36,10 @@ __device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
 // three bf16 planes (the value rounded to bf16, the remainder rounded, the
 // rest: 8 + 8 + 8 significant bits), and a product of two values is the six
 // plane products down to 2^-16 of the largest, added smallest first into the
-// f32 accumulator; what is left out is below 2^-26 of the product.  The bf16
+// f32 accumulator.  Left out are the second plane of one value times the third of the
+// other, twice: each below 2^-8 x 2^-17 of the values' powers of two, so at most 2^-24
+// of the product (half a unit of its last place; on N(0, 1) pairs 2^-27.4 in the
+// mean square), and what is left has six roundings per 32 products.  The bf16
 // MFMA does a plane product in 1/16 of the time of the f32 MFMAs.  Weights stay
 // f32 in memory and are split by the GEMM; activations (x_perm, h) are split
 // once, by the kernels that write them (kernels.hpp).
@@ -50,7 +53,7 @@ __device__ __forceinline__ f32x4_t mfma_f32(float a, float b, f32x4_t c) {
 // those, and products with a value that has no planes (2^103 and more, infinite,
 // NaN: the mark below) or with a weight that rounds past bf16's largest.
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-constexpr int kPlanes = 3;
+constexpr int kPlanes = kActPlanes;
 constexpr int kProducts = 6;
 constexpr float kPlaneMax = 0x1p127f;  // of a value times kPlaneScale
 constexpr uint32_t kRawMark = 0x7f80;  // plane 1 (infinite) of a value stored as its raw halves in planes 0 and 2

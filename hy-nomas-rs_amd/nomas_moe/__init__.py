@@ -450,6 +450,8 @@ class FeedForward:
     """Dense SwiGLU feed-forward (FeedForward::SwiGlu, mlp.rs:9-59) on one MI355X:
     y = down(silu(gate(x)) * up(x)), on the expert GEMM kernels without routing."""
 
+    # ("router", "tile_table" and "combine" have no kernel here and read zero; the
+    # copy of x, where there is one, also writes the tile table)
     STAGES = ("router", "tile_table", "kblock_copy", "gemm_gate_up", "gemm_down", "combine")
 
     def __init__(self, handle: C.c_void_p, dim: int, hidden: int, dtype: DataType, device: int):
