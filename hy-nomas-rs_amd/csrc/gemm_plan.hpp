@@ -64,9 +64,10 @@ constexpr RowsCost kRowsCost[2][2][4] = {
 
 // A routed rows over E experts; Dk and Hp are the padded widths of D and H.
 // dense_copy: >= 0 in the dense feed-forward, the us of the K-blocked copy of x that
-// it saves where gemm_rows runs both GEMMs.
+// it saves where gemm_rows runs both GEMMs.  shared: of the A rows, those of the shared
+// dense branch, one of the E experts, which has every row of the call.
 inline GemmPlan gemm_plan(DType dt, int64_t A, int64_t E, int64_t Dk, int64_t Hp, int64_t D, int64_t H,
-                          double dense_copy = -1) {
+                          double dense_copy = -1, int64_t shared = 0) {
     // padded widths keep one order of summation at any row count: one wave, no K split
     const bool padded = D % kMfmaBN != 0 || H != Hp;
     const bool f32 = dt == DType::F32;
@@ -74,9 +75,15 @@ inline GemmPlan gemm_plan(DType dt, int64_t A, int64_t E, int64_t Dk, int64_t Hp
     // k steps of gate/up and down: gemm_mfma's, and gemm_rows' (kernels.hpp)
     const double kt1 = Dk / kb, kt2 = Hp / kb, kr1 = step_k(D) / kb, kr2 = step_k(H) / kb;
     const double live = (double)std::max<int64_t>(1, std::min(A, E)), mean = A / live;
-    // row tiles: of evenly loaded experts, and on average over uneven ones (of one: the same)
-    auto even = [&](int bm) { return live * std::ceil(mean / bm); };
-    auto tiles = [&](int bm) { return live == 1 ? even(bm) : live * std::max(1.0, mean / bm + 0.5); };
+    // row tiles: of evenly loaded experts, and on average over uneven ones (of one: the
+    // same); the shared branch's exactly
+    const double routed = (double)(A - shared), on = (double)std::min(A - shared, E - (shared ? 1 : 0));
+    auto even = [&](int bm) {
+        return (on > 0 ? on * std::ceil(routed / on / bm) : 0) + std::ceil((double)shared / bm);
+    };
+    auto tiles = [&](int bm) {
+        return on <= 1 ? even(bm) : on * std::max(1.0, routed / on / bm + 0.5) + std::ceil((double)shared / bm);
+    };
     auto cost_mfma_of = [&](double all, double kt) {
         const MfmaCost& c = kMfmaCost[padded][f32];
         const double rounds = all / kRound;

@@ -367,7 +367,8 @@ GemmPlan MoeLayer::gemm_plan(int64_t rows) const {
     // copy (5 us and both ways of x at 5 TB/s) is saved
     const bool copy = dt_ != DType::F32 && D_ == Dk_;
     return nomas::gemm_plan(dt_, rows * kslots_, Ecols_, Dk_, Hp_, D_, H_,
-                            !dense_only_ ? -1.0 : copy ? 5.0 + rows * D_ * 4 / 5e6 : 0.0);
+                            !dense_only_ ? -1.0 : copy ? 5.0 + rows * D_ * 4 / 5e6 : 0.0,
+                            Ecols_ > E_ ? rows : 0);
 }
 
 int MoeLayer::max_tiles(int64_t rows, int bm) const {

@@ -32,9 +32,10 @@ int main() {
           const int64_t Dk = padded_k(D, (int)dtype_size(dt)), Hp = round_up(H, 128);
           int64_t most = 0;  // tiles of any call so far (A ascending)
           for (int64_t A = 1; A < 40000000; A += 1 + A / 7) {
-           for (double copy : {-1.0, 0.0, 20.0}) {  // routed; dense without and with a copy of x to save
+           // routed; dense without and with a copy of x to save; a shared branch with half of the rows
+           for (double copy : {-1.0, 0.0, 20.0, -2.0}) {
             if (copy >= 0 && E != 1) continue;
-            const GemmPlan p = gemm_plan(dt, A, E, Dk, Hp, D, H, copy);
+            const GemmPlan p = gemm_plan(dt, A, E, Dk, Hp, D, H, copy, copy == -2.0 ? A / 2 : 0);
             const int bms[2] = {p.bm1, p.bm2}, waves[2] = {p.waves1, p.waves2};
             for (int g = 0; g < 2; ++g) {
               const int bm = bms[g];
