@@ -109,7 +109,8 @@ private:
     void* pin_[kBufs] = {};
     hipEvent_t ev_[kBufs] = {};
     int next_ = 0;  // the buffer of the next chunk
-    size_t chunk_ = 0, cap_ = 0;  // bytes per chunk of this call, and of each buffer
+    size_t chunk_ = (size_t)4 << 20;  // bytes per chunk of this call
+    size_t cap_ = 0;                  // and of each buffer
     std::unique_ptr<CopyPool> pool_;
 };
 
